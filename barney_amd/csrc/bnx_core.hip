@@ -51,19 +51,19 @@ __global__ void k_prim_boxes(const GeomBuild *gb, int num_geoms, int n, float4 *
         h[a] = fmx(h[a], v[a]);
       }
     }
-    lo[p] = make_float4(l[0], l[1], l[2], 0.f);
+    lo[p] = make_float4(l[0], l[1], l[2], __int_as_float(p));
     hi[p] = make_float4(h[0], h[1], h[2], 0.f);
   } else if (G.type == 1) {
     // SpheresPrograms::bounds (Spheres.dev.cu:29-40)
     float4 s = G.spheres[prim];
-    lo[p] = make_float4(s.x - s.w, s.y - s.w, s.z - s.w, 0.f);
+    lo[p] = make_float4(s.x - s.w, s.y - s.w, s.z - s.w, __int_as_float(p));
     hi[p] = make_float4(s.x + s.w, s.y + s.w, s.z + s.w, 0.f);
   } else if (G.type == 2) {
     // CylindersPrograms::bounds (native/geometry/Cylinders.dev.cu:69-85):
     // the boxes of both end spheres
     const float4 a = G.cyls[2 * prim], b = G.cyls[2 * prim + 1];
     const float r = a.w;
-    lo[p] = make_float4(fmn(a.x - r, b.x - r), fmn(a.y - r, b.y - r), fmn(a.z - r, b.z - r), 0.f);
+    lo[p] = make_float4(fmn(a.x - r, b.x - r), fmn(a.y - r, b.y - r), fmn(a.z - r, b.z - r), __int_as_float(p));
     hi[p] = make_float4(fmx(a.x + r, b.x + r), fmx(a.y + r, b.y + r), fmx(a.z + r, b.z + r), 0.f);
   } else {
     // capsules and cones: the boxes of both end spheres (getBounds,
@@ -73,7 +73,7 @@ __global__ void k_prim_boxes(const GeomBuild *gb, int num_geoms, int n, float4 *
     // or not depending on traversal order, so cones take the box that holds
     // them
     const float4 a = G.cyls[2 * prim], b = G.cyls[2 * prim + 1];
-    lo[p] = make_float4(fmn(a.x - a.w, b.x - b.w), fmn(a.y - a.w, b.y - b.w), fmn(a.z - a.w, b.z - b.w), 0.f);
+    lo[p] = make_float4(fmn(a.x - a.w, b.x - b.w), fmn(a.y - a.w, b.y - b.w), fmn(a.z - a.w, b.z - b.w), __int_as_float(p));
     hi[p] = make_float4(fmx(a.x + a.w, b.x + b.w), fmx(a.y + a.w, b.y + b.w), fmx(a.z + a.w, b.z + b.w), 0.f);
   }
 }
@@ -108,7 +108,7 @@ __global__ void k_boxes_from_floats(const float *b, int n, float4 *lo, float4 *h
 {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  lo[i] = make_float4(b[6 * i + 0], b[6 * i + 1], b[6 * i + 2], 0.f);
+  lo[i] = make_float4(b[6 * i + 0], b[6 * i + 1], b[6 * i + 2], __int_as_float(i));
   hi[i] = make_float4(b[6 * i + 3], b[6 * i + 4], b[6 * i + 5], 0.f);
 }
 
@@ -136,7 +136,7 @@ int build_blas(Group *g)
     gb.push_back(b);
     n += geom->num_prims;
   }
-  DevMem d_gb, lo, hi, pgeom;
+  DevMem &d_gb = dev->build.geoms, &lo = dev->build.box_lo, &hi = dev->build.box_hi, &pgeom = dev->build.pgeom;
   int rc;
   if ((rc = upload(dev, d_gb, gb.data(), gb.size())) != BNX_OK) return rc;
   BNX_HIP(lo.ensure(sizeof(float4) * (size_t)(n ? n : 1)));
@@ -313,7 +313,9 @@ int build_tlas(Group *g)
         }
       }
     }
-    lo[i] = make_float4(bl[0], bl[1], bl[2], 0.f);
+    float index;
+    memcpy(&index, &i, sizeof(index));
+    lo[i] = make_float4(bl[0], bl[1], bl[2], index);
     hi[i] = make_float4(bh[0], bh[1], bh[2], 0.f);
   }
   std::vector<BlasDev> blas(blas_groups.size());
@@ -347,7 +349,7 @@ int build_tlas(Group *g)
     dev->xf_worlds += has_xf ? 1 : -1;
     g->has_xf = has_xf;
   }
-  DevMem d_lo, d_hi;
+  DevMem &d_lo = dev->build.box_lo, &d_hi = dev->build.box_hi;
   int rc;
   if ((rc = upload(dev, d_lo, lo.data(), n)) != BNX_OK) return rc;
   if ((rc = upload(dev, d_hi, hi.data(), n)) != BNX_OK) return rc;
@@ -1091,7 +1093,7 @@ int bnx_bvh_build_boxes(bnx_device d, const float *d_boxes, int n, int max_leaf,
   GUARD_BEGIN
   BNX_CHECK(d && (n == 0 || d_boxes) && n >= 0 && max_leaf >= 1 && max_leaf <= 7, BNX_ERR_INVALID,
             "bnx_bvh_build_boxes: bad argument");
-  DevMem lo, hi;
+  DevMem &lo = d->build.box_lo, &hi = d->build.box_hi;
   BNX_HIP(lo.ensure(sizeof(float4) * (size_t)(n ? n : 1)));
   BNX_HIP(hi.ensure(sizeof(float4) * (size_t)(n ? n : 1)));
   if (n) k_boxes_from_floats<<<nblk(n, 256), 256, 0, d->stream>>>(d_boxes, n, lo.as<float4>(), hi.as<float4>());

@@ -81,10 +81,13 @@ struct DevMem {
 
 struct Device;
 
-// scratch arrays of the BVH builder, kept per device and grown on demand
+// scratch arrays of the BVH builder, kept per device and grown on demand:
+// the boxes being built over (box_lo, box_hi) with their second copy, the
+// primitives' geometries, and the builder's tables
 struct BuildScratch {
-  DevMem lo, hi, order, order_tmp, slot_task, flags, scan, cub_tmp;
-  DevMem tasks, tasks_next, bins, big_map, small_tasks, counters, bounds, split;
+  DevMem box_lo, box_hi, geoms, pgeom;
+  DevMem lo, hi, slot_task, windows, tasks, task_node, bounds, bins, split, mid_tasks, counters;
+  DevMem collapse, levels;
 };
 
 struct Device {
@@ -225,8 +228,9 @@ struct Frame {
   DevMem dn_in, dn_normal, dn_out;
 };
 
-// builder entry (bnx_bvh.hip): boxes in d_lo/d_hi (float4, n); returns host info
-int build_bvh(Device *dev, const float4 *d_lo, const float4 *d_hi, int n, int max_leaf, Bvh &out);
+// builder entry (bnx_bvh.hip): boxes in d_lo/d_hi (float4, n; d_lo.w holds
+// the primitive's index as bits), which the build permutes; returns host info
+int build_bvh(Device *dev, float4 *d_lo, float4 *d_hi, int n, int max_leaf, Bvh &out);
 // collapse the built binary BVH into 4-wide nodes (out.nodes4)
 int collapse_bvh4(Device *dev, Bvh &bvh);
 // trace-pool refill threshold for the secondary rays of a world: refilling

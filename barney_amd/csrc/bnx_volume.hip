@@ -96,7 +96,7 @@ BNX_D void cell_box(const int4 *tets, const int4 *ext, const uint8_t *types, con
   }
 }
 
-// world-space box of every cell (element-BVH build input); ext and types
+// world-space box and index of every cell (element-BVH build input); ext and types
 // null: every cell is a tet
 __global__ void k_cell_boxes(const int4 *tets, const int4 *ext, const uint8_t *types, const float4 *verts, int n,
                              float4 *lo, float4 *hi)
@@ -105,7 +105,7 @@ __global__ void k_cell_boxes(const int4 *tets, const int4 *ext, const uint8_t *t
   if (t >= n) return;
   float4 l, h;
   cell_box(tets, ext, types, verts, t, l, h);
-  lo[t] = make_float4(l.x, l.y, l.z, 0.f);
+  lo[t] = make_float4(l.x, l.y, l.z, __int_as_float(t));
   hi[t] = make_float4(h.x, h.y, h.z, 0.f);
 }
 
@@ -589,7 +589,8 @@ int volume_build_umesh(Volume *v, const int4 *tets4, const int4 *ext4, const uin
   const bool mixed = types != nullptr;
   BNX_HIP(v->uverts.ensure(sizeof(float4) * (size_t)nvert));
   BNX_HIP(hipMemcpyAsync(v->uverts.ptr, verts4, sizeof(float4) * (size_t)nvert, hipMemcpyHostToDevice, st));
-  DevMem tets, ext, typ, lo, hi, rlo, rhi;
+  DevMem tets, ext, typ, rlo, rhi;
+  DevMem &lo = dev->build.box_lo, &hi = dev->build.box_hi;
   BNX_HIP(tets.ensure(sizeof(int4) * (size_t)ntet));
   BNX_HIP(hipMemcpyAsync(tets.ptr, tets4, sizeof(int4) * (size_t)ntet, hipMemcpyHostToDevice, st));
   if (mixed) {
