@@ -1139,6 +1139,17 @@ static int set_tf(Volume *v, const bnx_transfer_function *tf)
   v->dd.dom0 = tf->domain[0];
   v->dd.dom1 = tf->domain[1];
   v->dd.base_density = tf->base_density;
+  v->dd.rcp_span = 1.f / (tf->domain[1] - tf->domain[0]);
+  // majorants are alphas of the map, or weighted means of two, times the
+  // density: with these bounds they and the quotients by them stay far from
+  // the ends of the float range
+  auto in = [](float x, float lo, float hi) { return x >= lo && x <= hi; };
+  bool rn = in(tf->base_density, 0x1p-30f, 0x1p30f) && in(tf->domain[1] - tf->domain[0], 0x1p-60f, 0x1p60f);
+  for (int i = 0; i < tf->num_values && rn; i++) {
+    const float a = tf->values[4 * i + 3];
+    rn = a == 0.f || in(a, 0x1p-20f, 0x1p20f);
+  }
+  v->dd.rn = rn && v->grid_rn;
   v->version++;
   return BNX_OK;
 }
@@ -1177,6 +1188,9 @@ int bnx_volume_create_structured(bnx_device d, const bnx_structured_desc *f, con
     dd.mc_origin[k] = dd.lo[k];
     dd.mc_rcp_spacing[k] = 1.f / ((float)c * f->grid_spacing[k]);
   }
+  v->grid_rn = true;
+  for (int k = 0; k < 3; k++)
+    v->grid_rn = v->grid_rn && dd.mc_rcp_spacing[k] >= 0x1p-40f && dd.mc_rcp_spacing[k] <= 0x1p40f;
   dd.user_id = user_id;
   // the sampler reads the linear array unless BNX_VOLUME_BRICK asks for a
   // bricked copy (bricks of 2^shift cells a side with a one-texel apron); a
@@ -1186,7 +1200,8 @@ int bnx_volume_create_structured(bnx_device d, const bnx_structured_desc *f, con
   // the latency of its dependent gathers, not by their bytes
   int shift = 0;
   if (const char *e = getenv("BNX_VOLUME_BRICK")) shift = std::min(5, std::max(0, atoi(e)));
-  if ((rc = set_tf(v, tf)) != BNX_OK || (rc = volume_build(v)) != BNX_OK || (rc = volume_brick(v, shift)) != BNX_OK) {
+  if ((rc = set_tf(v, tf)) != BNX_OK || (rc = volume_build(v)) != BNX_OK || (rc = volume_brick(v, shift)) != BNX_OK ||
+      (shift == 0 && (rc = volume_corners(v)) != BNX_OK)) {
     delete v;
     return rc;
   }
@@ -1278,7 +1293,6 @@ int bnx_volume_create_umesh(bnx_device d, const bnx_umesh_desc *f, const bnx_tra
   bnx_volume v = new bnx_volume_s;
   v->dev = d;
   VolumeDev &dd = v->dd;
-  dd.field = FIELD_UMESH;
   // computeWorldBounds (UMeshField.cu:304-318): union of the cells' boxes
   float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
   for (int c = 0; c < nc; c++) {
@@ -1311,6 +1325,9 @@ int bnx_volume_create_umesh(bnx_device d, const bnx_umesh_desc *f, const bnx_tra
     const float spacing = size[k] * (1.f / (float)dd.mc[k]);
     dd.mc_rcp_spacing[k] = 1.f / spacing;
   }
+  v->grid_rn = true;
+  for (int k = 0; k < 3; k++)
+    v->grid_rn = v->grid_rn && dd.mc_rcp_spacing[k] >= 0x1p-40f && dd.mc_rcp_spacing[k] <= 0x1p40f;
   dd.user_id = user_id;
   int rc;
   if ((rc = set_tf(v, tf)) != BNX_OK ||

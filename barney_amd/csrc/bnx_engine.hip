@@ -73,14 +73,14 @@ constexpr int SORT_MIN_RAYS = 1 << 16;
 struct BatchShape {
   long long count0 = 0, cap = 0;
   bool surfaces = false, volumes = false;
-  int full = 0;       // the march kernel: 0 lean, else MARCH_FULL / MARCH_CELLS bits
+  MarchKind march;
   int refill = 64, stack = 16, walk = 0, blocks_per_cu = 8, shade_block = 1024;
   bool ext = false;   // the trace kernels with the cylinder test and the cut plane
   bool xf = false;    // the trace kernels that change the ray's frame at instances
   bool operator<(const BatchShape &o) const
   {
-    return std::tie(count0, cap, surfaces, volumes, full, refill, stack, walk, blocks_per_cu, shade_block, ext, xf) <
-           std::tie(o.count0, o.cap, o.surfaces, o.volumes, o.full, o.refill, o.stack, o.walk, o.blocks_per_cu,
+    return std::tie(count0, cap, surfaces, volumes, march.fields, march.isos, march.vols, refill, stack, walk, blocks_per_cu, shade_block, ext, xf) <
+           std::tie(o.count0, o.cap, o.surfaces, o.volumes, o.march.fields, o.march.isos, o.march.vols, o.refill, o.stack, o.walk, o.blocks_per_cu,
                     o.shade_block, o.ext, o.xf);
   }
 };
@@ -96,7 +96,7 @@ struct BatchGraph {
 // queues, tables and staging of one wavefront
 struct Wavefront {
   Queues Q;
-  DevMem slots, chunks, segs, blk256, blk1024, blkT, pool, out_base, out_cnt;
+  DevMem slots, chunks, segs, blk256, blk1024, blkT, pool, claims, out_base, out_cnt;
   Pinned h_slots, h_chunks, h_segs, h_out_base, h_out_cnt;
   int slot_cap = 0, chunk_cap = 0, seg_cap = 0;
   // device-driven bounce loops: per-generation counts, timing events (four
@@ -131,7 +131,7 @@ struct Wavefront {
     std::vector<const void *> b = {Q.org[0].ptr, Q.org[1].ptr, Q.dir[0].ptr, Q.dir[1].ptr, Q.rng[0].ptr,
                                    Q.rng[1].ptr, Q.ps[0].ptr, Q.ps[1].ptr, Q.hit[0].ptr, Q.hit[1].ptr,
                                    Q.hit_v[0].ptr, Q.hit_v[1].ptr, Q.vcol[0].ptr, Q.vcol[1].ptr, Q.stats.ptr,
-                                   slots.ptr, segs.ptr, blk256.ptr, blk1024.ptr, blkT.ptr, pool.ptr,
+                                   slots.ptr, segs.ptr, blk256.ptr, blk1024.ptr, blkT.ptr, pool.ptr, claims.ptr,
                                    out_base.ptr, out_cnt.ptr, gen_counts.ptr, stamps.ptr};
     if (b != graph_bufs) {
       drop_graphs();
@@ -177,6 +177,7 @@ struct Wavefront {
       BNX_HIP(segs.ensure(sizeof(Segment) * nsegs));
       BNX_HIP(h_segs.ensure(sizeof(Segment) * nsegs));
       BNX_HIP(pool.ensure(sizeof(int) * nsegs));
+      BNX_HIP(claims.ensure(march_claims_bytes()));
       seg_cap = nsegs;
     }
     // every segment adds at most one partial block
@@ -229,7 +230,8 @@ struct GenTiming {
 // Enqueue one generation over queue `cur`: upload the segments, build the
 // block maps, trace, volume march, shade into queue 1 - cur.  The caller
 // has uploaded the output region bases and cleared the output counters.
-int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool surfaces, bool volumes, int full)
+int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool surfaces, bool volumes,
+                       const MarchKind &march)
 {
   Queues &Q = F.Q;
   RayQueue in = Q.q(cur), out = Q.q(1 - cur);
@@ -239,7 +241,7 @@ int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool sur
   sl.layout_trace(dev->trace_blocks_per_cu * dev->num_cus);
   BNX_HIP(hipMemcpyAsync(F.segs.ptr, sl.v, sizeof(Segment) * sl.n, hipMemcpyHostToDevice, dev->stream));
   const SegView sv{F.segs.as<Segment>(), F.blk256.as<int>(), F.blk1024.as<int>(), F.blkT.as<int>(),
-                   F.pool.as<int>()};
+                   F.pool.as<int>(), F.claims.as<int>()};
   if ((rc = launch_segment_blocks(dev, sv, sl.n, sl.blocks256, sl.blocks1024, sl.blocksT)) != BNX_OK) return rc;
   TraceQueue tq{in.org, in.dir, in.hit, in.hit_v, in.rng, in.ps};
   // with neither surfaces nor volumes the trace kernel still writes the misses
@@ -257,7 +259,7 @@ int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool sur
   if (timed) BNX_HIP(hipEventRecord(Q.ev_end, dev->stream));
   if (volumes) {
     if (timed) BNX_HIP(hipEventRecord(Q.ev_vbegin, dev->stream));
-    if ((rc = launch_volume_march(dev, slots, sv, sl.blocks256, in, trace, full, st)) != BNX_OK) return rc;
+    if ((rc = launch_volume_march(dev, slots, sv, sl.n, sl.blocks256, in, trace, march, st)) != BNX_OK) return rc;
     if (timed) BNX_HIP(hipEventRecord(Q.ev_vend, dev->stream));
   }
   const SlotOut so{F.out_base.as<int>(), F.out_cnt.as<int>()};
@@ -277,7 +279,7 @@ int enqueue_dd(Device *dev, Wavefront &F, int cur0, int G, const BatchShape &b)
   unsigned long long *st = Q.stats.as<unsigned long long>();
   const SlotDev *slots = F.slots.as<SlotDev>();
   const SegView sv{F.segs.as<Segment>(), F.blk256.as<int>(), F.blk1024.as<int>(), F.blkT.as<int>(),
-                   F.pool.as<int>()};
+                   F.pool.as<int>(), F.claims.as<int>()};
   const SlotOut so{F.out_base.as<int>(), F.out_cnt.as<int>()};
   const bool trace = b.surfaces || !b.volumes;
   const long long target = (long long)dev->trace_blocks_per_cu * dev->num_cus;
@@ -308,7 +310,7 @@ int enqueue_dd(Device *dev, Wavefront &F, int cur0, int G, const BatchShape &b)
     }
     if (b.volumes) {
       if ((rc = launch_stamp(dev, ts + 2)) != BNX_OK) return rc;
-      if ((rc = launch_volume_march(dev, slots, sv, blocks256, in, trace, b.full, st)) != BNX_OK) return rc;
+      if ((rc = launch_volume_march(dev, slots, sv, 1, blocks256, in, trace, b.march, st)) != BNX_OK) return rc;
       if ((rc = launch_stamp(dev, ts + 3)) != BNX_OK) return rc;
     }
     if ((rc = launch_shade(dev, slots, sv, blocks256, blocks1024, in, out, so, st)) != BNX_OK) return rc;
@@ -404,10 +406,8 @@ int trace_refill_for(const Device *dev, const World *w)
 
 namespace {
 
-// full: the march kernel the world needs (MARCH_FULL: it has isosurfaces or
-// unstructured volumes; MARCH_CELLS: some unstructured field has other cells
-// than tets)
-int fill_slot(World *w, const bnx_camera &cam, const bnx_renderer &rr, Frame *f, SlotDev &s, int &full)
+// march: what the world's rays have to be marched through
+int fill_slot(World *w, const bnx_camera &cam, const bnx_renderer &rr, Frame *f, SlotDev &s, MarchKind &march)
 {
   VolumeList vl{};
   int rc = world_volumes(w, vl);
@@ -417,9 +417,9 @@ int fill_slot(World *w, const bnx_camera &cam, const bnx_renderer &rr, Frame *f,
   s.vols = vl.vols;
   s.num_vols = vl.count;
   if ((rc = world_isos(w, s.isos, s.num_isos)) != BNX_OK) return rc;
-  full = s.num_isos > 0 ? MARCH_FULL : 0;
-  for (const Volume *v : w->volumes) full |= march_kind(v);
-  for (const IsoSurface *iso : w->isos) full |= march_kind(iso->field);
+  march = MarchKind{0, s.num_isos, s.num_vols};
+  for (const Volume *v : w->volumes) march.fields |= 1 << v->dd.field;
+  for (const IsoSurface *iso : w->isos) march.fields |= 1 << iso->field->dd.field;
   BNX_SET(s.dir_lights, w->d_dir_lights.ptr);
   s.num_dir_lights = (int)w->dir_lights.size();
   s.env = env_dev(w);
@@ -482,8 +482,8 @@ int render_frame_impl(World *w, const bnx_camera &cam, const bnx_renderer &rr, F
       BNX_OK)
     return rc;
   SlotDev *hs = F.h_slots.as<SlotDev>();
-  int full = 0;
-  if ((rc = fill_slot(w, cam, rr, f, *hs, full)) != BNX_OK) return rc;
+  MarchKind march;
+  if ((rc = fill_slot(w, cam, rr, f, *hs, march)) != BNX_OK) return rc;
   const bool surfaces = hs->scene.num_insts > 0;
   const bool volumes = hs->num_vols > 0 || hs->num_isos > 0;
   const bool traced = surfaces || !volumes;
@@ -511,7 +511,7 @@ int render_frame_impl(World *w, const bnx_camera &cam, const bnx_renderer &rr, F
     // below), run that many as one captured bounce loop with one read-back
     const bool dd = !F.noalloc && dev->graph_paths > 0 && np * nS <= dev->graph_paths;
     const BatchShape shape{np * nS,          2 * np * nS,           surfaces,
-                           volumes,          full,                  trace_refill_for(dev, w),
+                           volumes,          march,                 trace_refill_for(dev, w),
                            dev->trace_stack_lds, dev->trace_walk, dev->trace_blocks_per_cu, dev->shade_block,
                            ext_kernels(dev, has_cut_plane(rr)), dev->xf_worlds > 0};
     int dd_gens = 0;
@@ -574,7 +574,7 @@ int render_frame_impl(World *w, const bnx_camera &cam, const bnx_renderer &rr, F
       SegList sl{F.h_segs.as<Segment>()};
       sl.add(0, 0, count, primary ? 64 : trace_refill_for(dev, w));
       if ((rc = zero_words(dev, F.out_cnt.ptr, 2 * sizeof(int), F.noalloc)) != BNX_OK) return rc;
-      if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, full)) != BNX_OK) return rc;
+      if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, march)) != BNX_OK) return rc;
       BNX_HIP(hipMemcpyAsync(hcnt, F.out_cnt.ptr, 2 * sizeof(int), hipMemcpyDeviceToHost, dev->stream));
       BNX_HIP(hipStreamSynchronize(dev->stream));
       if ((rc = collect_timing(F, count, traced, volumes, tm)) != BNX_OK) return rc;
@@ -636,11 +636,12 @@ constexpr long long NOALLOC_PATHS = 1LL << 16;
 constexpr size_t NOALLOC_RAYS = 2 * (size_t)NOALLOC_PATHS;
 constexpr size_t NOALLOC_BLOCKS = NOALLOC_RAYS / 256 + 2;   // one segment: one partial block at most
 constexpr size_t al256(size_t b) { return (b + 255) / 256 * 256; }
+constexpr size_t NOALLOC_CLAIMS = 16384;   // march_claims_bytes()
 constexpr size_t NOALLOC_QUEUE_BYTES =
     al256(16 * NOALLOC_RAYS) * 5 + al256(8 * NOALLOC_RAYS) + al256(4 * NOALLOC_RAYS);   // one queue
 constexpr size_t NOALLOC_BYTES = 2 * NOALLOC_QUEUE_BYTES + al256(8 * STAT_COUNT * STAT_SLOTS) +
                                  al256(sizeof(SlotDev)) + al256(sizeof(RaygenChunk)) + al256(sizeof(Segment)) +
-                                 4 * 256 + 3 * al256(4 * NOALLOC_BLOCKS);
+                                 4 * 256 + NOALLOC_CLAIMS + 3 * al256(4 * NOALLOC_BLOCKS);
 
 // The scratch memory of bnx_render_noalloc: one copy per GPU the library
 // runs on, held until the process ends.  Host code never passes this name to
@@ -678,6 +679,7 @@ void noalloc_layout(NoallocWavefront &N, unsigned char *base)
   take(F.chunks, sizeof(RaygenChunk));
   take(F.segs, sizeof(Segment));
   take(F.pool, 4);
+  take(F.claims, NOALLOC_CLAIMS);
   take(F.out_base, 4);
   take(F.out_cnt, 8);
   take(F.blk256, 4 * NOALLOC_BLOCKS);
@@ -926,7 +928,7 @@ struct Request {
   double cost_ms = 0.0;            // share of step time by its rays in each step
   double deadline_ms = -1.0;       // set at admission when the top-up is deadline-ordered
   bool surfaces = false, volumes = false;
-  int full = 0;
+  MarchKind march;
 };
 
 // measured cost of a world's paths: step time attributed to completed
@@ -1038,7 +1040,7 @@ struct Server {
       r->slot = free_slots.back();
       free_slots.pop_back();
       SlotDev *hs = F.h_slots.as<SlotDev>() + r->slot;
-      if ((rc = fill_slot(r->world, r->cam, r->rr, f, *hs, r->full)) != BNX_OK) {
+      if ((rc = fill_slot(r->world, r->cam, r->rr, f, *hs, r->march)) != BNX_OK) {
         // the request fails: its slot and its frame go back, it leaves the
         // queue, and its ticket reads BNX_REQ_FAILED until released
         free_slots.push_back(r->slot);
@@ -1152,14 +1154,14 @@ struct Server {
     int *hb = F.h_out_base.as<int>();
     long long out_end = 0;
     bool surfaces = false, volumes = false;
-    int full = 0;
+    MarchKind march;
     int max_slot = 0;
     for (Request *r : active) {
       hb[r->slot] = (int)out_end;
       out_end += 2LL * (r->live_paths + r->added);
       surfaces |= r->surfaces;
       volumes |= r->volumes;
-      full |= r->full;
+      march.merge(r->march);
       max_slot = std::max(max_slot, r->slot + 1);
     }
     BNX_HIP(hipMemcpyAsync(F.out_base.ptr, hb, sizeof(int) * max_slot, hipMemcpyHostToDevice, dev->stream));
@@ -1170,7 +1172,7 @@ struct Server {
                               F.Q.q(cur))) != BNX_OK)
         return rc;
     }
-    if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, full)) != BNX_OK) return rc;
+    if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, march)) != BNX_OK) return rc;
     int *hcnt = F.h_out_cnt.as<int>();
     BNX_HIP(hipMemcpyAsync(hcnt, F.out_cnt.ptr, sizeof(int) * 2 * max_slot, hipMemcpyDeviceToHost, dev->stream));
     BNX_HIP(hipStreamSynchronize(dev->stream));
@@ -1231,7 +1233,7 @@ struct Server {
     const int A = (int)active.size(), O = (int)order.size();
     long long rays0 = 0, paths = 0, rem = 0;
     bool surfaces = false, volumes = false, pooled = false, cut = false;
-    int full = 0;
+    MarchKind march;
     int max_slot = 0;
     for (int i = 0; i < A; i++) {
       Request *r = active[i];
@@ -1243,7 +1245,7 @@ struct Server {
       rem += r->total_paths - r->next_path;
       surfaces |= r->surfaces;
       volumes |= r->volumes;
-      full |= r->full;
+      march.merge(r->march);
       pooled |= refill < 64;
       cut |= has_cut_plane(r->rr);
       max_slot = std::max(max_slot, r->slot + 1);
@@ -1263,7 +1265,7 @@ struct Server {
                     F.chunks.as<RaygenChunk>(), F.out_base.as<int>(), F.out_cnt.as<int>(),
                     d_scal.as<long long>(), F.gen_counts.as<long long>(), max_paths, target};
     const SegView sv{F.segs.as<Segment>(), F.blk256.as<int>(), F.blk1024.as<int>(), F.blkT.as<int>(),
-                     F.pool.as<int>()};
+                     F.pool.as<int>(), F.claims.as<int>()};
     const SlotOut so{F.out_base.as<int>(), F.out_cnt.as<int>()};
     const SlotDev *slots = F.slots.as<SlotDev>();
     unsigned long long *stat = F.Q.stats.as<unsigned long long>();
@@ -1289,7 +1291,7 @@ struct Server {
       }
       if (volumes) {
         if ((rc = launch_stamp(dev, tsp + 2)) != BNX_OK) return rc;
-        if ((rc = launch_volume_march(dev, slots, sv, blocks256, in, trace, full, stat)) != BNX_OK) return rc;
+        if ((rc = launch_volume_march(dev, slots, sv, nsegs, blocks256, in, trace, march, stat)) != BNX_OK) return rc;
         if ((rc = launch_stamp(dev, tsp + 3)) != BNX_OK) return rc;
       }
       if ((rc = launch_shade(dev, slots, sv, blocks256, blocks1024, in, out, so, stat)) != BNX_OK) return rc;

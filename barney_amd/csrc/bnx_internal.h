@@ -109,6 +109,7 @@ struct Device {
   int trace_blocks_per_cu = 8;   // trace launch size: blocks per CU
   long long render_paths = 8LL << 20;       // bnx_render: paths per batch
   long long graph_paths = 4LL << 20;        // bnx_render: batches this small run a captured bounce loop
+  int march_fit[6] = {0, 0, 0, 0, 0, 0};   // waves per CU of the march kernels (0: not asked yet)
   BuildScratch build;
   DevMem counters;      // small device counters (trace work queue etc.)
   void *queues = nullptr;   // render queues (bnx_render.h Queues)

@@ -101,6 +101,7 @@ struct SegView {
   const int *blk1024;          // segment of each 1024-thread block
   const int *blkT;             // segment of each trace block
   int *pool;                   // per segment: next ray of the trace pool
+  int *claims;                 // the march launches' chunk counters, cleared with the block maps
 };
 
 // shade output of one generation: request slot s appends to its own region
@@ -197,6 +198,10 @@ int sort_rays(Device *dev, SortScratch &S, const RayQueue &src, const RayQueue &
               const float hi[3]);
 // fill the block -> segment maps of nsegs segments (blocks256 / blocks1024 /
 // blocksT blocks in all) and reset the segments' trace pools
+// launches of a generation's march whose counters the block maps' kernel
+// clears, and their bytes
+constexpr int MARCH_PROGRAMS = 8;
+size_t march_claims_bytes();
 int launch_segment_blocks(Device *dev, const SegView &sv, int nsegs, int blocks256, int blocks1024, int blocksT);
 // shade every ray of the segments (blocks256 blocks of 256 threads or
 // blocks1024 of 1024, by the device's shade_block),

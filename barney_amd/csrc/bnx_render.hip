@@ -755,9 +755,11 @@ __global__ __launch_bounds__(SHADE_BLOCK) void k_shade(const SlotDev *__restrict
 }
 
 // block -> segment maps: one thread per block of either launch width
-__global__ void k_segment_blocks(SegView sv, int nsegs, int blocks256, int blocks1024, int blocksT)
+__global__ void k_segment_blocks(SegView sv, int nsegs, int blocks256, int blocks1024, int blocksT, int claims)
 {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < claims; i += blockDim.x) sv.claims[i] = 0;
   const Segment *segs = sv.segs;
   // the pool of segment b starts after its static part: 256 rays (one chunk
   // per wave) for each of its trace blocks
@@ -1057,7 +1059,8 @@ int launch_segment_blocks(Device *dev, const SegView &sv, int nsegs, int blocks2
 {
   const int n = std::max(std::max(blocks256, blocksT), nsegs);
   if (nsegs > 0 && n > 0)
-    k_segment_blocks<<<nblk(n, 256), 256, 0, dev->stream>>>(sv, nsegs, blocks256, blocks1024, blocksT);
+    k_segment_blocks<<<nblk(n, 256), 256, 0, dev->stream>>>(sv, nsegs, blocks256, blocks1024, blocksT,
+                                                             (int)(march_claims_bytes() / sizeof(int)));
   BNX_HIP(hipGetLastError());
   return BNX_OK;
 }

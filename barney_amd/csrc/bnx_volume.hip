@@ -1,24 +1,16 @@
-// bnx_volume.hip -- volumes and isosurfaces on gfx950: structured and
-// tetrahedral fields, macrocell value ranges, majorants, and the DDA +
-// Woodcock (delta tracking) and isosurface march.
+// bnx_volume.hip -- volumes on gfx950: structured and unstructured fields,
+// macrocell value ranges and majorants.
 //
-// Replaces MCVolumeAccel (volume/MCAccelerator.h:155-195, 550-689) and
-// MCIsoSurfaceAccel (:325-548) over StructuredDataSampler and
-// UMeshCuBQLSampler, StructuredData_computeMCs (volume/StructuredData.cu:
-// 30-62), umeshRasterCells (umesh/common/UMeshField.cu:28-161), mapMCs
-// (volume/MCGrid.cu:96-113), dda3 (volume/DDA.h:60-201) and
-// Woodcock::sampleRange (volume/Volume.h:154-203).
+// Replaces MCVolumeAccel's build (volume/MCAccelerator.h:155-195) over
+// StructuredDataSampler and UMeshCuBQLSampler, StructuredData_computeMCs
+// (volume/StructuredData.cu:30-62), umeshRasterCells (umesh/common/
+// UMeshField.cu:28-161) and mapMCs (volume/MCGrid.cu:96-113).
 //
-// Design: isosurfaces and volumes are handled in their own wavefront kernel
-// after the surface trace (one thread per queued ray), clipped to the
-// closest hit so far.  The march is long, data-dependent and gather-bound,
-// so keeping it out of the BVH traversal kernel keeps that kernel's
-// registers and divergence low.  Structured fields are filtered in software
-// on the raw float grid (hardware texture filtering uses 8-bit fixed-point
-// weights); a 256^3 field is 64 MiB and stays resident in the 256 MiB
-// Infinity Cache.  Tet fields keep vertices as float4 (position, scalar: one
-// 16-byte load per corner) and tets as int4 in element-BVH slot order; the
-// point query's stack is a 16-entry ring per thread in LDS.
+// Structured fields are filtered in software on the raw float grid (hardware
+// texture filtering uses 8-bit fixed-point weights); a 256^3 field is 64 MiB
+// and stays resident in the 256 MiB Infinity Cache.  Unstructured fields keep
+// each cell's vertices (position, scalar) together in element-BVH slot order.
+// The march itself is in bnx_march.hip.
 #include "bnx_internal.h"
 #include "bnx_render.h"
 #include "bnx_volume.h"
@@ -109,34 +101,67 @@ __global__ void k_cell_boxes(const int4 *tets, const int4 *ext, const uint8_t *t
   hi[t] = make_float4(h.x, h.y, h.z, 0.f);
 }
 
-// cells in element-BVH slot order
-__global__ void k_cell_sort(const int4 *tets, const int4 *ext, const uint8_t *types, const int *order, int n,
-                            int4 *tets_out, int4 *ext_out, uint8_t *types_out)
+// tets in element-BVH slot order
+__global__ void k_tet_sort(const int4 *tets, const int *order, int n, int4 *out)
 {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  const int c = order[s];
-  tets_out[s] = tets[c];
-  if (types) {
-    ext_out[s] = ext[c];
-    types_out[s] = types[c];
-  }
+  if (s < n) out[s] = tets[order[s]];
 }
 
-// the 80-byte tet records (VolumeDev::utetv) in slot order: four vertices
-// and the face neighbours
-__global__ void k_tet_pack(const int4 *tets, const float4 *verts, const int4 *nbr, int n, float4 *rec)
+// the 128-byte tet records (VolumeDev::utetv) in slot order; lo, hi: the
+// mesh's bounds
+__global__ void k_tet_pack(const int4 *tets, const float4 *verts, const int4 *nbr, int n, v3 lo, v3 hi, float4 *rec)
 {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
-  const int4 t = tets[s];
-  float4 *r = rec + 5 * (size_t)s;
-  r[0] = verts[t.x];
-  r[1] = verts[t.y];
-  r[2] = verts[t.z];
-  r[3] = verts[t.w];
-  const int4 b = nbr[s];
-  r[4] = make_float4(__int_as_float(b.x), __int_as_float(b.y), __int_as_float(b.z), __int_as_float(b.w));
+  const int4 t = tets[s], b = nbr[s];
+  const float4 v0 = verts[t.x], v1 = verts[t.y], v2 = verts[t.z], w = verts[t.w];
+  float4 *r = rec + TET_REC * (size_t)s;
+  auto face = [&](float4 a, float4 p, float4 q, int nb) {
+    if (nb < 0) {
+      auto on = [&](float x, float y, float z, float l, float h) { return x == y && y == z && (x == l || x == h); };
+      nb = on(a.x, p.x, q.x, lo.x, hi.x) || on(a.y, p.y, q.y, lo.y, hi.y) || on(a.z, p.z, q.z, lo.z, hi.z) ? TET_HULL
+                                                                                                    : TET_OPEN;
+    }
+    const v3 N = cross(xyz(p) - xyz(a), xyz(q) - xyz(a));
+    return make_float4(N.x, N.y, N.z, __int_as_float(nb));
+  };
+  r[0] = face(v1, w, v2, b.x);
+  r[1] = face(v0, v2, w, b.y);
+  r[2] = face(v0, w, v1, b.z);
+  r[3] = face(v0, v1, v2, b.w);
+  r[4] = v0;
+  r[5] = v1;
+  r[6] = make_float4(v2.w, w.w, 0.f, 0.f);
+}
+
+// Cells in element-BVH slot order: 128 bytes of vertices, and the filter box
+// that a point query tests before a cell's Newton inversion.  A point that
+// the inversion accepts lies in the hull of the cell's vertices but for the
+// domain's margin (1e-6), the last Newton step (below 1e-4 of the cell in
+// each parameter) and the rounding of coordinates: a twentieth of the
+// cell's extent and 1e-5 of the coordinates hold all of that many times
+// over.  A tet's own test accepts what its planes accept, however thin the
+// tet: its box is open.
+__global__ void k_cell_pack(const int4 *tets, const int4 *ext, const uint8_t *types, const float4 *verts,
+                            const int *order, int n, float4 *rec, float4 *box)
+{
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;
+  const int c = order[s], type = types[c], nv = cell_nverts(type);
+  float4 *r = rec + 8 * (size_t)s;
+  for (int k = 0; k < 8; k++) r[k] = cell_vertex(tets, ext, verts, c, k < nv ? k : 0);
+  float4 lo, hi;
+  cell_box(tets, ext, types, verts, c, lo, hi);
+  float m = INFINITY;
+  if (type != CELL_TET) {
+    const float size = fmx(fmx(hi.x - lo.x, hi.y - lo.y), hi.z - lo.z);
+    const float far = fmx(fmx(fmx(fabsf(lo.x), fabsf(hi.x)), fmx(fabsf(lo.y), fabsf(hi.y))),
+                          fmx(fabsf(lo.z), fabsf(hi.z)));
+    m = .05f * size + 1e-5f * far;
+  }
+  box[2 * (size_t)s] = make_float4(lo.x - m, lo.y - m, lo.z - m, __int_as_float(type));
+  box[2 * (size_t)s + 1] = make_float4(hi.x + m, hi.y + m, hi.z + m, 0.f);
 }
 
 __global__ void k_fill_ranges(int *lo, int *hi, int n)
@@ -263,129 +288,6 @@ __global__ void k_umesh_raster(const int4 *tets, const int4 *ext, const uint8_t 
   cache.flush(rlo, rhi);
 }
 
-// ----------------------------------------------------------------- march
-// March every ray of the generation's segments through its request's
-// isosurfaces (first) and volumes, one ray per thread, each clipped to the
-// closest hit so far; each block lies inside one request's segment, so the
-// tables are block-uniform.  With no surface instances in the batch the
-// trace kernel is skipped and every ray enters here as a surface miss
-// (surfaces == 0).  MODE 0: every volume of the batch is structured and
-// there are no isosurfaces; MARCH_FULL: isosurfaces and unstructured fields
-// may occur; with MARCH_CELLS, fields with other cells than tets too (a
-// kernel of its own: the cells' Newton inversions would otherwise raise the
-// register pressure of the tet kernel).
-// waves per SIMD the march kernel is compiled for, lean and full variant.
-// The full variant (tet point location + isosurfaces) needs 126 VGPRs to
-// run without spilling, which allows 4 waves per SIMD.  Compiled for 6 (80
-// VGPRs) it spills 112 of them to scratch, and the spill stores then make up
-// most of its memory writes (4.9 GB per launch against 0.95 GB at 4 waves),
-// yet on the 20.5M-tet volume with an isosurface (1024^2, 32 spp) a launch
-// takes 24.2 ms against 27.9 ms at 4 waves and 25.2 ms at 5 (40 spilled):
-// the dependent gathers of the point queries need the extra waves to hide
-// their latency more than the spills cost.  Splitting the kernel into an
-// isosurface pass and a volume pass would not remove the spills (each alone
-// spills 46 and 64 VGPRs at 6 waves).
-#ifndef BNX_MARCH_WAVES_LEAN
-#define BNX_MARCH_WAVES_LEAN 5
-#endif
-#ifndef BNX_MARCH_WAVES_FULL
-#define BNX_MARCH_WAVES_FULL 6
-#endif
-template <int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE ? BNX_MARCH_WAVES_FULL
-                                                                          : BNX_MARCH_WAVES_LEAN))) void
-k_volume_march(const SlotDev *__restrict__ slots, SegView sv, RayQueue q,
-                                                      int surfaces, unsigned long long *stats)
-{
-  constexpr bool FULL = MODE != 0, CELLS = (MODE & MARCH_CELLS) != 0;
-  __shared__ uint32_t ring[FULL ? PQ_SHORT * PQ_TB : 1];
-  MarchCtx cx{ring + threadIdx.x, 0, 0, 0, 0};
-  int i;
-  bool valid;
-  const Segment sg = segment_of<256>(sv, i, valid);
-  const SlotDev &SL = slots[sg.slot];
-  const VolumeList vl{SL.vols, SL.num_vols};
-  const IsoDev BNX_G *isos = SL.isos;
-  const int niso = FULL ? SL.num_isos : 0;
-  if (valid) {
-    float4 o = q.org[i];
-    float4 d = q.dir[i];
-    int4 hit = surfaces ? q.hit[i] : make_int4(-1, -1, -1, 0);
-    const bool shadow = (__float_as_uint(d.w) & FLAG_SHADOW) != 0;
-    if (!(shadow && hit.x >= 0)) {                 // an occluded shadow ray is done
-      const v3 org = xyz(o), dir = fix_dir(xyz(d));
-      float tcur = o.w;
-      uint64_t rng = q.rng[i];
-      const uint64_t rng0 = rng;
-      int ik = -1;
-      float it = 0.f;
-      v3 iN = splat(0.f);
-      for (int k = 0; k < niso; k++) {
-        float t;
-        v3 N;
-        if (iso_march<CELLS>(isos[k], org, dir, 0.f, tcur, rng, t, N, cx)) {
-          ik = k;
-          it = t;
-          iN = N;
-          tcur = t;
-          if (shadow) break;
-        }
-      }
-      int vk = -1;
-      float vt = 0.f, rgb[3] = {0.f, 0.f, 0.f};
-      // ratio tracking: a shadow ray's transmittance estimate through the
-      // volumes scales its MIS weight (the light sample it carries); zero
-      // transmittance occludes it as a delta-tracking event does
-      const bool ratio = shadow && (SL.rr.flags & BNX_RENDER_RATIO_TRACKING) != 0;
-      float T = 1.f;
-      for (int k = 0; k < vl.count && !(shadow && ik >= 0); k++) {
-        float t, c[3];
-        if (ratio) {
-          T *= ratio_track<FULL, CELLS>(vl.vols[k], org, dir, 0.f, tcur, rng, cx);
-          if (T == 0.f) {
-            vk = k;
-            vt = tcur;
-            break;
-          }
-          continue;
-        }
-        if (volume_march<FULL, CELLS>(vl.vols[k], org, dir, 0.f, tcur, rng, t, c, cx)) {
-          vk = k;
-          vt = t;
-          tcur = t;
-          rgb[0] = c[0]; rgb[1] = c[1]; rgb[2] = c[2];
-          if (shadow) break;
-        }
-      }
-      if (rng != rng0) q.rng[i] = rng;
-      if (ratio && vk < 0 && T < 1.f) q.ps[i].w = __float_as_uint(__uint_as_float(q.ps[i].w) * T);
-      if (vk >= 0) {
-        q.org[i].w = vt;
-        hit = make_int4(0, VOLUME_GEOM_BASE + vk, vl.vols[vk].rtc_inst, 0);
-        q.vcol[i] = make_float4(rgb[0], rgb[1], rgb[2], 0.f);
-        q.hit[i] = hit;
-      } else if (FULL && ik >= 0) {
-        q.org[i].w = it;
-        hit = make_int4(0, ISO_GEOM_BASE + ik, isos[ik].rtc_inst, 0);
-        q.vcol[i] = make_float4(iN.x, iN.y, iN.z, 0.f);
-        q.hit[i] = hit;
-      } else if (!surfaces) {
-        q.hit[i] = hit;
-      }
-    } else if (!surfaces) {
-      q.hit[i] = hit;
-    }
-  }
-  const uint32_t s = wave_sum(cx.samples), c = wave_sum(cx.cells);
-  const uint32_t un = wave_sum(cx.unodes), ut = wave_sum(cx.utets);
-  if (lane_id() == 0) {
-    stat_add(stats, STAT_SAMPLES, s);
-    stat_add(stats, STAT_CELLS, c);
-    stat_add(stats, STAT_UNODES, un);
-    stat_add(stats, STAT_UTETS, ut);
-  }
-}
-
 // one thread per brick texel: the texel of the linear field at the brick's
 // cell origin + (lx, ly, lz), clamped to the field (apron texels past the
 // last vertex repeat it; no footprint reads them)
@@ -404,7 +306,53 @@ __global__ void k_brick(const float *src, int nx, int ny, int nz, int shift, int
   dst[i] = src[(size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * z)];
 }
 
+// one thread per cell: its eight corners; *bad is raised for a value that is
+// not finite
+__global__ void k_corners(const float *src, int nx, int ny, int cx, int cy, long long ncells, float4 *dst, int *bad)
+{
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= ncells) return;
+  const int x = (int)(i % cx), y = (int)((i / cx) % cy), z = (int)(i / ((long long)cx * cy));
+  const float *p = src + (size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * z);
+  const size_t sy = nx, sz = (size_t)nx * ny;
+  const float4 a = make_float4(p[0], p[1], p[sy], p[sy + 1]);
+  const float4 b = make_float4(p[sz], p[sz + 1], p[sz + sy], p[sz + sy + 1]);
+  dst[2 * i] = a;
+  dst[2 * i + 1] = b;
+  const float m = fabsf(a.x) + fabsf(a.y) + fabsf(a.z) + fabsf(a.w) + fabsf(b.x) + fabsf(b.y) + fabsf(b.z) + fabsf(b.w);
+  if (!(m < INFINITY)) *bad = 1;
+}
+
 } // namespace
+
+int volume_corners(Volume *v)
+{
+  VolumeDev &d = v->dd;
+  hipStream_t st = v->dev->stream;
+  d.corners = nullptr;
+  const long long n = (long long)d.ncells[0] * d.ncells[1] * d.ncells[2];
+  const size_t bytes = 2 * sizeof(float4) * (size_t)n;
+  size_t free_bytes = 0, total = 0;
+  BNX_HIP(hipMemGetInfo(&free_bytes, &total));
+  if (bytes > free_bytes / 8 || n >= (1LL << 31)) return BNX_OK;
+  DevMem bad;
+  BNX_HIP(bad.ensure(sizeof(int)));
+  if (v->corners.ensure(bytes) != hipSuccess) {
+    (void)hipGetLastError();            // no room: the linear layout serves
+    return BNX_OK;
+  }
+  BNX_HIP(hipMemsetAsync(bad.ptr, 0, sizeof(int), st));
+  k_corners<<<nblk(n, 256), 256, 0, st>>>(v->scalars.as<float>(), d.dims[0], d.dims[1], d.ncells[0], d.ncells[1], n,
+                                          v->corners.as<float4>(), bad.as<int>());
+  BNX_HIP(hipGetLastError());
+  int h = 0;
+  BNX_HIP(hipMemcpyAsync(&h, bad.ptr, sizeof(int), hipMemcpyDeviceToHost, st));
+  BNX_HIP(hipStreamSynchronize(st));
+  if (h) v->corners.release();
+  else BNX_SET(d.corners, v->corners.ptr);
+  v->version++;
+  return BNX_OK;
+}
 
 int volume_brick(Volume *v, int shift)
 {
@@ -530,53 +478,105 @@ int build_tet_neighbors(Device *dev, const int4 *tets, int ntet, DevMem &nbr)
   return BNX_OK;
 }
 
-// the seed grid: per cell, the tet (depth-first query) holding its centre
-__global__ __launch_bounds__(PQ_TB) void k_umesh_seeds(VolumeDev d, int ncells, int *seeds)
+// ------------------------------------------------------------ fine grid
+// The value ranges: every cell adds the range of its vertices' scalars to the
+// grid cells that its box touches, grown by a twentieth of its extent and
+// 1e-5 of its coordinates (a test accepts points outside the cell by far
+// less, see k_cell_pack).  A cell with more than FINE_MOST grid cells adds to
+// the range that all grid cells share.  Values are means of the scalars with
+// weights above -1e-3 (a Newton inversion's last step), so the ranges take in
+// a thousandth of their width and 1e-5 of the scalars at either end.
+constexpr int FINE_MOST = 4096;
+constexpr float FINE_SLACK = 1e-5f;
+__global__ void k_fine_ranges(const int4 *tets, const int4 *ext, const uint8_t *types, const float4 *verts, int n,
+                              VolumeDev d, int *lo, int *hi, int *all)
 {
-  __shared__ uint32_t ring[PQ_SHORT * PQ_TB];
-  MarchCtx cx{ring + threadIdx.x, 0, 0, 0, 0};
-  const int c = blockIdx.x * PQ_TB + threadIdx.x;
-  if (c >= ncells) return;
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= n) return;
+  float4 l, h;
+  cell_box(tets, ext, types, verts, c, l, h);
+  const float size = fmx(fmx(h.x - l.x, h.y - l.y), h.z - l.z);
+  const float far = fmx(fmx(fmx(fabsf(l.x), fabsf(h.x)), fmx(fabsf(l.y), fabsf(h.y))), fmx(fabsf(l.z), fabsf(h.z)));
+  const float m = .05f * size + 1e-5f * far, slack = 1e-3f * (h.w - l.w) + FINE_SLACK * fmx(fabsf(l.w), fabsf(h.w));
+  const int a = seed_cell(d, v3{l.x - m, l.y - m, l.z - m}), b = seed_cell(d, v3{h.x + m, h.y + m, h.z + m});
   const int nx = d.seed_dims[0], ny = d.seed_dims[1];
-  const int ix = c % nx, iy = (c / nx) % ny, iz = c / (nx * ny);
-  const v3 P = v3{d.seed_origin[0] + ((float)ix + .5f) / d.seed_rcp[0],
-                  d.seed_origin[1] + ((float)iy + .5f) / d.seed_rcp[1],
-                  d.seed_origin[2] + ((float)iz + .5f) / d.seed_rcp[2]};
-  float f;
-  seeds[c] = umesh_dfs(d, P, cx, f);
+  const int ax = a % nx, ay = (a / nx) % ny, az = a / (nx * ny), bx = b % nx, by = (b / nx) % ny, bz = b / (nx * ny);
+  const int vl = f2o(l.w - slack), vh = f2o(h.w + slack);
+  const bool finite = slack < INFINITY;       // an infinite scalar: any value may come of it
+  if (!finite || (long long)(bx - ax + 1) * (by - ay + 1) * (bz - az + 1) > FINE_MOST) {
+    atomicMin(all, finite ? vl : f2o(-INFINITY));
+    atomicMax(all + 1, finite ? vh : f2o(INFINITY));
+    return;
+  }
+  for (int z = az; z <= bz; z++)
+    for (int y = ay; y <= by; y++)
+      for (int x = ax; x <= bx; x++) {
+        const int i = (z * ny + y) * nx + x;
+        atomicMin(lo + i, vl);
+        atomicMax(hi + i, vh);
+      }
 }
 
-// seed grid of about one cell per four tets over the bounds (at most 256 a
-// side); an empty axis gets one cell
-int build_seed_grid(Volume *v, int ntet)
+// per grid cell the tet (depth-first query) holding its centre, and its range
+constexpr int SEED_TB = 256;
+__global__ __launch_bounds__(SEED_TB) void k_fine_pack(VolumeDev d, int ncells, const int *lo, const int *hi,
+                                                       const int *all, float4 *fine)
+{
+  __shared__ uint32_t ring[PQ_SHORT * SEED_TB];
+  QueryCtx cx{ring + threadIdx.x, 0, 0};
+  const int c = blockIdx.x * SEED_TB + threadIdx.x;
+  if (c >= ncells) return;
+  int seed = -1;
+  if (d.field == FIELD_KIND_TETS) {
+    const int nx = d.seed_dims[0], ny = d.seed_dims[1];
+    const int ix = c % nx, iy = (c / nx) % ny, iz = c / (nx * ny);
+    const v3 P = v3{d.seed_origin[0] + ((float)ix + .5f) / d.seed_rcp[0],
+                    d.seed_origin[1] + ((float)iy + .5f) / d.seed_rcp[1],
+                    d.seed_origin[2] + ((float)iz + .5f) / d.seed_rcp[2]};
+    float f;
+    seed = umesh_dfs<SEED_TB>(d, P, cx, f);
+  }
+  fine[c] = make_float4(__int_as_float(seed), o2f(min(lo[c], all[0])), o2f(max(hi[c], all[1])), 0.f);
+}
+
+// fine grid of about one cell per two tets, or eight per other cell, over the
+// bounds (at most 256 a side); ext, types null: tets
+int build_fine_grid(Volume *v, const int4 *tets, const int4 *ext, const uint8_t *types, const float4 *verts, int n)
 {
   VolumeDev &d = v->dd;
-  double ext[3], vol = 1.0;
-  int flat = 0;
+  hipStream_t st = v->dev->stream;
+  double size[3], vol = 1.0;
+  bool flat = false;
+  d.ufine = nullptr;
   for (int k = 0; k < 3; k++) {
-    ext[k] = (double)d.hi[k] - (double)d.lo[k];
-    if (ext[k] > 0.0) vol *= ext[k];
-    else flat++;
+    size[k] = (double)d.hi[k] - (double)d.lo[k];
+    if (size[k] > 0.0) vol *= size[k];
+    else flat = true;
   }
-  const double h = std::cbrt(vol / std::max(1.0, ntet / 4.0));
+  if (flat) return BNX_OK;      // a flat mesh holds no cell with volume
+  const double h = std::cbrt(vol / std::max(1.0, d.field == FIELD_KIND_TETS ? n / 2.0 : 8.0 * n));
   long long ncells = 1;
   for (int k = 0; k < 3; k++) {
-    int n = 1;
-    if (ext[k] > 0.0 && flat == 0) n = (int)std::min(256.0, std::max(1.0, std::ceil(ext[k] / h)));
-    d.seed_dims[k] = n;
+    d.seed_dims[k] = (int)std::min(256.0, std::max(1.0, std::ceil(size[k] / h)));
     d.seed_origin[k] = d.lo[k];
-    d.seed_rcp[k] = ext[k] > 0.0 ? (float)n / (float)ext[k] : 0.f;
-    ncells *= n;
+    d.seed_rcp[k] = (float)d.seed_dims[k] / (float)size[k];
+    ncells *= d.seed_dims[k];
   }
-  if (flat > 0) {
-    // a flat mesh holds no tet with volume: no seeds
-    d.useed = nullptr;
-    return BNX_OK;
-  }
-  BNX_HIP(v->useed.ensure(sizeof(int) * (size_t)ncells));
-  k_umesh_seeds<<<nblk(ncells, PQ_TB), PQ_TB, 0, v->dev->stream>>>(d, (int)ncells, v->useed.as<int>());
+  DevMem lo, hi;
+  BNX_HIP(v->ufine.ensure(sizeof(float4) * (size_t)ncells));
+  BNX_HIP(lo.ensure(sizeof(int) * (size_t)ncells));
+  BNX_HIP(hi.ensure(sizeof(int) * (size_t)ncells));
+  k_fill_ranges<<<nblk(ncells, 256), 256, 0, st>>>(lo.as<int>(), hi.as<int>(), (int)ncells);
+  DevMem all;
+  BNX_HIP(all.ensure(2 * sizeof(int)));
+  k_fill_ranges<<<1, 64, 0, st>>>(all.as<int>(), all.as<int>() + 1, 1);
+  k_fine_ranges<<<nblk(n, 256), 256, 0, st>>>(tets, ext, types, verts, n, d, lo.as<int>(), hi.as<int>(),
+                                              all.as<int>());
+  k_fine_pack<<<nblk(ncells, SEED_TB), SEED_TB, 0, st>>>(d, (int)ncells, lo.as<int>(), hi.as<int>(), all.as<int>(),
+                                                         v->ufine.as<float4>());
   BNX_HIP(hipGetLastError());
-  BNX_SET(d.useed, v->useed.ptr);
+  BNX_HIP(hipStreamSynchronize(st));
+  BNX_SET(d.ufine, v->ufine.ptr);
   return BNX_OK;
 }
 
@@ -587,10 +587,10 @@ int volume_build_umesh(Volume *v, const int4 *tets4, const int4 *ext4, const uin
   VolumeDev &d = v->dd;
   hipStream_t st = dev->stream;
   const bool mixed = types != nullptr;
-  BNX_HIP(v->uverts.ensure(sizeof(float4) * (size_t)nvert));
-  BNX_HIP(hipMemcpyAsync(v->uverts.ptr, verts4, sizeof(float4) * (size_t)nvert, hipMemcpyHostToDevice, st));
-  DevMem tets, ext, typ, rlo, rhi;
+  DevMem verts, tets, ext, typ, rlo, rhi;
   DevMem &lo = dev->build.box_lo, &hi = dev->build.box_hi;
+  BNX_HIP(verts.ensure(sizeof(float4) * (size_t)nvert));
+  BNX_HIP(hipMemcpyAsync(verts.ptr, verts4, sizeof(float4) * (size_t)nvert, hipMemcpyHostToDevice, st));
   BNX_HIP(tets.ensure(sizeof(int4) * (size_t)ntet));
   BNX_HIP(hipMemcpyAsync(tets.ptr, tets4, sizeof(int4) * (size_t)ntet, hipMemcpyHostToDevice, st));
   if (mixed) {
@@ -604,7 +604,7 @@ int volume_build_umesh(Volume *v, const int4 *tets4, const int4 *ext4, const uin
   // element BVH over the cells' boxes; cells stored in its slot order
   BNX_HIP(lo.ensure(sizeof(float4) * (size_t)ntet));
   BNX_HIP(hi.ensure(sizeof(float4) * (size_t)ntet));
-  k_cell_boxes<<<nblk(ntet, 256), 256, 0, st>>>(tets.as<int4>(), ext_d, typ_d, v->uverts.as<float4>(), ntet,
+  k_cell_boxes<<<nblk(ntet, 256), 256, 0, st>>>(tets.as<int4>(), ext_d, typ_d, verts.as<float4>(), ntet,
                                                 lo.as<float4>(), hi.as<float4>());
   BNX_HIP(hipGetLastError());
   int rc = build_bvh(dev, lo.as<float4>(), hi.as<float4>(), ntet, 4, v->ebvh);
@@ -613,54 +613,40 @@ int volume_build_umesh(Volume *v, const int4 *tets4, const int4 *ext4, const uin
     set_error("bnx_volume_create_umesh: element BVH deeper than the point-query stack");
     return BNX_ERR_UNSUPPORTED;
   }
-  BNX_HIP(v->utets.ensure(sizeof(int4) * (size_t)ntet));
-  if (mixed) {
-    BNX_HIP(v->uext.ensure(sizeof(int4) * (size_t)ntet));
-    BNX_HIP(v->utypes.ensure((size_t)ntet));
-  } else {
-    v->uext.release();
-    v->utypes.release();
-  }
-  k_cell_sort<<<nblk(ntet, 256), 256, 0, st>>>(tets.as<int4>(), ext_d, typ_d, v->ebvh.order.as<int>(), ntet,
-                                               v->utets.as<int4>(), v->uext.as<int4>(), v->utypes.as<uint8_t>());
-  BNX_HIP(hipGetLastError());
-  BNX_SET(d.uverts, v->uverts.ptr);
-  BNX_SET(d.utets, v->utets.ptr);
   BNX_SET(d.ebvh, v->ebvh.nodes.ptr);
-  d.useed = nullptr;
-  d.uext = nullptr;
-  d.utypes = nullptr;
+  d.field = mixed ? FIELD_KIND_CELLS : FIELD_KIND_TETS;
   if (mixed) {
     // other cells than tets: point queries go depth first through the
-    // element BVH (no tet walk, no seeds)
-    BNX_SET(d.uext, v->uext.ptr);
-    BNX_SET(d.utypes, v->utypes.ptr);
-    v->useed.release();
-    // no neighbours: a walk (only in a tets-only kernel, which such a field
-    // never meets) ends at its first cell
-    BNX_HIP(v->unbr.ensure(sizeof(int4) * (size_t)ntet));
-    BNX_HIP(hipMemsetAsync(v->unbr.ptr, 0xff, sizeof(int4) * (size_t)ntet, st));
+    // element BVH (no tet walk)
+    BNX_HIP(v->ucells.ensure(sizeof(float4) * 8 * (size_t)ntet));
+    BNX_HIP(v->ucellbox.ensure(sizeof(float4) * 2 * (size_t)ntet));
+    k_cell_pack<<<nblk(ntet, 256), 256, 0, st>>>(tets.as<int4>(), ext_d, typ_d, verts.as<float4>(),
+                                                 v->ebvh.order.as<int>(), ntet, v->ucells.as<float4>(),
+                                                 v->ucellbox.as<float4>());
+    BNX_HIP(hipGetLastError());
+    if ((rc = collapse_bvh4(dev, v->ebvh)) != BNX_OK) return rc;
+    BNX_CHECK(v->ebvh.stack_need4 <= PQ_SHORT + PQ_DEEP4, BNX_ERR_UNSUPPORTED,
+              "bnx_volume_create_umesh: element BVH deeper than the point-query stack");
+    BNX_SET(d.ebvh4, v->ebvh.nodes4.ptr);
+    BNX_SET(d.ucells, v->ucells.ptr);
+    BNX_SET(d.ucellbox, v->ucellbox.ptr);
   } else {
-    // face neighbours of the tets, in slot order, for the walking point query
-    if ((rc = build_tet_neighbors(dev, v->utets.as<int4>(), ntet, v->unbr)) != BNX_OK) return rc;
+    // the tet records: planes and face neighbours (for the walking point
+    // query) in one 128-byte record per slot
+    DevMem sorted, nbr;
+    BNX_HIP(sorted.ensure(sizeof(int4) * (size_t)ntet));
+    k_tet_sort<<<nblk(ntet, 256), 256, 0, st>>>(tets.as<int4>(), v->ebvh.order.as<int>(), ntet, sorted.as<int4>());
+    BNX_HIP(hipGetLastError());
+    if ((rc = build_tet_neighbors(dev, sorted.as<int4>(), ntet, nbr)) != BNX_OK) return rc;
+    BNX_HIP(v->utetv.ensure(sizeof(float4) * TET_REC * (size_t)ntet));
+    k_tet_pack<<<nblk(ntet, 256), 256, 0, st>>>(sorted.as<int4>(), verts.as<float4>(), nbr.as<int4>(), ntet,
+                                                v3{d.lo[0], d.lo[1], d.lo[2]}, v3{d.hi[0], d.hi[1], d.hi[2]},
+                                                v->utetv.as<float4>());
+    BNX_HIP(hipGetLastError());
+    BNX_SET(d.utetv, v->utetv.ptr);
+    BNX_HIP(hipStreamSynchronize(st));
   }
-  // the tet records: vertices and neighbours in one 80-byte record per slot
-  BNX_HIP(v->utetv.ensure(sizeof(float4) * 5 * (size_t)ntet));
-  k_tet_pack<<<nblk(ntet, 256), 256, 0, st>>>(v->utets.as<int4>(), v->uverts.as<float4>(), v->unbr.as<int4>(), ntet,
-                                              v->utetv.as<float4>());
-  BNX_HIP(hipGetLastError());
-  BNX_SET(d.utetv, v->utetv.ptr);
-  BNX_HIP(hipStreamSynchronize(st));
-  // the records hold the neighbours; the index array stays only for the
-  // other cells' vertex lists
-  v->unbr.release();
-  if (!mixed) {
-    v->utets.release();
-    d.utets = nullptr;
-    // seeds for point queries (built with the element BVH in place, before
-    // the seed pointer is set, so the build's own queries are depth first)
-    if ((rc = build_seed_grid(v, ntet)) != BNX_OK) return rc;
-  }
+  if ((rc = build_fine_grid(v, tets.as<int4>(), ext_d, typ_d, verts.as<float4>(), ntet)) != BNX_OK) return rc;
   // macrocell value ranges
   const int nmc = d.mc[0] * d.mc[1] * d.mc[2];
   BNX_HIP(rlo.ensure(sizeof(int) * (size_t)nmc));
@@ -670,7 +656,7 @@ int volume_build_umesh(Volume *v, const int4 *tets4, const int4 *ext4, const uin
   BNX_SET(d.ranges, v->ranges.ptr);
   BNX_SET(d.majorants, v->majorants.ptr);
   k_fill_ranges<<<nblk(nmc, 256), 256, 0, st>>>(rlo.as<int>(), rhi.as<int>(), nmc);
-  k_umesh_raster<<<nblk(ntet, 128), 128, 0, st>>>(tets.as<int4>(), ext_d, typ_d, v->uverts.as<float4>(), ntet, d,
+  k_umesh_raster<<<nblk(ntet, 128), 128, 0, st>>>(tets.as<int4>(), ext_d, typ_d, verts.as<float4>(), ntet, d,
                                                   rlo.as<int>(), rhi.as<int>());
   k_finish_ranges<<<nblk(nmc, 256), 256, 0, st>>>(rlo.as<int>(), rhi.as<int>(), nmc, v->ranges.as<float2>());
   k_majorants<<<nblk(nmc, 256), 256, 0, st>>>(d, v->ranges.as<float2>(), v->majorants.as<float>());
@@ -686,19 +672,6 @@ int volume_rebuild_majorants(Volume *v)
   k_majorants<<<nblk((long)nmc, 256), 256, 0, dev->stream>>>(v->dd, v->ranges.as<float2>(),
                                                              v->majorants.as<float>());
   BNX_HIP(hipStreamSynchronize(dev->stream));
-  BNX_HIP(hipGetLastError());
-  return BNX_OK;
-}
-
-int launch_volume_march(Device *dev, const SlotDev *slots, const SegView &sv, int blocks256, const RayQueue &q,
-                        bool surfaces, int full, unsigned long long *stats)
-{
-  if (blocks256 > 0 && (full & MARCH_CELLS))
-    k_volume_march<MARCH_FULL | MARCH_CELLS><<<blocks256, 256, 0, dev->stream>>>(slots, sv, q, surfaces ? 1 : 0, stats);
-  else if (blocks256 > 0 && full)
-    k_volume_march<MARCH_FULL><<<blocks256, 256, 0, dev->stream>>>(slots, sv, q, surfaces ? 1 : 0, stats);
-  else if (blocks256 > 0)
-    k_volume_march<0><<<blocks256, 256, 0, dev->stream>>>(slots, sv, q, surfaces ? 1 : 0, stats);
   BNX_HIP(hipGetLastError());
   return BNX_OK;
 }

@@ -1,0 +1,91 @@
+"""The march kernels where they can go wrong, on the GPU against the CPU
+oracle: frames whose rays do not fill a wave, a 256-ray block or its chunks;
+more volumes in a world than a launch has claim counters; scalars that are
+not finite (no corner copy, open value ranges); isosurfaces whose samples'
+sides come from a fine grid of a single cell up to one a few cells wide, at
+values inside, at the ends and outside of the field's range.  IDs, ray and
+sample counts exact; depth within 1e-5 relative and pixels within 1e-3, the
+bounds of the volume tests next to this one."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import barney_amd as bx
+from barney_amd import abi, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _compare(dev, orc, sc, world, scene, spp, flags=0):
+    rend = abi.renderer(bg=sc.bg_color, ambient=sc.ambient, flags=flags)
+    c = sc.camera
+    fr = bx.Frame(dev, sc.width, sc.height)
+    st = bx.render(world, bx.camera_perspective(c["position"], c["direction"], c["up"], c["fovy"]), rend, fr, spp)
+    of = orc.Frame(sc.width, sc.height)
+    _, ost = orc.render(scene, orc.camera_perspective(c["position"], c["direction"], c["up"], c["fovy"]), rend, of,
+                        spp)
+    for ch in (abi.BNX_FB_PRIMID, abi.BNX_FB_INSTID, abi.BNX_FB_OBJID):
+        g, r = fr.read(ch), of.read(ch)
+        assert np.array_equal(g, r), (ch, int((g != r).sum()))
+    assert np.allclose(fr.read(abi.BNX_FB_DEPTH), of.read(abi.BNX_FB_DEPTH), rtol=1e-5, atol=0)
+    assert np.abs(fr.read(abi.BNX_FB_COLOR) - of.read(abi.BNX_FB_COLOR)).max() <= 1e-3
+    assert st["rays"] == ost["rays"]
+    assert st["volume_samples"] == ost["volume_samples"]
+    fr.close()
+
+
+@pytest.mark.parametrize("w,h,flags", [(1, 1, 0), (17, 3, 0), (16, 16, abi.BNX_RENDER_RATIO_TRACKING), (129, 67, 0),
+                                       (333, 33, abi.BNX_RENDER_RATIO_TRACKING)])
+def test_ray_counts(dev, orc, w, h, flags):
+    print(f"march {w}x{h} flags={flags}", flush=True)
+    vs = scenes.config2(n=33, mc_grid=8, width=w, height=h)
+    _compare(dev, orc, vs, bx.VolumeWorld(dev, vs).world, orc.volume_scene(vs), 1, flags)
+
+
+@pytest.mark.parametrize("n,flags", [(2, 0), (11, 0), (11, abi.BNX_RENDER_RATIO_TRACKING)])
+def test_many_volumes(dev, orc, n, flags):
+    print(f"march of {n} volumes flags={flags}", flush=True)
+    vs = scenes.config2(n=17, mc_grid=4, width=40, height=30)
+    thin = [dataclasses.replace(vs, grid_origin=(.07 * k, -.05 * k, .03 * k), base_density=vs.base_density / 4)
+            for k in range(n)]
+    world = bx.World(dev, bx.Group.instances(dev, [], []).build(), vs.dir_lights)
+    scene = orc.Scene()
+    vols = [bx.Volume(dev, t, user_id=k) for k, t in enumerate(thin)]
+    for k, t in enumerate(thin):
+        world.add_volume(vols[k], k)
+        scene.add_volume(t, user_id=k, user_inst=k)
+    scene.set_dir_lights(vs.dir_lights)
+    scene.build()
+    _compare(dev, orc, vs, world, scene, 2, flags)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_scalars_not_finite(dev, orc, bad):
+    print(f"march scalar {bad}", flush=True)
+    vs = scenes.config2(n=20, mc_grid=4, width=48, height=48)
+    f = vs.scalars.copy()
+    f[9:11, 7, 12] = bad
+    vs = dataclasses.replace(vs, scalars=f)
+    _compare(dev, orc, vs, bx.VolumeWorld(dev, vs).world, orc.volume_scene(vs), 1)
+
+
+@pytest.mark.parametrize("n,iso", [(1, .2), (2, .3), (3, .05), (5, 1.), (5, 0.), (5, -3.), (9, .3)])
+@pytest.mark.parametrize("kind", ["tets", "mixed"])
+def test_isosurface_sides(dev, orc, kind, n, iso):
+    print(f"iso march {kind} n={n} iso={iso}", flush=True)
+    make = scenes.config4 if kind == "tets" else scenes.mixed_volume
+    us = make(n=n, width=60, height=52, volume=n % 2 == 1)
+    lo, hi = float(us.scalars.min()), float(us.scalars.max())
+    us = dataclasses.replace(us, iso_value=lo + iso * (hi - lo))      # 0 and 1: the ends of the range
+    _compare(dev, orc, us, bx.UMeshWorld(dev, us).world, orc.umesh_scene(us), 1)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+def test_isosurface_of_scalars_not_finite(dev, orc, bad):
+    print(f"iso march scalar {bad}", flush=True)
+    us = scenes.config4(n=6, width=60, height=52)
+    f = us.scalars.copy()
+    f[len(f) // 2] = bad
+    us = dataclasses.replace(us, scalars=f)
+    _compare(dev, orc, us, bx.UMeshWorld(dev, us).world, orc.umesh_scene(us), 1)
