@@ -224,6 +224,27 @@ bool can_be_translucent(const Geom &gm, const Group *g)
   return below;
 }
 
+__global__ void k_enter(const int *order, const InstDev *insts, const BlasDev *blas, int n, EnterDev *enter)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int inst = order[i];
+  const InstDev &I = insts[inst];
+  const BlasDev &b = blas[I.blas];
+  EnterDev e;
+  for (int k = 0; k < 3; k++) e.w2o[k] = I.w2o[k];
+  e.nodes = b.nodes;
+  e.prims = b.prims;
+  e.refs = b.refs;
+  e.inst = inst;
+  e.geom_base = I.geom_base;
+  e.type = b.type;
+  e.identity = I.identity;
+  e.translucent = b.translucent;
+  e._pad = 0;
+  enter[i] = e;
+}
+
 int build_tlas(Group *g)
 {
   Device *dev = g->dev;
@@ -358,6 +379,11 @@ int build_tlas(Group *g)
   if ((rc = upload(dev, g->d_insts, insts.data(), insts.size())) != BNX_OK) return rc;
   if ((rc = upload(dev, g->d_blas, blas.data(), blas.size())) != BNX_OK) return rc;
   if ((rc = upload(dev, g->d_geoms, geoms.data(), geoms.size())) != BNX_OK) return rc;
+  BNX_HIP(g->d_enter.ensure(sizeof(EnterDev) * (size_t)std::max(1, n)));
+  if (n > 0)
+    k_enter<<<(n + 255) / 256, 256, 0, dev->stream>>>(g->bvh.order.as<int>(), g->d_insts.as<InstDev>(),
+                                                      g->d_blas.as<BlasDev>(), n, g->d_enter.as<EnterDev>());
+  BNX_HIP(hipGetLastError());
   BNX_HIP(hipStreamSynchronize(dev->stream));
   // a walk pushes at most the TLAS path's entries, the LEAVE marker and a BLAS path's entries
   if (g->bvh.stack_need4 + 1 + g->max_blas_depth + 1 > trace_stack_capacity()) {
@@ -365,7 +391,7 @@ int build_tlas(Group *g)
     return BNX_ERR_UNSUPPORTED;
   }
   BNX_SET(g->scene.tlas_nodes, g->bvh.nodes4.as<Node4>());
-  BNX_SET(g->scene.tlas_order, g->bvh.order.as<int>());
+  BNX_SET(g->scene.enter, g->d_enter.as<EnterDev>());
   BNX_SET(g->scene.insts, g->d_insts.as<InstDev>());
   BNX_SET(g->scene.blas, g->d_blas.as<BlasDev>());
   BNX_SET(g->scene.geoms, g->d_geoms.as<GeomDev>());
@@ -479,6 +505,10 @@ int bnx_device_create(int gpu_id, bnx_device *out)
   if (const char *e = getenv("BNX_TRACE_REFILL_PRIMS")) d->trace_refill_prims = std::max(0LL, atoll(e));
   if (const char *e = getenv("BNX_TRACE_BLOCKS_PER_CU")) d->trace_blocks_per_cu = std::min(1 << 20, std::max(1, atoi(e)));
   int rc = noalloc_init(d);
+  if (rc == BNX_OK && d->api_claims.ensure(sizeof(int) * CLAIM_GROUPS * CLAIM_STRIDE) != hipSuccess) {
+    set_error("bnx_device_create: out of device memory");
+    rc = BNX_ERR_OOM;
+  }
   if (rc != BNX_OK) {
     (void)hipStreamDestroy(d->stream);
     delete d;

@@ -243,9 +243,25 @@ struct GeomDev {
   AttrDev attr[ATTR_SLOTS];
 };
 
+// what a walk needs of an instance, in the order of the TLAS leaves: one
+// fetch, where the order, the instance and its BLAS were one after the other
+struct EnterDev {
+  float4 w2o[3];
+  const Node4 BNX_G *nodes;
+  const float4 BNX_G *prims;
+  const int2 BNX_G *refs;
+  int inst;
+  int geom_base;
+  int type;                // BLAS_*
+  int identity;
+  int translucent;
+  int _pad;
+};
+static_assert(sizeof(EnterDev) == 96, "whole 16-byte words");
+
 struct SceneDev {
   const Node4 BNX_G *tlas_nodes;
-  const int BNX_G *tlas_order;
+  const EnterDev BNX_G *enter;
   const InstDev BNX_G *insts;
   const BlasDev BNX_G *blas;
   const GeomDev BNX_G *geoms;

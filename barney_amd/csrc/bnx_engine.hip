@@ -96,7 +96,7 @@ struct BatchGraph {
 // queues, tables and staging of one wavefront
 struct Wavefront {
   Queues Q;
-  DevMem slots, chunks, segs, blk256, blk1024, blkT, pool, claims, out_base, out_cnt;
+  DevMem slots, chunks, segs, blk256, blk1024, claims, out_base, out_cnt;
   Pinned h_slots, h_chunks, h_segs, h_out_base, h_out_cnt;
   int slot_cap = 0, chunk_cap = 0, seg_cap = 0;
   // device-driven bounce loops: per-generation counts, timing events (four
@@ -131,7 +131,7 @@ struct Wavefront {
     std::vector<const void *> b = {Q.org[0].ptr, Q.org[1].ptr, Q.dir[0].ptr, Q.dir[1].ptr, Q.rng[0].ptr,
                                    Q.rng[1].ptr, Q.ps[0].ptr, Q.ps[1].ptr, Q.hit[0].ptr, Q.hit[1].ptr,
                                    Q.hit_v[0].ptr, Q.hit_v[1].ptr, Q.vcol[0].ptr, Q.vcol[1].ptr, Q.stats.ptr,
-                                   slots.ptr, segs.ptr, blk256.ptr, blk1024.ptr, blkT.ptr, pool.ptr, claims.ptr,
+                                   slots.ptr, segs.ptr, blk256.ptr, blk1024.ptr, claims.ptr,
                                    out_base.ptr, out_cnt.ptr, gen_counts.ptr, stamps.ptr};
     if (b != graph_bufs) {
       drop_graphs();
@@ -176,8 +176,7 @@ struct Wavefront {
     if (nsegs > seg_cap) {
       BNX_HIP(segs.ensure(sizeof(Segment) * nsegs));
       BNX_HIP(h_segs.ensure(sizeof(Segment) * nsegs));
-      BNX_HIP(pool.ensure(sizeof(int) * nsegs));
-      BNX_HIP(claims.ensure(march_claims_bytes()));
+      BNX_HIP(claims.ensure(sizeof(int) * CLAIMS_LAUNCHES * CLAIM_GROUPS * CLAIM_STRIDE));
       seg_cap = nsegs;
     }
     // every segment adds at most one partial block
@@ -185,7 +184,6 @@ struct Wavefront {
     if (blocks > blk_cap) {
       BNX_HIP(blk256.ensure(sizeof(int) * blocks));
       BNX_HIP(blk1024.ensure(sizeof(int) * blocks));
-      BNX_HIP(blkT.ensure(sizeof(int) * blocks));
       blk_cap = blocks;
     }
     return BNX_OK;
@@ -195,30 +193,16 @@ struct Wavefront {
 // segments of one generation, written straight into pinned staging
 struct SegList {
   Segment *v;
-  int n = 0, blocks256 = 0, blocks1024 = 0, blocksT = 0;
+  int n = 0, blocks256 = 0, blocks1024 = 0;
   long long rays = 0;
-  // refill: idle lanes per wave that trigger a trace-pool refill.  Whole-
-  // wave refills (64) keep consecutive primary rays together; secondary
-  // rays are incoherent anyway, and refilling lanes as they finish keeps
-  // the waves busy
+  // refill: idle lanes that make a trace wave take new rays; 64: its own count
   void add(int slot, int begin, int count, int refill)
   {
     if (count <= 0) return;
-    v[n++] = Segment{slot, begin, count, blocks256, blocks1024, 0, refill, 0};
+    v[n++] = Segment{slot, begin, count, blocks256, blocks1024, refill, {}};
     blocks256 += (count + 255) / 256;
     blocks1024 += (count + 1023) / 1024;
     rays += count;
-  }
-  // trace blocks: each draws rays from its segment's pool; size the launch
-  // to about `target` blocks (a few per CU), at least one ray per thread
-  void layout_trace(int target)
-  {
-    const long long per = 256LL * std::max(1LL, (rays + 256LL * target - 1) / (256LL * target));
-    blocksT = 0;
-    for (int k = 0; k < n; k++) {
-      v[k].blockT = blocksT;
-      blocksT += (int)((v[k].count + per - 1) / per);
-    }
   }
 };
 
@@ -238,23 +222,18 @@ int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool sur
   unsigned long long *st = Q.stats.as<unsigned long long>();
   const SlotDev *slots = F.slots.as<SlotDev>();
   int rc;
-  sl.layout_trace(dev->trace_blocks_per_cu * dev->num_cus);
   BNX_HIP(hipMemcpyAsync(F.segs.ptr, sl.v, sizeof(Segment) * sl.n, hipMemcpyHostToDevice, dev->stream));
-  const SegView sv{F.segs.as<Segment>(), F.blk256.as<int>(), F.blk1024.as<int>(), F.blkT.as<int>(),
-                   F.pool.as<int>(), F.claims.as<int>()};
-  if ((rc = launch_segment_blocks(dev, sv, sl.n, sl.blocks256, sl.blocks1024, sl.blocksT)) != BNX_OK) return rc;
+  const SegView sv{F.segs.as<Segment>(), F.blk256.as<int>(), F.blk1024.as<int>(), F.claims.as<int>()};
+  if ((rc = launch_segment_blocks(dev, sv, sl.n, sl.blocks256, sl.blocks1024)) != BNX_OK) return rc;
   TraceQueue tq{in.org, in.dir, in.hit, in.hit_v, in.rng, in.ps};
   // with neither surfaces nor volumes the trace kernel still writes the misses
   const bool trace = surfaces || !volumes;
   const bool timed = Q.ev_begin != nullptr;
   if (timed) BNX_HIP(hipEventRecord(Q.ev_begin, dev->stream));
-  bool pooled = false, cut = false;
+  bool cut = false;
   const SlotDev *hs = F.h_slots.as<SlotDev>();
-  for (int k = 0; k < sl.n; k++) {
-    pooled = pooled || sl.v[k].refill < 64;
-    cut = cut || has_cut_plane(hs[sl.v[k].slot].rr);
-  }
-  if (trace && (rc = launch_trace_queue(dev, slots, sv, sl.blocks256, sl.blocksT, pooled, cut, tq, st)) != BNX_OK)
+  for (int k = 0; k < sl.n; k++) cut = cut || has_cut_plane(hs[sl.v[k].slot].rr);
+  if (trace && (rc = launch_trace_queue(dev, slots, sv, sl.n, sl.blocks256, cut, tq, st)) != BNX_OK)
     return rc;
   if (timed) BNX_HIP(hipEventRecord(Q.ev_end, dev->stream));
   if (volumes) {
@@ -278,34 +257,26 @@ int enqueue_dd(Device *dev, Wavefront &F, int cur0, int G, const BatchShape &b)
   Queues &Q = F.Q;
   unsigned long long *st = Q.stats.as<unsigned long long>();
   const SlotDev *slots = F.slots.as<SlotDev>();
-  const SegView sv{F.segs.as<Segment>(), F.blk256.as<int>(), F.blk1024.as<int>(), F.blkT.as<int>(),
-                   F.pool.as<int>(), F.claims.as<int>()};
+  const SegView sv{F.segs.as<Segment>(), F.blk256.as<int>(), F.blk1024.as<int>(), F.claims.as<int>()};
   const SlotOut so{F.out_base.as<int>(), F.out_cnt.as<int>()};
   const bool trace = b.surfaces || !b.volumes;
-  const long long target = (long long)dev->trace_blocks_per_cu * dev->num_cus;
   int rc;
   for (int g = 0; g < G; g++) {
     const int cur = (cur0 + g) & 1;
     // primary rays one per thread (whole-wave refills), as in the host loop
     const int refill = g == 0 ? 64 : b.refill;
-    const bool pooled = refill < 64;
     const long long c = g == 0 ? b.count0 : b.cap;
     const int blocks256 = (int)((c + 255) / 256), blocks1024 = (int)((c + 1023) / 1024);
-    int blocksT = 0;
-    if (pooled) {
-      const long long per = 256LL * std::max(1LL, (c + 256LL * target - 1) / (256LL * target));
-      blocksT = (int)((c + per - 1) / per);
-    }
     if ((rc = launch_gen_setup(dev, F.segs.as<Segment>(), F.out_cnt.as<int>(), F.gen_counts.as<long long>(), g,
                                (int)b.count0, refill)) != BNX_OK)
       return rc;
-    if ((rc = launch_segment_blocks(dev, sv, 1, blocks256, blocks1024, blocksT)) != BNX_OK) return rc;
+    if ((rc = launch_segment_blocks(dev, sv, 1, blocks256, blocks1024)) != BNX_OK) return rc;
     RayQueue in = Q.q(cur), out = Q.q(1 - cur);
     TraceQueue tq{in.org, in.dir, in.hit, in.hit_v, in.rng, in.ps};
     unsigned long long *ts = F.stamps.as<unsigned long long>() + 4 * g;
     if (trace) {
       if ((rc = launch_stamp(dev, ts)) != BNX_OK) return rc;
-      if ((rc = launch_trace_queue(dev, slots, sv, blocks256, blocksT, pooled, b.ext, tq, st)) != BNX_OK) return rc;
+      if ((rc = launch_trace_queue(dev, slots, sv, 1, blocks256, b.ext, tq, st)) != BNX_OK) return rc;
       if ((rc = launch_stamp(dev, ts + 1)) != BNX_OK) return rc;
     }
     if (b.volumes) {
@@ -636,12 +607,12 @@ constexpr long long NOALLOC_PATHS = 1LL << 16;
 constexpr size_t NOALLOC_RAYS = 2 * (size_t)NOALLOC_PATHS;
 constexpr size_t NOALLOC_BLOCKS = NOALLOC_RAYS / 256 + 2;   // one segment: one partial block at most
 constexpr size_t al256(size_t b) { return (b + 255) / 256 * 256; }
-constexpr size_t NOALLOC_CLAIMS = 16384;   // march_claims_bytes()
+constexpr size_t NOALLOC_CLAIMS = sizeof(int) * CLAIMS_LAUNCHES * CLAIM_GROUPS * CLAIM_STRIDE;
 constexpr size_t NOALLOC_QUEUE_BYTES =
     al256(16 * NOALLOC_RAYS) * 5 + al256(8 * NOALLOC_RAYS) + al256(4 * NOALLOC_RAYS);   // one queue
 constexpr size_t NOALLOC_BYTES = 2 * NOALLOC_QUEUE_BYTES + al256(8 * STAT_COUNT * STAT_SLOTS) +
                                  al256(sizeof(SlotDev)) + al256(sizeof(RaygenChunk)) + al256(sizeof(Segment)) +
-                                 4 * 256 + NOALLOC_CLAIMS + 3 * al256(4 * NOALLOC_BLOCKS);
+                                 4 * 256 + NOALLOC_CLAIMS + 2 * al256(4 * NOALLOC_BLOCKS);
 
 // The scratch memory of bnx_render_noalloc: one copy per GPU the library
 // runs on, held until the process ends.  Host code never passes this name to
@@ -678,13 +649,11 @@ void noalloc_layout(NoallocWavefront &N, unsigned char *base)
   take(F.slots, sizeof(SlotDev));
   take(F.chunks, sizeof(RaygenChunk));
   take(F.segs, sizeof(Segment));
-  take(F.pool, 4);
   take(F.claims, NOALLOC_CLAIMS);
   take(F.out_base, 4);
   take(F.out_cnt, 8);
   take(F.blk256, 4 * NOALLOC_BLOCKS);
   take(F.blk1024, 4 * NOALLOC_BLOCKS);
-  take(F.blkT, 4 * NOALLOC_BLOCKS);
   F.Q.cap = NOALLOC_RAYS;
   F.slot_cap = F.chunk_cap = F.seg_cap = 1;
   F.blk_cap = NOALLOC_BLOCKS;
@@ -737,7 +706,7 @@ struct SrvSlot {
   long long rays;              // rays of the slot that entered a generation in this step
   int region;                  // first queue index of its rays in the current input queue
   int live_rays, live_paths;   // rays there; paths they continue
-  int refill;                  // trace-pool refill of its secondary rays
+  int refill;                  // Segment::refill of its secondary rays
   int added;                   // primary rays added in the current generation
   int pad;
 };
@@ -759,7 +728,6 @@ struct SrvStep {
   long long *scal;
   long long *gen_counts;       // rays per generation
   long long max_paths;
-  int target;                  // trace blocks to aim for (pooled layout)
 };
 
 constexpr int SRV_TB = 1024;
@@ -802,8 +770,7 @@ __device__ long long srv_sum(long long v)
 //    taking min(what is left, room) paths while the paths in flight stay
 //    within max_paths; their raygen chunks follow the old regions;
 //  - segments: old regions of every active slot, then the new primaries,
-//    with their block offsets for both launch widths and the trace pool
-//    layout (about `target` blocks, as SegList::layout_trace);
+//    with their block offsets for both launch widths;
 //  - output regions in the other queue, 2 rays per path in flight, in the
 //    order of the active slots, with their counters cleared.
 // fold_only: the fold alone (after a step's last generation).
@@ -868,20 +835,17 @@ __global__ __launch_bounds__(SRV_TB) void k_srv_setup(SrvStep p, int g, int fold
     n += seg(k, slot, begin, refill);
   }
   n = srv_sum(n);
-  const long long per = 256LL * max(1LL, (n + 256LL * p.target - 1) / (256LL * p.target));
-  long long c256 = 0, c1024 = 0, cT = 0;
+  long long c256 = 0, c1024 = 0;
   for (int base = 0; base < nsegs; base += SRV_TB) {
     const int k = base + tid;
     int slot = 0, begin = 0, refill = 64, count = 0;
     if (k < nsegs) count = seg(k, slot, begin, refill);
-    long long t256, t1024, tT;
+    long long t256, t1024;
     const long long b256 = c256 + srv_scan((count + 255) / 256, t256);
     const long long b1024 = c1024 + srv_scan((count + 1023) / 1024, t1024);
-    const long long bT = cT + srv_scan((count + per - 1) / per, tT);
-    if (k < nsegs) p.segs[k] = Segment{slot, begin, count, (int)b256, (int)b1024, (int)bT, refill, 0};
+    if (k < nsegs) p.segs[k] = Segment{slot, begin, count, (int)b256, (int)b1024, refill, {}};
     c256 += t256;
     c1024 += t1024;
-    cT += tT;
   }
   // output regions
   carry = 0;
@@ -1232,7 +1196,7 @@ struct Server {
     long long *hsc = h_scal.as<long long>();
     const int A = (int)active.size(), O = (int)order.size();
     long long rays0 = 0, paths = 0, rem = 0;
-    bool surfaces = false, volumes = false, pooled = false, cut = false;
+    bool surfaces = false, volumes = false, cut = false;
     MarchKind march;
     int max_slot = 0;
     for (int i = 0; i < A; i++) {
@@ -1246,7 +1210,6 @@ struct Server {
       surfaces |= r->surfaces;
       volumes |= r->volumes;
       march.merge(r->march);
-      pooled |= refill < 64;
       cut |= has_cut_plane(r->rr);
       max_slot = std::max(max_slot, r->slot + 1);
     }
@@ -1260,12 +1223,10 @@ struct Server {
     const long long added_max = std::min(max_paths, rem);
     const long long P = std::min(max_paths, paths + rem);
     const int nsegs = A + O;
-    const int target = dev->trace_blocks_per_cu * dev->num_cus;
     const SrvStep p{d_srv.as<SrvSlot>(), d_act.as<int>(), d_ord.as<int>(), A, O, F.segs.as<Segment>(),
                     F.chunks.as<RaygenChunk>(), F.out_base.as<int>(), F.out_cnt.as<int>(),
-                    d_scal.as<long long>(), F.gen_counts.as<long long>(), max_paths, target};
-    const SegView sv{F.segs.as<Segment>(), F.blk256.as<int>(), F.blk1024.as<int>(), F.blkT.as<int>(),
-                     F.pool.as<int>(), F.claims.as<int>()};
+                    d_scal.as<long long>(), F.gen_counts.as<long long>(), max_paths};
+    const SegView sv{F.segs.as<Segment>(), F.blk256.as<int>(), F.blk1024.as<int>(), F.claims.as<int>()};
     const SlotOut so{F.out_base.as<int>(), F.out_cnt.as<int>()};
     const SlotDev *slots = F.slots.as<SlotDev>();
     unsigned long long *stat = F.Q.stats.as<unsigned long long>();
@@ -1273,19 +1234,18 @@ struct Server {
     for (int g = 0; g < G; g++) {
       const long long N = g == 0 ? rays0 + added_max : 2 * P + added_max;
       const int blocks256 = (int)((N + 255) / 256) + nsegs, blocks1024 = (int)((N + 1023) / 1024) + nsegs;
-      const int blocksT = pooled ? std::min(target + nsegs, blocks256) : 0;
       k_srv_setup<<<1, SRV_TB, 0, st>>>(p, g, 0);
       BNX_HIP(hipGetLastError());
       RayQueue in = F.Q.q(cur), out = F.Q.q(1 - cur);
       if (added_max > 0 && O > 0 &&
           (rc = launch_raygen_dev(dev, p.chunks, O, slots, p.scal + 1, added_max, in)) != BNX_OK)
         return rc;
-      if ((rc = launch_segment_blocks(dev, sv, nsegs, blocks256, blocks1024, blocksT)) != BNX_OK) return rc;
+      if ((rc = launch_segment_blocks(dev, sv, nsegs, blocks256, blocks1024)) != BNX_OK) return rc;
       TraceQueue tq{in.org, in.dir, in.hit, in.hit_v, in.rng, in.ps};
       unsigned long long *tsp = F.stamps.as<unsigned long long>() + 4 * g;
       if (trace) {
         if ((rc = launch_stamp(dev, tsp)) != BNX_OK) return rc;
-        if ((rc = launch_trace_queue(dev, slots, sv, blocks256, blocksT, pooled, cut, tq, stat)) != BNX_OK)
+        if ((rc = launch_trace_queue(dev, slots, sv, nsegs, blocks256, cut, tq, stat)) != BNX_OK)
           return rc;
         if ((rc = launch_stamp(dev, tsp + 1)) != BNX_OK) return rc;
       }

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <new>
 #include <stdexcept>
 #include <string>
@@ -101,15 +102,18 @@ struct Device {
   // launch tuning (bnx_device_set_tuning, bnx_autotune); none of it changes results
   int raygen_tile_w = 8, raygen_tile_h = 8;   // primary-ray pixel order: tiles (0: row-major)
   int trace_stack_lds = 16;  // LDS stack entries per lane in the queue-trace kernels (8, 16, 32)
-  int trace_walk = 0;        // one-ray-per-thread walk: 0 node step or leaf per trip, 1 speculative while-while
+  int trace_walk = 0;        // 0 waves that take new rays as walks end, 1 one ray per thread, speculative while-while
   int sort_rays = 0;         // bnx_render: reorder secondary generations by direction and origin
   int shade_block = 1024;    // threads per shade block (256 or 1024)
-  int trace_refill = 16;    // secondary rays of large scenes: idle lanes that trigger a trace-pool refill
+  int trace_refill = 16;    // secondary rays of large scenes: idle lanes that make a trace wave take new rays
   long long trace_refill_prims = 1 << 20;   // "large": at least this many primitives
-  int trace_blocks_per_cu = 8;   // trace launch size: blocks per CU
+  int trace_blocks_per_cu = 8;   // at most this many times four trace waves per CU
   long long render_paths = 8LL << 20;       // bnx_render: paths per batch
   long long graph_paths = 4LL << 20;        // bnx_render: batches this small run a captured bounce loop
-  int march_fit[6] = {0, 0, 0, 0, 0, 0};   // waves per CU of the march kernels (0: not asked yet)
+  int march_fit[6] = {};    // waves per CU of the march kernels (0: not asked yet)
+  int trace_fit[16] = {};   // and of the trace kernels
+  DevMem api_claims;        // claim counters of the ray-array trace, ...
+  std::mutex api_mutex;     // ... whose clearing and launch go to the stream as one
   BuildScratch build;
   DevMem counters;      // small device counters (trace work queue etc.)
   void *queues = nullptr;   // render queues (bnx_render.h Queues)
@@ -181,7 +185,7 @@ struct Group {
   std::vector<float> xfms;   // 12 floats per instance, owl affine3f layout
   DevMem inst_attr[5];       // instance attributes (attribute0..3, color): float4 per instance
   bool inst_attr_w_below_1[5] = {false, false, false, false, false};
-  DevMem d_insts, d_blas, d_geoms;
+  DevMem d_insts, d_blas, d_geoms, d_enter;
   SceneDev scene{};
   int max_blas_depth = 0;    // largest traversal-stack need of its BLASes (4-wide walk)
   long long blas_prims = 0;  // primitives in the distinct BLASes it instances
@@ -251,12 +255,11 @@ struct TraceQueue {
 int launch_trace_api(Group *g, const bnx_ray *d_rays, int n, bnx_hit *d_hits, uint32_t flags);
 struct SlotDev;
 struct SegView;
-// trace every ray of the generation's segments: one ray per thread
-// (blocks256 blocks of 256 threads) or, pooled, blocksT blocks drawing rays
-// from their segment's pool; cut: a request in the launch has a cut plane
-// (the launch then takes the kernels that apply it)
-int launch_trace_queue(Device *dev, const SlotDev *d_slots, const SegView &sv, int blocks256, int blocksT,
-                       bool pooled, bool cut, const TraceQueue &q, unsigned long long *counters);
+// trace every ray of the generation's nsegs segments (blocks256 blocks of 256
+// rays); cut: a request in the launch has a cut plane (the launch then takes
+// the kernels that apply it)
+int launch_trace_queue(Device *dev, const SlotDev *d_slots, const SegView &sv, int nsegs, int blocks256, bool cut,
+                       const TraceQueue &q, unsigned long long *counters);
 // whether a trace launch takes the extended kernels (cylinder test, cut
 // plane, stochastic opacity): a built world holds cylinders or translucent
 // triangles, or a request of the launch has a cut plane

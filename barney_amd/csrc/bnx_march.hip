@@ -25,6 +25,7 @@
 // (isosurfaces first), clipped to the closest hit so far, which the launches
 // hand on in the queue.  A block is one wave: its field's parameters are
 // wave-uniform and sit in scalar registers.
+#include "bnx_claims.h"
 #include "bnx_internal.h"
 #include "bnx_render.h"
 #include "bnx_volume.h"
@@ -241,123 +242,6 @@ BNX_D void wave_sync()
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
   __builtin_amdgcn_wave_barrier();
 }
-
-// a record at a wave-uniform address that no running kernel writes: scalar
-// loads, which the compiler may repeat where it is short of registers
-#if defined(__HIP_DEVICE_COMPILE__)
-#define BNX_CONST __attribute__((address_space(4)))
-#else
-#define BNX_CONST
-#endif
-template <typename T> BNX_D T uniform_load(const T BNX_G *p)
-{
-  static_assert(sizeof(T) % 4 == 0, "whole words");
-  const uint32_t BNX_CONST *c = (const uint32_t BNX_CONST *)p;
-  uint32_t w[sizeof(T) / 4];
-#pragma unroll
-  for (int i = 0; i < (int)(sizeof(T) / 4); i++) w[i] = c[i];
-  T r;
-  __builtin_memcpy(&r, w, sizeof(T));
-  return r;
-}
-
-// How the waves of a launch share its rays.  The generation's blocks of 256
-// rays, each inside one segment, are cut into `parts` chunks each (so that a
-// small generation still has a chunk for every wave) and dealt to CLAIM_GROUPS
-// groups of waves; a wave starts on a chunk of its own and then takes its
-// group's next one from the group's counter, or another group's once its own
-// is out.  One counter for all waves would be in the way: its atomics are
-// served one after the other beyond the XCDs' caches (14 ns each, 3.4
-// against 2.4 ms on the 256^3 volume).  Shares fixed beforehand would leave
-// the waves with the long rays behind (isosurface of 20.5M tets: 19.6
-// against 12.9 ms).
-constexpr int CLAIM_GROUPS = 16, CLAIM_STRIDE = 32;   // ints from counter to counter: a line each
-struct Claims {
-  const Segment *segs;
-  const int *blk;              // segment of each 256-ray block
-  int *ctr;                    // this launch's counters, 0 when it begins
-  int chunks, shift, per, waves;   // chunks of `per` = 256 >> shift rays
-  int chunk, group, tries;     // the chunk in hand (-1: none left)
-  int seg;                     // the segment being worked on
-  int first, total;            // its first 256-ray block, its rays
-  int base, next, stop;        // [next, stop) is in hand, segment-local, from queue index base
-  bool dry;                    // none left in this segment
-
-  BNX_D void begin(const SegView &sv, int nsegs, int program)
-  {
-    segs = sv.segs;
-    blk = sv.blk256;
-    ctr = sv.claims + program * CLAIM_GROUPS * CLAIM_STRIDE;
-    const Segment z = uniform_load((const Segment BNX_G *)(segs + nsegs - 1));
-    const int blocks = z.block256 + (z.count + 255) / 256;
-    waves = (int)gridDim.x;
-    shift = 0;
-    while (shift < 4 && (blocks << shift) < waves) shift++;
-    per = 256 >> shift;
-    chunks = blocks << shift;
-    chunk = (int)blockIdx.x < chunks ? (int)blockIdx.x : -1;
-    group = (int)blockIdx.x % CLAIM_GROUPS;
-    tries = chunks > waves ? 0 : CLAIM_GROUPS;   // every chunk is some wave's first
-  }
-  // the chunk after the one in hand
-  BNX_D void advance()
-  {
-    chunk = -1;
-    const int rounds = waves / CLAIM_GROUPS;   // the launch has whole rounds of waves
-    while (chunk < 0 && tries < CLAIM_GROUPS) {
-      int c = 0;
-      if (lane_id() == 0) c = atomicAdd(ctr + group * CLAIM_STRIDE, 1);
-      c = (rounds + __builtin_amdgcn_readfirstlane(c)) * CLAIM_GROUPS + group;
-      if (c < chunks) {
-        chunk = c;
-      } else {
-        group = (group + 1) % CLAIM_GROUPS;
-        tries++;
-      }
-    }
-  }
-  // take up the segment of the chunk in hand
-  BNX_D const Segment open()
-  {
-    seg = segment_of_chunk();
-    const Segment sg = uniform_load((const Segment BNX_G *)(segs + seg));
-    base = sg.begin;
-    first = sg.block256;
-    total = sg.count;
-    dry = false;
-    range();
-    return sg;
-  }
-  BNX_D int segment_of_chunk() { return __builtin_amdgcn_readfirstlane(blk[chunk >> shift]); }
-  BNX_D void range()
-  {
-    const int b = chunk >> shift;
-    next = (b - first) * 256 + (chunk - (b << shift)) * per;
-    stop = min(next + per, total);
-  }
-  // once the chunk in hand is taken: the next one, if it is of this segment
-  BNX_D void refill()
-  {
-    while (next >= stop && !dry) {
-      advance();
-      if (chunk < 0 || segment_of_chunk() != seg) {
-        dry = true;
-      } else {
-        range();
-      }
-    }
-  }
-  // the rays for the next `want` lanes in line: this lane's (place: its place
-  // in the line), and whether there is one
-  BNX_D int claim(int want, int place, bool &on)
-  {
-    on = next + place < stop;
-    const int i = base + next + (on ? place : 0);
-    next += want;
-    refill();
-    return i;
-  }
-};
 
 // the segments of this launch's program, one after the other: fn(slot,
 // fresh) works through the claims of one.  No trace has run when fresh_launch
@@ -1046,7 +930,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves(
   __shared__ uint32_t ready[READY * 64];
   __shared__ uint32_t ring[FIELD == FIELD_KIND_CELLS ? PQ_SHORT * 64 : 1];
   Claims cl;
-  cl.begin(sv, nsegs, program);
+  cl.begin(sv, nsegs, program, (int)gridDim.x);
   each_segment(cl, slots, q, k, fresh != 0, false, [&](const SlotDev &SL, bool f) -> bool {
     return March<FIELD>::run(cl, SL, q, k, f, stats, ready, ring);
   });
@@ -1060,15 +944,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(iso_waves(FI
   __shared__ IsoShared L;
   __shared__ uint32_t ring[FIELD == FIELD_KIND_CELLS ? PQ_SHORT * 64 : 1];
   Claims cl;
-  cl.begin(sv, nsegs, program);
+  cl.begin(sv, nsegs, program, (int)gridDim.x);
   each_segment(cl, slots, q, k, fresh != 0, true, [&](const SlotDev &SL, bool f) -> bool {
     return IsoMarch<FIELD>::run(cl, SL, q, k, f, stats, L, ring);
   });
-}
-
-__global__ void k_claims_clear(int *ctr)
-{
-  ctr[threadIdx.x * CLAIM_STRIDE] = 0;
 }
 
 using MarchKernel = void (*)(const SlotDev *, SegView, RayQueue, int, int, int, int, unsigned long long *);
@@ -1077,8 +956,6 @@ const MarchKernel KERNELS[2][FIELD_KINDS] = {
     {k_iso_march<FIELD_KIND_STRUCTURED>, k_iso_march<FIELD_KIND_TETS>, k_iso_march<FIELD_KIND_CELLS>}};
 
 } // namespace
-
-size_t march_claims_bytes() { return sizeof(int) * MARCH_PROGRAMS * CLAIM_GROUPS * CLAIM_STRIDE; }
 
 int launch_volume_march(Device *dev, const SlotDev *slots, const SegView &sv, int nsegs, int blocks256,
                         const RayQueue &q, bool surfaces, const MarchKind &kind, unsigned long long *stats)
@@ -1101,8 +978,10 @@ int launch_volume_march(Device *dev, const SlotDev *slots, const SegView &sv, in
       const int waves = std::min(fit * dev->num_cus, 16 * blocks256) / CLAIM_GROUPS * CLAIM_GROUPS;
       // the block maps' kernel clears the counters of the first launches
       const int slot = launch % MARCH_PROGRAMS;
-      if (launch >= MARCH_PROGRAMS)
-        k_claims_clear<<<1, CLAIM_GROUPS, 0, dev->stream>>>(sv.claims + slot * CLAIM_GROUPS * CLAIM_STRIDE);
+      if (launch >= MARCH_PROGRAMS) {
+        const int rc = launch_claims_clear(dev, sv.claims + slot * CLAIM_GROUPS * CLAIM_STRIDE);
+        if (rc != BNX_OK) return rc;
+      }
       kernel<<<std::max(CLAIM_GROUPS, waves), 64, 0, dev->stream>>>(slots, sv, q, k, nsegs, slot, surfaces ? 0 : 1,
                                                                     stats);
       launch++;

@@ -79,19 +79,23 @@ EnvDev env_dev(const World *w);
 // frame) with scalar loads, and the request's parameters sit in scalar
 // registers for the whole block.  Segment k covers blocks
 // [block256, block256 + ceil(count / 256)) of a 256-thread launch,
-// [block1024, ...) of a 1024-thread launch, and [blockT, ...) of the trace
-// launch, whose blocks draw the segment's rays from a shared pool.
+// and [block1024, ...) of a 1024-thread launch; trace and march waves take
+// its rays in chunks (Claims).
 struct Segment {
   int slot;
   int begin;                   // first queue index
   int count;                   // rays
   int block256;
   int block1024;
-  int blockT;
-  int refill;                  // trace pool: idle lanes per wave that trigger a refill
-  int pad;
+  int refill;                  // trace: idle lanes that make a wave take new rays (64: the kernel's own count)
+  int pad[2];
 };
 static_assert(sizeof(Segment) == 32, "segment");
+
+// counters by which the waves of a trace or march launch share its rays
+// (Claims): of each generation, the trace's and its first march launches'
+constexpr int CLAIM_GROUPS = 16, CLAIM_STRIDE = 32;   // ints from counter to counter: a line each
+constexpr int MARCH_PROGRAMS = 8, CLAIMS_TRACE = MARCH_PROGRAMS, CLAIMS_LAUNCHES = MARCH_PROGRAMS + 1;
 
 // kernel-side view of one generation's input: segments and the block ->
 // segment maps of both launch widths
@@ -99,9 +103,7 @@ struct SegView {
   const Segment *segs;
   const int *blk256;           // segment of each 256-thread block
   const int *blk1024;          // segment of each 1024-thread block
-  const int *blkT;             // segment of each trace block
-  int *pool;                   // per segment: next ray of the trace pool
-  int *claims;                 // the march launches' chunk counters, cleared with the block maps
+  int *claims;                 // the trace and march launches' chunk counters, cleared with the block maps
 };
 
 // shade output of one generation: request slot s appends to its own region
@@ -196,13 +198,11 @@ struct SortScratch {
 // shadow flag, direction octant and the origin's Morton code in [lo, hi]
 int sort_rays(Device *dev, SortScratch &S, const RayQueue &src, const RayQueue &dst, int n, const float lo[3],
               const float hi[3]);
-// fill the block -> segment maps of nsegs segments (blocks256 / blocks1024 /
-// blocksT blocks in all) and reset the segments' trace pools
-// launches of a generation's march whose counters the block maps' kernel
-// clears, and their bytes
-constexpr int MARCH_PROGRAMS = 8;
-size_t march_claims_bytes();
-int launch_segment_blocks(Device *dev, const SegView &sv, int nsegs, int blocks256, int blocks1024, int blocksT);
+// fill the block -> segment maps of nsegs segments (blocks256 / blocks1024
+// blocks in all) and clear the claim counters
+int launch_segment_blocks(Device *dev, const SegView &sv, int nsegs, int blocks256, int blocks1024);
+// the claim counters of one more launch
+int launch_claims_clear(Device *dev, int *counters);
 // shade every ray of the segments (blocks256 blocks of 256 threads or
 // blocks1024 of 1024, by the device's shade_block),
 // appending each request's shadow and continuation rays to its region of out

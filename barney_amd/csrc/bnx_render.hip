@@ -755,18 +755,12 @@ __global__ __launch_bounds__(SHADE_BLOCK) void k_shade(const SlotDev *__restrict
 }
 
 // block -> segment maps: one thread per block of either launch width
-__global__ void k_segment_blocks(SegView sv, int nsegs, int blocks256, int blocks1024, int blocksT, int claims)
+__global__ void k_segment_blocks(SegView sv, int nsegs, int blocks256, int blocks1024)
 {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (blockIdx.x == 0)
-    for (int i = threadIdx.x; i < claims; i += blockDim.x) sv.claims[i] = 0;
+    for (int i = threadIdx.x; i < CLAIMS_LAUNCHES * CLAIM_GROUPS; i += blockDim.x) sv.claims[i * CLAIM_STRIDE] = 0;
   const Segment *segs = sv.segs;
-  // the pool of segment b starts after its static part: 256 rays (one chunk
-  // per wave) for each of its trace blocks
-  if (b < nsegs) {
-    const int nb = (b + 1 < nsegs ? segs[b + 1].blockT : blocksT) - segs[b].blockT;
-    sv.pool[b] = min(segs[b].count, 256 * nb);
-  }
   if (b < blocks256) {
     int lo = 0, hi = nsegs - 1;
     while (lo < hi) {
@@ -785,15 +779,6 @@ __global__ void k_segment_blocks(SegView sv, int nsegs, int blocks256, int block
     }
     ((int *)sv.blk1024)[b] = lo;
   }
-  if (b < blocksT) {
-    int lo = 0, hi = nsegs - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (segs[mid].blockT <= b) lo = mid;
-      else hi = mid - 1;
-    }
-    ((int *)sv.blkT)[b] = lo;
-  }
 }
 
 // One generation's set-up for a device-driven bounce loop (one request,
@@ -805,7 +790,7 @@ __global__ void k_gen_setup(Segment *segs, int *out_cnt, long long *gen_counts, 
 {
   if (threadIdx.x != 0) return;
   const int count = g == 0 ? count0 : out_cnt[0];
-  segs[0] = Segment{0, 0, count, 0, 0, 0, refill, 0};
+  segs[0] = Segment{0, 0, count, 0, 0, refill, {}};
   out_cnt[0] = 0;
   out_cnt[1] = 0;
   gen_counts[g] = count;
@@ -1055,12 +1040,21 @@ int launch_stamp(Device *dev, unsigned long long *t)
   return BNX_OK;
 }
 
-int launch_segment_blocks(Device *dev, const SegView &sv, int nsegs, int blocks256, int blocks1024, int blocksT)
+int launch_segment_blocks(Device *dev, const SegView &sv, int nsegs, int blocks256, int blocks1024)
 {
-  const int n = std::max(std::max(blocks256, blocksT), nsegs);
-  if (nsegs > 0 && n > 0)
-    k_segment_blocks<<<nblk(n, 256), 256, 0, dev->stream>>>(sv, nsegs, blocks256, blocks1024, blocksT,
-                                                             (int)(march_claims_bytes() / sizeof(int)));
+  if (nsegs > 0 && blocks256 > 0)
+    k_segment_blocks<<<nblk(blocks256, 256), 256, 0, dev->stream>>>(sv, nsegs, blocks256, blocks1024);
+  BNX_HIP(hipGetLastError());
+  return BNX_OK;
+}
+
+__global__ void k_claims_clear(int *ctr)
+{
+  ctr[threadIdx.x * CLAIM_STRIDE] = 0;
+}
+int launch_claims_clear(Device *dev, int *counters)
+{
+  k_claims_clear<<<1, CLAIM_GROUPS, 0, dev->stream>>>(counters);
   BNX_HIP(hipGetLastError());
   return BNX_OK;
 }

@@ -5,13 +5,22 @@
 // kernels/traceRays.dev.cu:26-54.
 //
 // Design (wave64):
-//   * queue traversal, one ray per thread (k_trace_static), or, for the
-//     secondary rays of large scenes, from a per-segment pool (k_trace_pool):
-//     a wave claims 64 rays at a time and refills lanes as their walks end,
-//     so short walks do not idle behind the wave's longest;
+//   * as many waves as fit (five per SIMD: the walk's 96 registers without
+//     spills; seven with 19 to 39 spilled took 34.2 ms where five take 26.4,
+//     secondary rays of 37.5M primitives, 1920x1080, 8 spp) share a
+//     generation's rays out in chunks (Claims) and take new rays as walks
+//     end, so short walks do not idle behind the wave's longest;
+//   * a wave runs one kind of step a trip, the one most of its lanes are at
+//     (a node, a leaf, into or out of an instance), so that it does not pay
+//     for every kind on every trip.  Bound by VALU issue where it has rays
+//     for all waves; the 128-byte nodes and 48-byte triangles come from L2
+//     and beyond.  One ray a thread until its walk ended, either kind of step
+//     per trip: the same frame's traces 48.3 ms, a batch of 60001 rays 170 us
+//     (112 now), a million any-hit rays 580 us (303);
 //   * nearest-child-first traversal of a 4-wide BVH (collapsed from the
 //     binary build) over 128-byte nodes: the four child boxes in one fetch
-//     (seven 16-byte loads), entry distances ordered by a sorting network;
+//     (seven 16-byte loads, near and far planes told apart by their offsets, not
+//     by compares), entry distances ordered by a sorting network;
 //   * short stack: a 16-entry ring per lane in LDS laid out [entry][lane]
 //     (bank-conflict free), spilling its oldest entries to a per-lane
 //     private array when deeper;
@@ -26,8 +35,11 @@
 //     in every trace (OptixGlobals::hitOnInvisibleSide, render/
 //     OptixGlobals.h:36-45); worlds without cylinders traced without a cut
 //     plane keep the plain kernels and their register allocation.
+#include "bnx_claims.h"
 #include "bnx_internal.h"
 #include "bnx_render.h"
+
+#include <algorithm>
 
 namespace bnx {
 namespace {
@@ -37,13 +49,14 @@ constexpr int TB = 256;        // threads per block
 // 512 / waves VGPRs); the walks are latency bound, so more resident waves
 // hide more of each dependent node fetch
 #ifndef BNX_TRACE_WAVES
-#define BNX_TRACE_WAVES 7
+#define BNX_TRACE_WAVES 5
 #endif
 // traversal stack: the top SH entries per lane in an LDS ring (SH a power
 // of two: 8, 16 or 32, chosen per device; 16 by default), the rest spilled
 // to a private array, STACK_CAP entries in all whatever SH is
 constexpr int STACK_CAP = 192;
 constexpr int API_SHORT = 16;  // the ray-array entry point's ring
+constexpr int TAKE = 16;       // idle lanes that make a wave take new rays
 
 struct HitRec {
   float t, u, v;
@@ -136,9 +149,8 @@ template <bool EXT> BNX_D bool cut_rejects(const Cut &c, float t)
 // loads issue at once (the values of every accepted hit are the same
 // operations as the reference's, in the same order)
 template <bool EXT>
-BNX_D bool tri_test(const float4 *rec, v3 o, v3 d, float tmin, HitRec &best, int inst, const Cut &cut)
+BNX_D bool tri_test(float4 A, float4 B, float4 C, v3 o, v3 d, float tmin, HitRec &best, int inst, const Cut &cut)
 {
-  const float4 A = rec[0], B = rec[1], C = rec[2];
   const v3 v0 = xyz(A), e1 = xyz(B), e2 = xyz(C);
   const int prim = __float_as_int(A.w), geom = __float_as_int(B.w);
   const v3 N = cross(e1, e2);
@@ -258,6 +270,52 @@ struct Counts {
   uint32_t nodes, tris, spheres;
 };
 
+// the BLAS a ray is in
+struct Blas {
+  const Node4 BNX_G *nodes;
+  const float4 BNX_G *prims;
+  const int2 BNX_G *refs;
+  int type, inst, geom_base;
+  bool translucent;
+};
+
+// the tests of a leaf (at most 4 primitives): whether one was accepted.  The
+// records are fetched two triangles or four spheres at a time, ahead of the
+// tests.
+template <bool EXT>
+BNX_D bool leaf_test(uint32_t code, const Blas &b, v3 o, v3 d, float tmin, HitRec &best, const Cut &cut, Counts &cnt)
+{
+  const uint32_t first = (code & ~LEAF_BIT) >> 3;
+  const int count = (int)(code & 7u);
+  bool found = false;
+  if (b.type == BLAS_TRIANGLES) {
+    cnt.tris += count;
+    for (int k = 0; k < count; k += 2) {
+      const float4 BNX_G *r = b.prims + 3 * (size_t)(first + k);
+      const float4 BNX_G *s = b.prims + 3 * (size_t)(first + min(k + 1, count - 1));
+      const float4 A = r[0], B = r[1], C = r[2], D = s[0], E = s[1], F = s[2];
+      found |= tri_test<EXT>(A, B, C, o, d, tmin, best, b.inst, cut);
+      if (k + 1 < count) found |= tri_test<EXT>(D, E, F, o, d, tmin, best, b.inst, cut);
+    }
+    return found;
+  }
+  cnt.spheres += count;
+  if (!EXT || b.type == BLAS_SPHERES) {
+    float4 s[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) s[k] = b.prims[first + min(k, count - 1)];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (k < count)
+        found |= sphere_test<EXT>(s[k], (const int2 *)b.refs + first + k, o, d, tmin, best, b.inst, cut);
+  } else {
+    for (int k = 0; k < count; k++)
+      found |= pair_test(b.type, (const float4 *)b.prims + 2 * (first + k), (const int2 *)b.refs + first + k, o, d,
+                         tmin, best, b.inst, cut);
+  }
+  return found;
+}
+
 // The ray in the world frame, read again from its record (origin at rorg,
 // direction at rdir) when a walk leaves an instance, rather than held in
 // registers for the whole walk: the walks are short of registers, and a
@@ -269,14 +327,25 @@ BNX_D void world_ray(const float4 *rorg, const float4 *rdir, v3 &o, v3 &d, v3 &i
   inv = v3{1.f / d.x, 1.f / d.y, 1.f / d.z};
 }
 
-// the ray in an instance's object frame (identity instances keep the world
-// frame the walk is in)
-BNX_D void instance_ray(const InstDev &I, const float4 *rorg, const float4 *rdir, v3 &o, v3 &d, v3 &inv)
+// the ray in an instance's object frame
+BNX_D void instance_ray(const float4 w2o[3], const float4 *rorg, const float4 *rdir, v3 &o, v3 &d, v3 &inv)
 {
-  if (I.identity) return;
-  o = xfm_point_rows(I.w2o, xyz(*rorg));
-  d = fix_dir(xfm_vector_rows(I.w2o, fix_dir(xyz(*rdir))));
+  o = xfm_point_rows(w2o, xyz(*rorg));
+  d = fix_dir(xfm_vector_rows(w2o, fix_dir(xyz(*rdir))));
   inv = v3{1.f / d.x, 1.f / d.y, 1.f / d.z};
+}
+
+// into the instance of TLAS leaf entry i: its BLAS, and, if it moves the ray
+// (XF), the ray in its frame; true: moved
+template <bool XF>
+BNX_D bool enter_instance(const EnterDev BNX_G *e, const float4 *rorg, const float4 *rdir, Blas &b, v3 &o, v3 &d,
+                          v3 &inv)
+{
+  const EnterDev E = *e;
+  b = Blas{E.nodes, E.prims, E.refs, E.type, E.inst, E.geom_base, E.translucent != 0};
+  if (!XF || E.identity) return false;
+  instance_ray(E.w2o, rorg, rdir, o, d, inv);
+  return true;
 }
 
 // entry distance of child k of a 4-wide node, +inf when the ray misses it.
@@ -310,117 +379,170 @@ BNX_D void cswap(float &ta, uint32_t &ca, float &tb, uint32_t &cb)
   ca = c;
 }
 
-// lds: this lane's ring, &ring[0][lane]; the stack depth and the spill
-// array are locals so the depth stays in a register.  XF: some instance
-// transforms the ray (a non-identity instance in a launched world); without
-// it the frame never changes, so the ray (o, d, inv) is loop-invariant and
-// the compiler carries no copies of it around the walk's paths.
-template <int SH, bool EXT, bool XF>
-BNX_D HitRec traverse(const SceneDev &S, const float4 *rorg, const float4 *rdir, float tmin, float tmax, bool any_hit,
-                      uint32_t *lds, Counts &cnt, float4 cut_plane, const uint64_t *rng, HitRec &rej)
+// the near and the far plane of a node's axis lie 16 bytes apart; a ray that
+// runs down an axis has them the other way round.  `near`: byte offsets of
+// the near planes, per ray
+struct Octant {
+  uint32_t x, y, z;
+};
+BNX_D Octant octant_of(v3 d)
 {
-  Cut cut{cut_plane, rorg, rdir, rng, &S, 0, false, &rej};
-  uint32_t deep[STACK_CAP - SH];
-  int sp = 0;
-  auto push = [&](uint32_t v) {
-    const int s = sp & (SH - 1);
-    if (sp >= SH) deep[sp - SH] = lds[s * TB];
-    lds[s * TB] = v;
-    sp++;
-  };
-  auto pop = [&]() -> uint32_t {
-    sp--;
-    const int s = sp & (SH - 1);
-    const uint32_t v = lds[s * TB];
-    if (sp >= SH) lds[s * TB] = deep[sp - SH];
-    return v;
-  };
-  HitRec best{tmax, 0.f, 0.f, -1, -1, -1};
-  v3 o, d, inv;
-  world_ray(rorg, rdir, o, d, inv);
-  const Node4 *nodes = S.tlas_nodes;
-  BlasDev blas{};
-  bool in_blas = false;
-  int inst = -1;
-  uint32_t cur = 0;
-  uint32_t nvis = 0;
-  // every node is entered at most once per ray, so a ray can take no more
-  // loop trips than the scene has nodes and leaves; the cap only bounds the
-  // loop if the structure were corrupted
-  for (uint32_t trip = 0; trip < (1u << 28); trip++) {
-    if (cur < EMPTY4) {
-      // ------------------------------------------------ 4-wide inner node
-      nvis++;
-      const float4 *np = (const float4 *)(nodes + cur);
-      const float4 lx = np[0], hx = np[1], ly = np[2], hy = np[3], lz = np[4], hz = np[5];
-      const uint4 ch = ((const uint4 *)np)[6];
-      float t0 = child_entry(o, inv, lx.x, hx.x, ly.x, hy.x, lz.x, hz.x, ch.x, tmin, best.t);
-      float t1 = child_entry(o, inv, lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, ch.y, tmin, best.t);
-      float t2 = child_entry(o, inv, lx.z, hx.z, ly.z, hy.z, lz.z, hz.z, ch.z, tmin, best.t);
-      float t3 = child_entry(o, inv, lx.w, hx.w, ly.w, hy.w, lz.w, hz.w, ch.w, tmin, best.t);
-      uint32_t c0 = ch.x, c1 = ch.y, c2 = ch.z, c3 = ch.w;
-      // nearest first: a 4-element sorting network on the entry distances
-      cswap(t0, c0, t1, c1);
-      cswap(t2, c2, t3, c3);
-      cswap(t0, c0, t2, c2);
-      cswap(t1, c1, t3, c3);
-      cswap(t1, c1, t2, c2);
-      const float INF = __builtin_huge_valf();
-      if (t0 < INF) {
-        if (t3 < INF) push(c3);
-        if (t2 < INF) push(c2);
-        if (t1 < INF) push(c1);
-        cur = c0;
-        continue;
-      }
-    } else if (cur == LEAVE_BLAS) {
-      in_blas = false;
-      if (XF) world_ray(rorg, rdir, o, d, inv);
-      nodes = S.tlas_nodes;
-    } else {
-      // ------------------------------------------------------------ leaf
-      uint32_t first = (cur & ~LEAF_BIT) >> 3;
-      int count = (int)(cur & 7u);
-      if (!in_blas) {
-        inst = S.tlas_order[first];                  // TLAS leaves hold one instance
-        const InstDev &I = S.insts[inst];
-        blas = S.blas[I.blas];
-        if (EXT) {
-          cut.geom_base = I.geom_base;
-          cut.translucent = blas.translucent != 0;
-        }
-        if (XF && !I.identity) instance_ray(I, rorg, rdir, o, d, inv);
-        push(LEAVE_BLAS);
-        in_blas = true;
-        nodes = blas.nodes;
-        cur = 0;
-        continue;
-      }
-      bool found = false;
-      if (blas.type == BLAS_TRIANGLES) {
-        cnt.tris += count;
-        for (int k = 0; k < count; k++)
-          found |= tri_test<EXT>(blas.prims + 3 * (first + k), o, d, tmin, best, inst, cut);
-      } else if (!EXT || blas.type == BLAS_SPHERES) {
-        cnt.spheres += count;
-        for (int k = 0; k < count; k++)
-          found |= sphere_test<EXT>(blas.prims[first + k], blas.refs + first + k, o, d, tmin, best, inst, cut);
-      } else {
-        cnt.spheres += count;
-        for (int k = 0; k < count; k++)
-          found |= pair_test(blas.type, blas.prims + 2 * (first + k), blas.refs + first + k, o, d, tmin, best, inst,
-                               cut);
-      }
-      if (any_hit && found) break;
-    }
-    if (sp == 0) break;
-    cur = pop();
-  }
-  cnt.nodes += nvis;
-  return best;
+  return Octant{d.x < 0.f ? 16u : 0u, d.y < 0.f ? 48u : 32u, d.z < 0.f ? 80u : 64u};
 }
 
-// The walk of traverse() in speculative while-while order (Aila and Laine,
+// entry distance of a child whose near and far planes are known, +inf when
+// the ray misses it.  |inv| <= 1e6 (|d| >= 1e-6 after fix_dir), so the
+// distances are those of the slab test with its minima and maxima taken:
+// (plane - o) * inv is monotone in the plane.  An empty slot's planes are
+// inverted infinities: its entry lies behind its exit for every finite
+// origin, and an origin that is not finite hits nothing whichever way it
+// goes through the tree.
+BNX_D float slab_entry(v3 o, v3 inv, float nx, float fx, float ny, float fy, float nz, float fz, float tmin, float tmax)
+{
+  const float tn = fmaxf(fmaxf(fmaxf(tmin, (nx - o.x) * inv.x), (ny - o.y) * inv.y), (nz - o.z) * inv.z);
+  const float tf = fminf(fminf(fminf(tmax, (fx - o.x) * inv.x), (fy - o.y) * inv.y), (fz - o.z) * inv.z);
+  return tn <= tf * 1.00001f ? tn : __builtin_huge_valf();
+}
+
+// The walk of a wave.  Every lane walks its own ray (one node, or one leaf,
+// or into or out of an instance at a time, nearest child first) and the wave
+// runs, trip by trip, the kind of step that most of its lanes are at; lanes
+// whose rays have ended store their hits and take the next rays of the
+// wave's share together, once `take` of them are free.  A ray's own steps do
+// not depend on its wave.
+//
+// SRC: where rays come from and hits go (queue, ray array).  XF: some
+// instance transforms the ray; without it the frame never changes, so the
+// ray is not set up again.  EXT: see k_trace_static.
+template <int SH, bool EXT, bool XF, typename SRC>
+BNX_D void walk_rays(Claims &pr, const SceneDev &S, const SRC &src, int take, uint32_t *ring, Counts &cnt)
+{
+  const int lane = lane_id();
+  // stack: entries [low, sp) in the lane's ring, those below spilled.  Four
+  // move at a time, so that a node's pushes need no test of their own.
+  uint32_t *const lds = ring + lane;
+  uint32_t deep[STACK_CAP];
+  int sp = 0, low = 0;
+  auto slot = [&](int i) -> uint32_t & { return lds[(i & (SH - 1)) * 64]; };
+  auto room = [&]() {
+    if (sp - low > SH - 4) {
+      for (int k = 0; k < 4; k++) deep[low + k] = slot(low + k);
+      low += 4;
+    }
+  };
+  uint32_t cur = EMPTY4;              // EMPTY4: no ray, or one that has ended
+  auto pop = [&]() {
+    if (sp == low && sp > 0) {
+      low -= 4;
+      for (int k = 0; k < 4; k++) slot(low + k) = deep[low + k];
+    }
+    const uint32_t v = slot(sp - 1);
+    cur = sp > 0 ? v : EMPTY4;
+    sp = max(sp - 1, 0);
+  };
+  int ray = -1;
+  bool any_hit = false, in_blas = false;
+  float tmin = 0.f;
+  v3 o{0.f, 0.f, 0.f}, d{1.f, 1.f, 1.f}, inv{1.f, 1.f, 1.f};
+  Octant oct{0, 32, 64};
+  HitRec best{0.f, 0.f, 0.f, -1, -1, -1}, rej{0.f, 0.f, 0.f, -1, -1, -1};
+  const Node4 BNX_G *nodes = S.tlas_nodes;
+  Blas blas{};
+  // every node is entered at most once per ray: the walks, and so the loop,
+  // end
+  for (;;) {
+    const uint64_t idle = __ballot(cur == EMPTY4);
+    const int n_idle = __popcll(idle);
+    if (n_idle >= take && !pr.dry) {
+      if (cur == EMPTY4 && ray >= 0) src.store(S, ray, best, rej);
+      bool on;
+      const int i = pr.claim(n_idle, __popcll(idle & lanemask_lt()), on);
+      if (cur == EMPTY4) {
+        ray = -1;
+        if (on) {
+          ray = i;
+          float tmax;
+          src.load(i, o, d, tmin, tmax, any_hit);
+          d = fix_dir(d);
+          inv = v3{1.f / d.x, 1.f / d.y, 1.f / d.z};
+          oct = octant_of(d);
+          best = HitRec{tmax, 0.f, 0.f, -1, -1, -1};
+          if (EXT) rej = HitRec{__builtin_huge_valf(), 0.f, 0.f, -1, -1, -1};
+          nodes = S.tlas_nodes;
+          in_blas = false;
+          sp = low = 0;
+          cur = S.num_insts > 0 ? 0 : EMPTY4;
+        }
+      }
+      continue;
+    }
+    if (n_idle == 64) break;
+    const int n_node = __popcll(__ballot(cur < EMPTY4));
+    const int n_leaf = __popcll(__ballot(in_blas && (cur & LEAF_BIT) != 0));
+    const int n_turn = 64 - n_idle - n_node - n_leaf;
+    if (n_node >= n_leaf && n_node >= n_turn) {
+      // ------------------------------------------------ 4-wide inner node
+      if (cur < EMPTY4) {
+        cnt.nodes++;
+        const char BNX_G *np = (const char BNX_G *)(nodes + cur);
+        auto plane = [&](uint32_t off) -> float4 { return *(const float4 BNX_G *)(np + off); };
+        const float4 nx = plane(oct.x), fx = plane(oct.x ^ 16u), ny = plane(oct.y), fy = plane(oct.y ^ 16u),
+                     nz = plane(oct.z), fz = plane(oct.z ^ 16u);
+        const uint4 ch = *(const uint4 BNX_G *)(np + 96);
+        float t0 = slab_entry(o, inv, nx.x, fx.x, ny.x, fy.x, nz.x, fz.x, tmin, best.t);
+        float t1 = slab_entry(o, inv, nx.y, fx.y, ny.y, fy.y, nz.y, fz.y, tmin, best.t);
+        float t2 = slab_entry(o, inv, nx.z, fx.z, ny.z, fy.z, nz.z, fz.z, tmin, best.t);
+        float t3 = slab_entry(o, inv, nx.w, fx.w, ny.w, fy.w, nz.w, fz.w, tmin, best.t);
+        uint32_t c0 = ch.x, c1 = ch.y, c2 = ch.z, c3 = ch.w;
+        // nearest first: a 4-element sorting network on the entry distances
+        cswap(t0, c0, t1, c1);
+        cswap(t2, c2, t3, c3);
+        cswap(t0, c0, t2, c2);
+        cswap(t1, c1, t3, c3);
+        cswap(t1, c1, t2, c2);
+        const float INF = __builtin_huge_valf();
+        room();
+        slot(sp) = c3;
+        sp += t3 < INF ? 1 : 0;
+        slot(sp) = c2;
+        sp += t2 < INF ? 1 : 0;
+        slot(sp) = c1;
+        sp += t1 < INF ? 1 : 0;
+        cur = c0;
+        if (!(t0 < INF)) pop();
+      }
+    } else if (n_leaf >= n_turn) {
+      // ------------------------------------------------------------ leaf
+      if (in_blas && (cur & LEAF_BIT) != 0) {
+        const Cut cut = EXT ? src.cut(S, ray, blas.geom_base, blas.translucent, &rej) : no_cut();
+        const bool found = leaf_test<EXT>(cur, blas, o, d, tmin, best, cut, cnt);
+        if (any_hit && found) cur = EMPTY4;
+        else pop();
+      }
+    } else if (cur == LEAVE_BLAS) {
+      // ------------------------------------------- out of an instance, ...
+      in_blas = false;
+      if (XF) {
+        world_ray(src.org(ray), src.dir(ray), o, d, inv);
+        oct = octant_of(d);
+      }
+      nodes = S.tlas_nodes;
+      pop();
+    } else if (!in_blas && (cur & LEAF_BIT) != 0) {
+      // ------------------------------------ ... or a TLAS leaf: into its own
+      if (enter_instance<XF>(S.enter + ((cur & ~LEAF_BIT) >> 3), src.org(ray), src.dir(ray), blas, o, d, inv))
+        oct = octant_of(d);
+      room();
+      slot(sp++) = LEAVE_BLAS;
+      in_blas = true;
+      nodes = blas.nodes;
+      cur = 0;
+    }
+  }
+  if (ray >= 0) src.store(S, ray, best, rej);
+}
+
+// The walk of a ray in speculative while-while order (Aila and Laine,
 // "Understanding the Efficiency of Ray Traversal on GPUs", HPG 2009): a
 // lane that reaches a primitive leaf sets it aside and keeps stepping inner
 // nodes from its stack while other lanes of the wave still step nodes, until
@@ -457,10 +579,9 @@ BNX_D HitRec traverse_spec(const SceneDev &S, const float4 *rorg, const float4 *
   HitRec best{tmax, 0.f, 0.f, -1, -1, -1};
   v3 o, d, inv;
   world_ray(rorg, rdir, o, d, inv);
-  const Node4 *nodes = S.tlas_nodes;
-  BlasDev blas{};
+  const Node4 BNX_G *nodes = S.tlas_nodes;
+  Blas blas{};
   bool in_blas = false;
-  int inst = -1;
   uint32_t cur = 0;
   uint32_t leaf = 0;             // primitive leaf set aside (leaf codes carry LEAF_BIT)
   uint32_t nvis = 0;
@@ -505,35 +626,15 @@ BNX_D HitRec traverse_spec(const SceneDev &S, const float4 *rorg, const float4 *
     // ------------------------------------------------------- leaf phase
     bool found = false;
     if (leaf != 0) {
-      const uint32_t first = (leaf & ~LEAF_BIT) >> 3;
-      const int count = (int)(leaf & 7u);
-      if (blas.type == BLAS_TRIANGLES) {
-        cnt.tris += count;
-        for (int k = 0; k < count; k++)
-          found |= tri_test<EXT>(blas.prims + 3 * (first + k), o, d, tmin, best, inst, cut);
-      } else if (!EXT || blas.type == BLAS_SPHERES) {
-        cnt.spheres += count;
-        for (int k = 0; k < count; k++)
-          found |= sphere_test<EXT>(blas.prims[first + k], blas.refs + first + k, o, d, tmin, best, inst, cut);
-      } else {
-        cnt.spheres += count;
-        for (int k = 0; k < count; k++)
-          found |= pair_test(blas.type, blas.prims + 2 * (first + k), blas.refs + first + k, o, d, tmin, best, inst,
-                               cut);
-      }
+      found = leaf_test<EXT>(leaf, blas, o, d, tmin, best, cut, cnt);
       leaf = 0;
     } else if ((cur & LEAF_BIT) && !in_blas) {
       // a TLAS leaf (the node phase sets every BLAS leaf aside): enter its
       // instance
-      inst = S.tlas_order[(cur & ~LEAF_BIT) >> 3];
-      const InstDev &I = S.insts[inst];
-      blas = S.blas[I.blas];
+      (void)enter_instance<XF>(S.enter + ((cur & ~LEAF_BIT) >> 3), rorg, rdir, blas, o, d, inv);
       if (EXT) {
-        cut.geom_base = I.geom_base;
-        cut.translucent = blas.translucent != 0;
-      }
-      if (XF && !I.identity) {
-        instance_ray(I, rorg, rdir, o, d, inv);
+        cut.geom_base = blas.geom_base;
+        cut.translucent = blas.translucent;
       }
       push(LEAVE_BLAS);
       in_blas = true;
@@ -552,27 +653,41 @@ BNX_D HitRec traverse_spec(const SceneDev &S, const float4 *rorg, const float4 *
   return best;
 }
 
-__global__ __launch_bounds__(TB) void k_trace_api(SceneDev S, const bnx_ray *rays, int n, bnx_hit *hits,
-                                                  uint32_t flags)
-{
-  __shared__ uint32_t ring[API_SHORT * TB];
-  uint32_t *lds = ring + threadIdx.x;
+// Into how many chunks a launch is cut at least.  Half as many as waves: full
+// waves before all waves (1.05M triangles, 512x512, 1 spp: 406 us in three
+// launches, and 552 with a chunk for each; 60001 rays: 111 and 135).  The
+// extended kernels run a leaf step once for each kind of primitive in the
+// wave, and a wave with 64 long rays is one that the launch waits for: twice
+// as many as waves (instances of four kinds, 640x360: 3.3 ms, and 4.7 with
+// half as many).
+BNX_D int least_chunks(bool ext) { return ext ? 2 * (int)gridDim.x : (int)gridDim.x / 2; }
+
+// rays and hits of the ray-array entry point
+struct ArraySource {
+  const bnx_ray *rays;
+  bnx_hit *hits;
+  bool any;
+  BNX_D const float4 *org(int i) const { return (const float4 *)(rays + i); }
+  BNX_D const float4 *dir(int i) const { return (const float4 *)(rays + i) + 1; }
+  BNX_D void load(int i, v3 &o, v3 &d, float &tmin, float &tmax, bool &any_hit) const
   {
-    const int i = blockIdx.x * TB + threadIdx.x;
-    if (i >= n) return;
-    const float4 *rp = (const float4 *)(rays + i);
-    float4 r0 = rp[0], r1 = rp[1];
-    Counts cnt{0, 0, 0};
-    HitRec rej{__builtin_huge_valf(), 0.f, 0.f, -1, -1, -1};
-    HitRec h = traverse<API_SHORT, true, true>(S, rp, rp + 1, r0.w, r1.w, (flags & BNX_TRACE_ANY) != 0, lds, cnt,
-                                               no_cut().plane, nullptr, rej);
+    const float4 r0 = *org(i), r1 = *dir(i);
+    o = xyz(r0);
+    d = xyz(r1);
+    tmin = r0.w;
+    tmax = r1.w;
+    any_hit = any;
+  }
+  BNX_D Cut cut(const SceneDev &, int, int, bool, HitRec *) const { return no_cut(); }
+  BNX_D void store(const SceneDev &S, int i, const HitRec &h, const HitRec &) const
+  {
     bnx_hit out;
     out.t = h.t;
     out.u = h.prim >= 0 ? h.u : 0.f;
     out.v = h.prim >= 0 ? h.v : 0.f;
     out.prim_id = h.prim;
     if (h.prim >= 0) {
-      const InstDev &I = S.insts[h.inst];
+      const InstDev &I = *(const InstDev *)(S.insts + h.inst);
       out.geom_id = h.geom;
       out.inst = h.inst;
       out.user_inst_id = I.user_id;
@@ -582,6 +697,18 @@ __global__ __launch_bounds__(TB) void k_trace_api(SceneDev S, const bnx_ray *ray
     }
     hits[i] = out;
   }
+};
+
+template <bool EXT, bool XF>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BNX_TRACE_WAVES))) void k_trace_api(
+    SceneDev S, const bnx_ray *rays, int n, bnx_hit *hits, uint32_t flags, int *claims)
+{
+  __shared__ uint32_t ring[API_SHORT * 64];
+  Claims cl;
+  cl.begin(n, claims, least_chunks(EXT));
+  Counts cnt{0, 0, 0};
+  const ArraySource src{rays, hits, (flags & BNX_TRACE_ANY) != 0};
+  walk_rays<API_SHORT, EXT, XF>(cl, S, src, TAKE, ring, cnt);
 }
 
 // A translucent candidate the opacity test rejected lies in front of the
@@ -606,11 +733,10 @@ BNX_D void translucent_ids(const SlotDev &P, const TraceQueue &q, int i, float4 
 // each block lies inside one request's segment, so the request's scene
 // pointers are block-uniform.  counters: statistics array (STAT_NODES,
 // STAT_TRIS, STAT_SPHERES)
-template <int SH, bool SPEC, bool EXT, bool XF>
-BNX_D void trace_static(const SlotDev *__restrict__ slots, const SegView &sv, const TraceQueue &q,
-                        unsigned long long *counters)
+template <int SH, bool EXT, bool XF>
+BNX_D void trace_spec(const SlotDev *__restrict__ slots, const SegView &sv, const TraceQueue &q,
+                      unsigned long long *counters, uint32_t *ring)
 {
-  __shared__ uint32_t ring[SH * TB];
   uint32_t *lds = ring + threadIdx.x;
   Counts cnt{0, 0, 0};
   int i;
@@ -625,10 +751,7 @@ BNX_D void trace_static(const SlotDev *__restrict__ slots, const SegView &sv, co
     HitRec h{o.w, 0.f, 0.f, -1, -1, -1};
     HitRec rej{__builtin_huge_valf(), 0.f, 0.f, -1, -1, -1};
     if (S.num_insts > 0)
-      h = SPEC ? traverse_spec<SH, EXT, XF>(S, q.org + i, q.dir + i, 0.f, o.w, shadow, lds, cnt, cut_plane,
-                                            q.rng + i, rej)
-               : traverse<SH, EXT, XF>(S, q.org + i, q.dir + i, 0.f, o.w, shadow, lds, cnt, cut_plane, q.rng + i,
-                                       rej);
+      h = traverse_spec<SH, EXT, XF>(S, q.org + i, q.dir + i, 0.f, o.w, shadow, lds, cnt, cut_plane, q.rng + i, rej);
     if (h.prim >= 0) q.org[i].w = h.t;
     q.hit[i] = make_int4(h.prim, h.geom, h.inst, __float_as_int(h.u));
     q.hit_v[i] = h.v;
@@ -642,201 +765,53 @@ BNX_D void trace_static(const SlotDev *__restrict__ slots, const SegView &sv, co
   }
 }
 
-// EXT: the leaf test knows cylinder BLASes and the cut plane of each
-// request.  The kernels without it serve worlds of triangles and spheres
-// traced without a cut plane; the launcher takes the _ext kernels while any
-// built world holds cylinders or a request in the launch has a cut plane.
-template <int SH, bool SPEC, bool XF>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BNX_TRACE_WAVES))) void k_trace_static(
-    const SlotDev *__restrict__ slots, SegView sv, TraceQueue q, unsigned long long *counters)
-{
-  trace_static<SH, SPEC, false, XF>(slots, sv, q, counters);
-}
-
-template <int SH, bool SPEC, bool XF>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BNX_TRACE_WAVES))) void k_trace_static_ext(
-    const SlotDev *__restrict__ slots, SegView sv, TraceQueue q, unsigned long long *counters)
-{
-  trace_static<SH, SPEC, true, XF>(slots, sv, q, counters);
-}
-
-// The generation's rays, segment by segment: every block lies inside one
-// request's segment (its scene pointers are block-uniform) and draws rays
-// from the segment's pool.  A wave claims POOL_CHUNK ray indices at a time
-// (one atomic per chunk) and hands them to its lanes as they finish, so a
-// lane whose walk ends early takes the next ray instead of idling until the
-// wave's longest walk is over.  The walk is the one of traverse() above,
-// taken one node or leaf per loop trip.
-constexpr int POOL_CHUNK = 64;
-
-template <int SH, bool EXT, bool XF>
-BNX_D void trace_pool(const SlotDev *__restrict__ slots, const SegView &sv, const TraceQueue &q,
-                      unsigned long long *counters)
-{
-  __shared__ uint32_t ring[SH * TB];
-  uint32_t *lds = ring + threadIdx.x;
-  uint32_t deep[STACK_CAP - SH];
-  int sp = 0;
-  auto push = [&](uint32_t v) {
-    const int s = sp & (SH - 1);
-    if (sp >= SH) deep[sp - SH] = lds[s * TB];
-    lds[s * TB] = v;
-    sp++;
-  };
-  auto pop = [&]() -> uint32_t {
-    sp--;
-    const int s = sp & (SH - 1);
-    const uint32_t v = lds[s * TB];
-    if (sp >= SH) lds[s * TB] = deep[sp - SH];
-    return v;
-  };
-  const int seg = sv.blkT[blockIdx.x];
-  const Segment sg = sv.segs[seg];
-  const SceneDev S = slots[sg.slot].scene;
-  const float4 cut_plane = EXT ? slot_cut_plane(slots[sg.slot]) : no_cut().plane;
-  const bool empty_scene = S.num_insts == 0;
-  const int refill_at = sg.refill;
-  Counts cnt{0, 0, 0};
-  // per-lane walk state
-  bool active = false, any_hit = false, in_blas = false;
-  int ray = 0, inst = -1;
-  v3 o{0.f, 0.f, 0.f}, d{1.f, 1.f, 1.f}, inv{1.f, 1.f, 1.f};
-  HitRec best{0.f, 0.f, 0.f, -1, -1, -1};
-  HitRec rej{0.f, 0.f, 0.f, -1, -1, -1};
-  int geom_base = 0;     // EXT: the lane's instance's first geometry-table entry
-  const Node4 *nodes = S.tlas_nodes;
-  BlasDev blas{};
-  uint32_t cur = 0;
-  // wave-uniform chunk [q_next, q_end) of segment-local ray indices: first
-  // the wave's own chunk of the segment's static part, then chunks from the
-  // pool (whose counter starts where the static part ends)
-  int q_next = (((int)blockIdx.x - sg.blockT) * (TB / 64) + (int)(threadIdx.x >> 6)) * POOL_CHUNK;
-  int q_end = min(q_next + POOL_CHUNK, sg.count);
-  bool dry = false;
-  for (;;) {
-    // ------------------------------------------------------- refill
-    const bool need = !active;
-    const uint64_t mask = __ballot(need);
-    if (mask != 0 && !dry) {
-      if (q_next >= q_end) {
-        int base = 0;
-        if (lane_id() == 0) base = atomicAdd(sv.pool + seg, POOL_CHUNK);
-        base = __builtin_amdgcn_readfirstlane(base);
-        if (base >= sg.count) {
-          dry = true;
-          q_next = q_end = 0;
-        } else {
-          q_next = base;
-          q_end = min(base + POOL_CHUNK, sg.count);
-        }
-      }
-      const int avail = max(0, q_end - q_next);
-      const int rank = __popcll(mask & lanemask_lt());
-      if (need && rank < avail) {
-        ray = sg.begin + q_next + rank;
-        const float4 ro = q.org[ray], rd = q.dir[ray];
-        any_hit = (__float_as_uint(rd.w) & FLAG_SHADOW) != 0;
-        o = xyz(ro);
-        d = fix_dir(xyz(rd));
-        inv = v3{1.f / d.x, 1.f / d.y, 1.f / d.z};
-        best = HitRec{ro.w, 0.f, 0.f, -1, -1, -1};
-        rej = HitRec{__builtin_huge_valf(), 0.f, 0.f, -1, -1, -1};
-        nodes = S.tlas_nodes;
-        in_blas = false;
-        inst = -1;
-        cur = 0;
-        sp = 0;
-        active = true;
-      }
-      q_next += min(__popcll(mask), avail);
-    }
-    if (__ballot(active) == 0) break;
-    // ---------------------------------------- walk until enough lanes idle
-    while (active) {
-      bool done = false;
-      if (empty_scene) {
-        done = true;
-      } else if (cur < EMPTY4) {
-        const float4 *np = (const float4 *)(nodes + cur);
-        const float4 lx = np[0], hx = np[1], ly = np[2], hy = np[3], lz = np[4], hz = np[5];
-        const uint4 ch = ((const uint4 *)np)[6];
-        cnt.nodes++;
-        float t0 = child_entry(o, inv, lx.x, hx.x, ly.x, hy.x, lz.x, hz.x, ch.x, 0.f, best.t);
-        float t1 = child_entry(o, inv, lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, ch.y, 0.f, best.t);
-        float t2 = child_entry(o, inv, lx.z, hx.z, ly.z, hy.z, lz.z, hz.z, ch.z, 0.f, best.t);
-        float t3 = child_entry(o, inv, lx.w, hx.w, ly.w, hy.w, lz.w, hz.w, ch.w, 0.f, best.t);
-        uint32_t c0 = ch.x, c1 = ch.y, c2 = ch.z, c3 = ch.w;
-        cswap(t0, c0, t1, c1);
-        cswap(t2, c2, t3, c3);
-        cswap(t0, c0, t2, c2);
-        cswap(t1, c1, t3, c3);
-        cswap(t1, c1, t2, c2);
-        const float INF = __builtin_huge_valf();
-        if (t0 < INF) {
-          if (t3 < INF) push(c3);
-          if (t2 < INF) push(c2);
-          if (t1 < INF) push(c1);
-          cur = c0;
-        } else if (sp == 0) {
-          done = true;
-        } else {
-          cur = pop();
-        }
-      } else if (cur == LEAVE_BLAS) {
-        in_blas = false;
-        if (XF) world_ray(q.org + ray, q.dir + ray, o, d, inv);
-        nodes = S.tlas_nodes;
-        if (sp == 0) done = true;
-        else cur = pop();
-      } else {
-        const uint32_t first = (cur & ~LEAF_BIT) >> 3;
-        const int count = (int)(cur & 7u);
-        if (!in_blas) {
-          inst = S.tlas_order[first];                  // TLAS leaves hold one instance
-          const InstDev &I = S.insts[inst];
-          blas = S.blas[I.blas];
-          geom_base = I.geom_base;
-          if (XF && !I.identity) {
-            instance_ray(I, q.org + ray, q.dir + ray, o, d, inv);
-          }
-          push(LEAVE_BLAS);
-          in_blas = true;
-          nodes = blas.nodes;
-          cur = 0;
-        } else {
-          bool found = false;
-          const Cut cut{cut_plane, q.org + ray, q.dir + ray, q.rng + ray, &S, geom_base, blas.translucent != 0, &rej};
-          if (blas.type == BLAS_TRIANGLES) {
-            cnt.tris += count;
-            for (int k = 0; k < count; k++)
-              found |= tri_test<EXT>(blas.prims + 3 * (first + k), o, d, 0.f, best, inst, cut);
-          } else if (!EXT || blas.type == BLAS_SPHERES) {
-            cnt.spheres += count;
-            for (int k = 0; k < count; k++)
-              found |= sphere_test<EXT>(blas.prims[first + k], blas.refs + first + k, o, d, 0.f, best, inst, cut);
-          } else {
-            cnt.spheres += count;
-            for (int k = 0; k < count; k++)
-              found |= pair_test(blas.type, blas.prims + 2 * (first + k), blas.refs + first + k, o, d, 0.f, best,
-                                   inst, cut);
-          }
-          if ((any_hit && found) || sp == 0) done = true;
-          else cur = pop();
-        }
-      }
-      if (done) {
-        if (best.prim >= 0) q.org[ray].w = best.t;
-        q.hit[ray] = make_int4(best.prim, best.geom, best.inst, __float_as_int(best.u));
-        q.hit_v[ray] = best.v;
-        if (EXT && rej.prim >= 0 && rej.t < best.t) translucent_ids(slots[sg.slot], q, ray, q.dir[ray], rej);
-        active = false;
-      }
-      // leave the walk for a refill once refill_at lanes are idle (the test
-      // is wave-uniform, so the lanes still walking leave together)
-      if (!dry && 64 - __popcll(__ballot(true)) >= refill_at) break;
-    }
+// the rays of a request's segment
+struct QueueSource {
+  const TraceQueue &q;
+  const SlotDev &P;
+  float4 plane;
+  BNX_D const float4 *org(int i) const { return q.org + i; }
+  BNX_D const float4 *dir(int i) const { return q.dir + i; }
+  BNX_D void load(int i, v3 &o, v3 &d, float &tmin, float &tmax, bool &any_hit) const
+  {
+    const float4 ro = q.org[i], rd = q.dir[i];
+    o = xyz(ro);
+    d = xyz(rd);
+    tmin = 0.f;
+    tmax = ro.w;
+    any_hit = (__float_as_uint(rd.w) & FLAG_SHADOW) != 0;
   }
-  uint32_t a = wave_sum(cnt.nodes), b = wave_sum(cnt.tris), c = wave_sum(cnt.spheres);
+  BNX_D Cut cut(const SceneDev &S, int i, int geom_base, bool translucent, HitRec *rej) const
+  {
+    return Cut{plane, q.org + i, q.dir + i, q.rng + i, &S, geom_base, translucent, rej};
+  }
+  BNX_D void store(const SceneDev &, int i, const HitRec &h, const HitRec &rej) const
+  {
+    if (h.prim >= 0) q.org[i].w = h.t;
+    q.hit[i] = make_int4(h.prim, h.geom, h.inst, __float_as_int(h.u));
+    q.hit_v[i] = h.v;
+    if (rej.prim >= 0 && rej.t < h.t) translucent_ids(P, q, i, q.dir[i], rej);
+  }
+};
+
+// a wave's share of the generation, segment by segment (each one request's,
+// so the scene's pointers are wave-uniform)
+template <int SH, bool EXT, bool XF>
+BNX_D void trace_waves(const SlotDev *__restrict__ slots, const SegView &sv, int nsegs, const TraceQueue &q,
+                       unsigned long long *counters, uint32_t *ring)
+{
+  Claims cl;
+  cl.begin(sv, nsegs, CLAIMS_TRACE, least_chunks(EXT));
+  Counts cnt{0, 0, 0};
+  while (cl.chunk >= 0) {
+    const Segment sg = cl.open();
+    const SlotDev &P = slots[sg.slot];
+    const SceneDev S = uniform_load((const SceneDev BNX_G *)&P.scene);
+    cl.refill();
+    const QueueSource src{q, P, EXT ? slot_cut_plane(P) : no_cut().plane};
+    walk_rays<SH, EXT, XF>(cl, S, src, sg.refill < 64 ? sg.refill : TAKE, ring, cnt);
+  }
+  const uint32_t a = wave_sum(cnt.nodes), b = wave_sum(cnt.tris), c = wave_sum(cnt.spheres);
   if (lane_id() == 0) {
     stat_add(counters, STAT_NODES, a);
     stat_add(counters, STAT_TRIS, b);
@@ -844,50 +819,64 @@ BNX_D void trace_pool(const SlotDev *__restrict__ slots, const SegView &sv, cons
   }
 }
 
-template <int SH, bool XF>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BNX_TRACE_WAVES))) void k_trace_pool(
-    const SlotDev *__restrict__ slots, SegView sv, TraceQueue q, unsigned long long *counters)
+// The trace of a generation.  SPEC: one ray per thread in blocks of TB, the
+// speculative walk; otherwise waves that share the rays out.  EXT: the leaf
+// test knows cylinder BLASes and the cut plane of each request.  The kernels
+// without it serve worlds of triangles and spheres traced without a cut
+// plane; the launcher takes the _ext kernels while any built world holds
+// cylinders or a request in the launch has a cut plane.
+template <int SH, bool SPEC, bool EXT, bool XF>
+BNX_D void trace_queue(const SlotDev *__restrict__ slots, const SegView &sv, int nsegs, const TraceQueue &q,
+                       unsigned long long *counters, uint32_t *ring)
 {
-  trace_pool<SH, false, XF>(slots, sv, q, counters);
+  if constexpr (SPEC) trace_spec<SH, EXT, XF>(slots, sv, q, counters, ring);
+  else trace_waves<SH, EXT, XF>(slots, sv, nsegs, q, counters, ring);
 }
+constexpr int trace_block(bool spec) { return spec ? TB : 64; }
 
-template <int SH, bool XF>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BNX_TRACE_WAVES))) void k_trace_pool_ext(
-    const SlotDev *__restrict__ slots, SegView sv, TraceQueue q, unsigned long long *counters)
+template <int SH, bool SPEC, bool XF>
+__global__ __launch_bounds__(trace_block(SPEC)) __attribute__((amdgpu_waves_per_eu(BNX_TRACE_WAVES))) void
+k_trace_static(const SlotDev *__restrict__ slots, SegView sv, int nsegs, TraceQueue q, unsigned long long *counters)
 {
-  trace_pool<SH, true, XF>(slots, sv, q, counters);
+  __shared__ uint32_t ring[SH * trace_block(SPEC)];
+  trace_queue<SH, SPEC, false, XF>(slots, sv, nsegs, q, counters, ring);
 }
 
 template <int SH, bool SPEC, bool XF>
-void launch_static_xf(Device *dev, bool ext, int blocks, const SlotDev *slots, const SegView &sv,
-                      const TraceQueue &q, unsigned long long *counters)
+__global__ __launch_bounds__(trace_block(SPEC)) __attribute__((amdgpu_waves_per_eu(BNX_TRACE_WAVES))) void
+k_trace_static_ext(const SlotDev *__restrict__ slots, SegView sv, int nsegs, TraceQueue q,
+                   unsigned long long *counters)
 {
-  if (ext) k_trace_static_ext<SH, SPEC, XF><<<blocks, TB, 0, dev->stream>>>(slots, sv, q, counters);
-  else k_trace_static<SH, SPEC, XF><<<blocks, TB, 0, dev->stream>>>(slots, sv, q, counters);
+  __shared__ uint32_t ring[SH * trace_block(SPEC)];
+  trace_queue<SH, SPEC, true, XF>(slots, sv, nsegs, q, counters, ring);
 }
 
-template <int SH, bool SPEC>
-void launch_static(Device *dev, bool ext, bool xf, int blocks, const SlotDev *slots, const SegView &sv,
-                   const TraceQueue &q, unsigned long long *counters)
+using TraceKernel = void (*)(const SlotDev *, SegView, int, TraceQueue, unsigned long long *);
+template <int SH, bool SPEC, bool XF> TraceKernel trace_kernel(bool ext)
 {
-  if (xf) launch_static_xf<SH, SPEC, true>(dev, ext, blocks, slots, sv, q, counters);
-  else launch_static_xf<SH, SPEC, false>(dev, ext, blocks, slots, sv, q, counters);
+  return ext ? k_trace_static_ext<SH, SPEC, XF> : k_trace_static<SH, SPEC, XF>;
+}
+template <int SH> TraceKernel trace_kernel(bool spec, bool ext, bool xf)
+{
+  if (spec) return xf ? trace_kernel<SH, true, true>(ext) : trace_kernel<SH, true, false>(ext);
+  return xf ? trace_kernel<SH, false, true>(ext) : trace_kernel<SH, false, false>(ext);
 }
 
-template <int SH>
-void launch_pool(Device *dev, bool ext, bool xf, int blocks, const SlotDev *slots, const SegView &sv,
-                 const TraceQueue &q, unsigned long long *counters)
+// waves of a launch over n rays: as many as are resident at once, in whole
+// rounds of the claim groups, and no more than there are chunks of 16 rays
+int trace_waves_for(const Device *dev, int fit, long long blocks256)
 {
-  if (ext) {
-    if (xf) k_trace_pool_ext<SH, true><<<blocks, TB, 0, dev->stream>>>(slots, sv, q, counters);
-    else k_trace_pool_ext<SH, false><<<blocks, TB, 0, dev->stream>>>(slots, sv, q, counters);
-  } else {
-    if (xf) k_trace_pool<SH, true><<<blocks, TB, 0, dev->stream>>>(slots, sv, q, counters);
-    else k_trace_pool<SH, false><<<blocks, TB, 0, dev->stream>>>(slots, sv, q, counters);
+  const long long waves = std::min<long long>((long long)fit * dev->num_cus, 16 * blocks256);
+  return (int)std::max<long long>(CLAIM_GROUPS, waves / CLAIM_GROUPS * CLAIM_GROUPS);
+}
+template <typename K> int resident(K kernel, int &fit)
+{
+  if (fit == 0) {
+    BNX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, (const void *)kernel, 64, 0));
+    fit = std::max(1, fit);
   }
+  return BNX_OK;
 }
-
-int grid_for(int n) { return n > 0 ? (n + TB - 1) / TB : 1; }
 
 } // namespace
 
@@ -896,37 +885,37 @@ int trace_stack_capacity() { return STACK_CAP; }
 int launch_trace_api(Group *g, const bnx_ray *d_rays, int n, bnx_hit *d_hits, uint32_t flags)
 {
   Device *dev = g->dev;
-  k_trace_api<<<grid_for(n), TB, 0, dev->stream>>>(g->scene, d_rays, n, d_hits, flags);
+  if (n <= 0) return BNX_OK;
+  const bool ext = g->has_cyl, xf = g->has_xf;
+  const auto kernel = ext ? (xf ? k_trace_api<true, true> : k_trace_api<true, false>)
+                          : (xf ? k_trace_api<false, true> : k_trace_api<false, false>);
+  int &fit = dev->trace_fit[12 + 2 * (ext ? 1 : 0) + (xf ? 1 : 0)];
+  int rc = resident(kernel, fit);
+  if (rc != BNX_OK) return rc;
+  const std::lock_guard<std::mutex> one(dev->api_mutex);
+  if ((rc = launch_claims_clear(dev, dev->api_claims.as<int>())) != BNX_OK) return rc;
+  kernel<<<trace_waves_for(dev, fit, ((long long)n + 255) / 256), 64, 0, dev->stream>>>(
+      g->scene, d_rays, n, d_hits, flags, dev->api_claims.as<int>());
   BNX_HIP(hipGetLastError());
   return BNX_OK;
 }
 
-int launch_trace_queue(Device *dev, const SlotDev *slots, const SegView &sv, int blocks256, int blocksT, bool pooled,
-                       bool cut, const TraceQueue &q, unsigned long long *counters)
+int launch_trace_queue(Device *dev, const SlotDev *slots, const SegView &sv, int nsegs, int blocks256, bool cut,
+                       const TraceQueue &q, unsigned long long *counters)
 {
+  if (blocks256 <= 0) return BNX_OK;
   const int sh = dev->trace_stack_lds;
-  const bool ext = ext_kernels(dev, cut);
-  const bool xf = dev->xf_worlds > 0;
-  if (pooled) {
-    if (blocksT > 0) {
-      if (sh == 8) launch_pool<8>(dev, ext, xf, blocksT, slots, sv, q, counters);
-      else if (sh == 32) launch_pool<32>(dev, ext, xf, blocksT, slots, sv, q, counters);
-      else launch_pool<16>(dev, ext, xf, blocksT, slots, sv, q, counters);
-    }
+  const bool ext = ext_kernels(dev, cut), xf = dev->xf_worlds > 0, spec = dev->trace_walk == 1;
+  const TraceKernel kernel = sh == 8    ? trace_kernel<8>(spec, ext, xf)
+                             : sh == 32 ? trace_kernel<32>(spec, ext, xf)
+                                        : trace_kernel<16>(spec, ext, xf);
+  if (spec) {
+    kernel<<<blocks256, TB, 0, dev->stream>>>(slots, sv, nsegs, q, counters);
   } else {
-    if (blocks256 > 0) {
-      const bool spec = dev->trace_walk == 1;
-      if (sh == 8) {
-        if (spec) launch_static<8, true>(dev, ext, xf, blocks256, slots, sv, q, counters);
-        else launch_static<8, false>(dev, ext, xf, blocks256, slots, sv, q, counters);
-      } else if (sh == 32) {
-        if (spec) launch_static<32, true>(dev, ext, xf, blocks256, slots, sv, q, counters);
-        else launch_static<32, false>(dev, ext, xf, blocks256, slots, sv, q, counters);
-      } else {
-        if (spec) launch_static<16, true>(dev, ext, xf, blocks256, slots, sv, q, counters);
-        else launch_static<16, false>(dev, ext, xf, blocks256, slots, sv, q, counters);
-      }
-    }
+    int &fit = dev->trace_fit[4 * (sh == 8 ? 0 : sh == 32 ? 2 : 1) + 2 * (ext ? 1 : 0) + (xf ? 1 : 0)];
+    const int rc = resident(kernel, fit);
+    if (rc != BNX_OK) return rc;
+    kernel<<<trace_waves_for(dev, std::min(fit, 4 * dev->trace_blocks_per_cu), blocks256), 64, 0, dev->stream>>>(slots, sv, nsegs, q, counters);
   }
   BNX_HIP(hipGetLastError());
   return BNX_OK;

@@ -213,8 +213,8 @@ int bnx_autotune(bnx_world world, const bnx_camera *camera, const bnx_renderer *
           stack_walks);
     if (rc == BNX_OK) rc = sweep([](bnx_tuning &t, int v) { t.sort_rays = v; }, onoff);
     if (rc == BNX_OK) rc = sweep([](bnx_tuning &t, int v) { t.shade_block = v; }, shade_blocks);
-    // the refill threshold for worlds of this size: 64 keeps one ray per
-    // thread for them; below 64 the pooled trace takes their secondary rays
+    // the refill threshold of secondary rays for worlds of this size: 64
+    // keeps the trace's own
     if (rc == BNX_OK)
       rc = sweep(
           [prims, &start](bnx_tuning &t, int v) {

@@ -111,15 +111,12 @@ def umesh_bytes(nodes, tets, cells, rays):
     return 64.0 * nodes + 80.0 * tets + 4.0 * cells + 48.0 * rays
 
 
-def trace_kernel_name(tuning, max_world_prims):
-    """the queue-trace kernels that ran: the LDS-stack and walk variant of
-    the tuning, for worlds without instance transforms (the bench worlds);
-    the pooled kernel too when a world is large enough to use it"""
+def trace_kernel_name(tuning):
+    """the queue-trace kernel that ran: the LDS-stack and walk variant of the
+    tuning, for worlds without instance transforms (the bench worlds)"""
     sh = tuning["trace_stack_lds"]
     walk = "true" if tuning.get("trace_walk", 0) == 1 else "false"
-    pooled = tuning["trace_refill"] < 64 and max_world_prims >= tuning["trace_refill_prims"]
-    static = f"k_trace_static<{sh}, {walk}, false>"
-    return f"{static}+k_trace_pool<{sh}, false>" if pooled else static
+    return f"k_trace_static<{sh}, {walk}, false>"
 
 
 def roofline(tot, workload=None, trace_kernel="k_trace_static<16, false, false>", trace_bytes=None, model=None):
@@ -785,7 +782,7 @@ def main():
         "warmup": warmup, "ms_per_step": round(elapsed * 1e3 / steps, 4), "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic (seeded PCG32 scenes and stream)",
         "config": desc, "frame_latency_ms": lat_line,
-        "roofline": roofline(tot, args.workload, trace_kernel_name(desc["tuning"], desc.get("max_world_prims", 0)),
+        "roofline": roofline(tot, args.workload, trace_kernel_name(desc["tuning"]),
                              trace_bytes, model),
     }
     if byte_detail and line["roofline"]["kernel"].startswith("k_trace"):

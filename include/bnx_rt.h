@@ -409,7 +409,7 @@ int bnx_device_restore_active(int previous_gpu);
  * Launch parameters of the render path, per device.  None of them changes a
  * result: they set the order in which primary rays enter the queue, how the
  * traversal stack is split between LDS and private memory, the size of the
- * pooled trace launch and how many paths bnx_render keeps in flight.  No
+ * trace launch and how many paths bnx_render keeps in flight.  No
  * counterpart in the reference, whose launch shapes are fixed (one thread
  * per ray in blocks of 256, kernels/traceRays.cu:20-121; all of a frame's
  * pixels per generation, native/Context.cpp:139-182); bnx_autotune chooses
@@ -421,19 +421,21 @@ typedef struct bnx_tuning {
   int32_t trace_stack_lds;          /* traversal-stack entries per lane kept in LDS:
                                        8, 16 or 32 (of 192; the rest in private
                                        memory)                                       */
-  int32_t trace_blocks_per_cu;      /* pooled trace launch: blocks per CU, 1..64     */
-  int32_t trace_refill;             /* pooled trace: idle lanes of a wave that make
-                                       it draw new rays, 1..64                       */
-  int32_t trace_walk;               /* one-ray-per-thread walk: 0 = a node step or a
-                                       leaf per trip; 1 = speculative while-while
-                                       (leaves set aside until every lane has one)  */
+  int32_t trace_blocks_per_cu;      /* trace launch: at most this many times four
+                                       waves per CU, 1..64                           */
+  int32_t trace_refill;             /* idle lanes that make a trace wave take new
+                                       rays, 1..64 (64: as for other worlds)         */
+  int32_t trace_walk;               /* 0 = waves that take new rays as walks end, a
+                                       node step or a leaf per trip; 1 = one ray per
+                                       thread, speculative while-while (leaves set
+                                       aside until every lane has one)               */
   int32_t sort_rays;                /* bnx_render: 1 = reorder each secondary
                                        generation of 2^16 rays or more by shadow
                                        flag, direction octant and origin Morton
                                        code before tracing it (0: queue order)      */
   int32_t shade_block;              /* threads per shade block: 256 or 1024          */
   int64_t trace_refill_prims;       /* secondary generations of worlds with at least
-                                       this many primitives use the pooled trace     */
+                                       this many primitives use trace_refill         */
   int64_t render_paths;             /* bnx_render: paths per batch of samples,
                                        2^16 .. 2^26                                  */
   int64_t graph_paths;              /* bnx_render: a batch of at most this many
@@ -459,7 +461,7 @@ typedef struct bnx_autotune_report {
 
 /* Choose the device's tuning for requests like this one: coordinate descent,
  * two passes, over the fields of bnx_tuning (raygen tile, LDS stack entries,
- * walk order, ray reordering, shade block, refill threshold, pooled-launch size, paths per batch, captured-loop
+ * walk order, ray reordering, shade block, refill threshold, trace-launch size, paths per batch, captured-loop
  * limit), each candidate timed on
  * probe renders of width x height at probe_spp samples into a scratch frame
  * (best of 2 to 20, so that each candidate is timed for about 10 ms; a

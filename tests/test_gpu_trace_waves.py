@@ -1,0 +1,86 @@
+"""The trace kernels' waves where they can go wrong, against the CPU oracle:
+ray counts at the edges of a wave, of a chunk and of a 256-ray block, for
+every variant of the ray-array kernel (triangles and spheres, or all
+primitives; with and without instance transforms); rays along and against
+every axis and rays that are not finite; and rays traced by several threads
+of one device at once.  Hits are compared bit for bit."""
+import threading
+
+import numpy as np
+import pytest
+
+from barney_amd import scenes
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+SPECS = {"plain": helpers.soup_spec, "xf": helpers.instanced_spec,
+         "ext": lambda: helpers.sticks_spec(False), "ext_xf": lambda: helpers.sticks_spec(True)}
+
+
+def _same(g, o):
+    bad = helpers.hits_equal(g, o)
+    assert len(bad) == 0, (len(bad), g[bad[:3]], o[bad[:3]])
+
+
+@pytest.mark.parametrize("name", sorted(SPECS))
+def test_ray_counts(dev, orc, name):
+    spec = SPECS[name]()
+    g, o = spec.gpu(dev), spec.oracle(orc)
+    rays = scenes.random_rays(21, 8200, radius=6.0, spread=3.0)
+    want = o.trace(rays)[0]
+    for n in (1, 15, 16, 17, 63, 64, 65, 255, 256, 257, 4095, 4097, 8200):
+        print(f"trace waves {name} n={n}", flush=True)
+        _same(g.trace(rays[:n]), want[:n])
+        hit = g.trace(rays[:n], any_hit=True)
+        assert np.array_equal(hit["prim_id"] >= 0, want[:n]["prim_id"] >= 0)
+
+
+@pytest.mark.parametrize("name", ["plain", "xf"])
+def test_directions(dev, orc, name):
+    """all signs of a direction, and components that are 0 or -0"""
+    print(f"trace waves directions {name}", flush=True)
+    spec = SPECS[name]()
+    g, o = spec.gpu(dev), spec.oracle(orc)
+    c = np.array([-1.0, -0.0, 0.0, 1.0, 0.3, -0.7], np.float32)
+    d = np.array([(x, y, z) for x in c for y in c for z in c if x or y or z], np.float32)
+    rays = scenes.random_rays(22, len(d) * 20, radius=6.0, spread=3.0).reshape(len(d), 20, 8)
+    rays[:, :, 4:7] = d[:, None, :]
+    rays[:, :, 0:3] = np.float32(0.2) * rays[:, :, 0:3] - np.float32(4.0) * d[:, None, :]
+    rays = np.ascontiguousarray(rays.reshape(-1, 8))
+    want = o.trace(rays)[0]
+    assert (want["prim_id"] >= 0).any()
+    _same(g.trace(rays), want)
+
+
+def test_rays_not_finite(dev):
+    print("trace waves not finite", flush=True)
+    g = helpers.soup_spec().gpu(dev)
+    rays = scenes.random_rays(23, 300, radius=5.0, spread=2.0)
+    for k, bad in enumerate((np.nan, np.inf, -np.inf)):
+        rays[k::3, 0:3] = bad
+    assert (g.trace(rays)["prim_id"] == -1).all()
+    assert (g.trace(rays, any_hit=True)["prim_id"] == -1).all()
+
+
+def test_threads(dev, orc):
+    print("trace waves threads", flush=True)
+    spec = helpers.soup_spec()
+    g, o = spec.gpu(dev), spec.oracle(orc)
+    sets = [scenes.random_rays(30 + k, 30000 + 777 * k, radius=5.0, spread=2.0) for k in range(4)]
+    want = [o.trace(r)[0] for r in sets]
+    got = [[] for _ in sets]
+
+    def work(k):
+        for _ in range(4):
+            got[k].append(g.trace(sets[k]))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(sets))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k, w in enumerate(want):
+        assert len(got[k]) == 4
+        for h in got[k]:
+            _same(h, w)
