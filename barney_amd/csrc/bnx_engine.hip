@@ -468,6 +468,7 @@ int render_frame_impl(World *w, const bnx_camera &cam, const bnx_renderer &rr, F
   for (int s0 = 0; s0 < spp; s0 += S) {
     const int nS = std::min(S, spp - s0);
     hs->accum_base = f->accum_id;
+    hs->samples = nS;
     hc[0] = RaygenChunk{0, 0, 0, 0};
     BNX_HIP(hipMemcpyAsync(F.slots.ptr, hs, sizeof(SlotDev), hipMemcpyHostToDevice, dev->stream));
     BNX_HIP(hipMemcpyAsync(F.chunks.ptr, hc, sizeof(RaygenChunk), hipMemcpyHostToDevice, dev->stream));
@@ -1017,6 +1018,7 @@ struct Server {
         return rc;
       }
       hs->accum_base = 0;
+      hs->samples = r->spp;
       BNX_HIP(hipMemcpyAsync(F.slots.as<SlotDev>() + r->slot, hs, sizeof(SlotDev), hipMemcpyHostToDevice,
                              dev->stream));
       r->surfaces = hs->scene.num_insts > 0;

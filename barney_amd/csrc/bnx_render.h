@@ -58,7 +58,7 @@ struct SlotDev {
   bnx_camera cam;
   int W, H;
   int accum_base;              // accumID of batch sample 0
-  int pad;
+  int samples;                 // the batch's samples per pixel
   FrameDev fb;
   EnvDev env;                  // HDRI light (env.tex null: ambient radiance)
 };
@@ -116,7 +116,8 @@ struct SlotOut {
 
 // A run of primary rays of one request: queue entries [begin, next chunk's
 // begin) hold the request's path indices first, first + 1, ... where path
-// index = sample * W * H + pixel and sample counts from the slot's accum_base.
+// index = pixel * samples + sample (pixels in tile order) and sample counts
+// from the slot's accum_base.
 struct RaygenChunk {
   long long begin;             // first queue index
   long long first;             // first path index

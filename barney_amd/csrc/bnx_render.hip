@@ -41,10 +41,11 @@ constexpr float ONE_OVER_TWO_PI = 1.f / TWO_PI;
 constexpr float ONE_OVER_FOUR_PI = 1.f / FOUR_PI;
 
 // ---------------------------------------------------------------- raygen
-// One thread per (request, sample, pixel) of the batch.  The chunk table
+// One thread per (request, pixel, sample) of the batch, a pixel's samples next
+// to each other.  The chunk table
 // lists each request's first queue index in ascending order; a thread finds
 // its request by binary search over it.
-// pixel of the pix-th path of a sample: row-major when tw == 0; otherwise
+// the pix-th pixel of the paths' order: row-major when tw == 0; otherwise
 // bands of th rows, each cut into tiles tw pixels wide (the last band and
 // tile of a row may be narrower), a tile's pixels row-major.  A bijection on
 // [0, W H): only the order of the primary rays in the queue changes, never a
@@ -87,9 +88,8 @@ __global__ void k_raygen(const RaygenChunk *chunks, int num_chunks, const SlotDe
   const bnx_camera &cam = SL.cam;
   const bnx_renderer &rr = SL.rr;
   const int W = SL.W, H = SL.H;
-  const int np = W * H;
   const long long path = ch.first + (idx - ch.begin);
-  const int s = (int)(path / np), pix = (int)(path - (long long)s * np);
+  const int pix = (int)(path / SL.samples), s = (int)(path - (long long)pix * SL.samples);
   const int accum_base = SL.accum_base;
   int ix, iy;
   tile_pixel(pix, W, H, tile_w, tile_h, ix, iy);
@@ -469,7 +469,41 @@ BNX_D float4 miss_color(const SlotDev &P, int pixel)
 }
 
 BNX_D int64_t to_fixed(float f) { return (int64_t)(f * 0x1p32f); }
-BNX_D void acc_add(unsigned long long *p, float f) { atomicAdd(p, (unsigned long long)to_fixed(f)); }
+
+// What a wave's lanes add to the frame, summed in LDS over runs of lanes that
+// shade rays of one pixel, so that a run takes one atomic on each of the
+// pixel's values instead of one a lane (an atomic is served beyond the XCD's
+// cache, those on one address one after the other).  The samples of a pixel
+// follow each other in the queue for it: shading 256^3 volume, 1024x1024, 16
+// spp, took 929 us sample by sample with an atomic a lane, 2064 pixel by
+// pixel, and takes 708 with the runs summed; tracing 37.5M primitives gains
+// 5% from the order and marching that volume 7%.  The sums are integers:
+// their order does not matter.
+struct PixelSums {
+  unsigned long long add[4][64];
+  int near_z[64];
+};
+BNX_D void accumulate(const FrameDev &fb, int pix, const uint64_t add[4], int near_z, PixelSums &L)
+{
+  const int lane = lane_id();
+  for (int c = 0; c < 4; c++) L.add[c][lane] = 0;
+  L.near_z[lane] = f2o(BNX_INF);
+  const int before = __shfl_up(pix, 1, 64);       // by every lane: an inactive one would be read as 0
+  const bool head = lane == 0 || before != pix;
+  const uint64_t heads = __ballot(head);
+  const int run = __popcll(heads & (lanemask_lt() | (1ull << lane))) - 1;
+  for (int c = 0; c < 4; c++)
+    if (add[c] != 0) atomicAdd(&L.add[c][run], (unsigned long long)add[c]);
+  if (near_z != f2o(BNX_INF)) atomicMin(&L.near_z[run], near_z);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  if (head && pix >= 0) {
+    unsigned long long *acc = (unsigned long long *)fb.accum + 4 * (size_t)pix;
+    for (int c = 0; c < 4; c++)
+      if (L.add[c][run] != 0) atomicAdd(acc + c, L.add[c][run]);
+    if (L.near_z[run] != f2o(BNX_INF)) atomicMin((int *)fb.depth + pix, L.near_z[run]);
+  }
+}
 
 struct OutRay {
   float4 org, dir;
@@ -499,6 +533,7 @@ __global__ __launch_bounds__(SHADE_BLOCK) void k_shade(const SlotDev *__restrict
   __shared__ int wave_base[SHADE_BLOCK / 64];
   __shared__ int wave_paths[SHADE_BLOCK / 64];
   __shared__ int block_base;
+  __shared__ PixelSums pixel_sums[SHADE_BLOCK / 64];
   int i;
   bool valid;
   const Segment sg = segment_of<SHADE_BLOCK>(sv, i, valid);
@@ -506,6 +541,10 @@ __global__ __launch_bounds__(SHADE_BLOCK) void k_shade(const SlotDev *__restrict
   const SlotDev &P = slots[slot_id];
   bool w_sh = false, w_ray = false;
   OutRay o_sh, o_ray;
+  // what the ray adds to its pixel (-1: nothing, past the segment's end)
+  int pix = -1;
+  uint64_t add[4] = {0, 0, 0, 0};
+  int near_z = f2o(BNX_INF);
   if (valid) {
     float4 ro = in.org[i], rd = in.dir[i];
     uint64_t rng = in.rng[i];
@@ -680,7 +719,7 @@ __global__ __launch_bounds__(SHADE_BLOCK) void k_shade(const SlotDev *__restrict
     // ------------------------------------------------ accumulate (shadeRays.cu:993-1040)
     const float clampMax = 10.f * (float)(1 + accumID);
     frag = vmin(frag, splat(clampMax));
-    unsigned long long *acc = fb.accum + 4 * (size_t)pixel;
+    pix = pixel;
     if (gen == 0) {
       if (accumID == 0 && !(flags & FLAG_IDS)) {
         fb.prim[pixel] = hit.x >= 0 ? hit.x : -1;
@@ -703,13 +742,14 @@ __global__ __launch_bounds__(SHADE_BLOCK) void k_shade(const SlotDev *__restrict
         fb.obj[pixel] = obj;
       }
       if (accumID == 0) fb.normal[pixel] = make_float4(inN.x, inN.y, inN.z, 0.f);
-      atomicMin(fb.depth + pixel, f2o(inZ));
-      if (alpha > 0.f) acc_add(acc + 3, alpha);
+      near_z = f2o(inZ);
+      if (alpha > 0.f) add[3] = to_fixed(alpha);
     }
-    if (frag.x > 0.f) acc_add(acc + 0, frag.x);
-    if (frag.y > 0.f) acc_add(acc + 1, frag.y);
-    if (frag.z > 0.f) acc_add(acc + 2, frag.z);
+    if (frag.x > 0.f) add[0] = to_fixed(frag.x);
+    if (frag.y > 0.f) add[1] = to_fixed(frag.y);
+    if (frag.z > 0.f) add[2] = to_fixed(frag.z);
   }
+  accumulate(P.fb, pix, add, near_z, pixel_sums[threadIdx.x >> 6]);
   // ------------------------------------------------ compacted append
   // wave ballot + popcount gives each lane its offset inside the wave, the
   // wave totals are scanned in LDS, and one atomic per block reserves the
@@ -733,8 +773,11 @@ __global__ __launch_bounds__(SHADE_BLOCK) void k_shade(const SlotDev *__restrict
       acc += c;
       paths += wave_paths[w];
     }
-    block_base = so.base[slot_id] + (acc > 0 ? atomicAdd(so.cnt + 2 * slot_id, acc) : 0);
-    if (paths > 0) atomicAdd(so.cnt + 2 * slot_id + 1, paths);
+    // both counters in one atomic: the rays in the low word, the paths among
+    // them in the high one (neither reaches 2^31)
+    const unsigned long long both = (uint32_t)acc | ((unsigned long long)(uint32_t)paths << 32);
+    block_base = so.base[slot_id] +
+                 (acc > 0 ? (int)(uint32_t)atomicAdd((unsigned long long *)(so.cnt + 2 * slot_id), both) : 0);
   }
   __syncthreads();
   int o = block_base + wave_base[wid] + pre;

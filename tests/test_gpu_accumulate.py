@@ -1,0 +1,42 @@
+"""The frame accumulation where it can go wrong: a pixel's samples lie next to
+each other in the ray queue and a wave adds them up in runs before it touches
+the frame, so one render of N samples per pixel is compared, channel by
+channel and bit for bit, with N renders of one sample (whose waves hold runs
+of other lengths, and whose sums are the same integers), for runs shorter
+than, equal to and longer than a wave, pixel 0 included, and for whole frames
+below a wave."""
+import numpy as np
+import pytest
+
+import barney_amd as bx
+from barney_amd import abi, scenes
+
+pytestmark = pytest.mark.gpu
+
+CHANNELS = (abi.BNX_FB_COLOR, abi.BNX_FB_DEPTH, abi.BNX_FB_PRIMID, abi.BNX_FB_INSTID, abi.BNX_FB_OBJID,
+            abi.BNX_FB_NORMAL)
+
+
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (1, 1, 200), (3, 2, 63), (7, 5, 64), (5, 7, 65), (33, 17, 3),
+                                     (64, 1, 2), (97, 61, 5)])
+@pytest.mark.parametrize("kind", ["surface", "volume"])
+def test_samples_together_equal_samples_apart(dev, kind, w, h, spp):
+    print(f"accumulate {kind} {w}x{h} spp={spp}", flush=True)
+    if kind == "surface":
+        sc = scenes.config1(width=w, height=h)
+        world = bx.SurfaceWorld(dev, sc)
+    else:
+        sc = scenes.config2(n=17, mc_grid=4, width=w, height=h)
+        world = bx.VolumeWorld(dev, sc)
+    c = sc.camera
+    cam = bx.camera_perspective(c["position"], c["direction"], c["up"], c["fovy"])
+    rend = abi.renderer(bg=sc.bg_color, ambient=sc.ambient)
+    together, apart = bx.Frame(dev, w, h), bx.Frame(dev, w, h)
+    bx.render(world.world, cam, rend, together, spp)
+    for _ in range(spp):
+        bx.render(world.world, cam, rend, apart, 1)
+    for ch in CHANNELS:
+        a, b = together.read(ch), apart.read(ch)
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), ch
+    together.close()
+    apart.close()
