@@ -74,7 +74,7 @@ struct BatchShape {
   long long count0 = 0, cap = 0;
   bool surfaces = false, volumes = false;
   MarchKind march;
-  int refill = 64, stack = 16, walk = 0, blocks_per_cu = 8, shade_block = 1024;
+  int refill = 64, stack = 16, walk = 0, blocks_per_cu = 8, shade_block = 256;
   bool ext = false;   // the trace kernels with the cylinder test and the cut plane
   bool xf = false;    // the trace kernels that change the ray's frame at instances
   bool operator<(const BatchShape &o) const

@@ -104,7 +104,7 @@ struct Device {
   int trace_stack_lds = 16;  // LDS stack entries per lane in the queue-trace kernels (8, 16, 32)
   int trace_walk = 0;        // 0 waves that take new rays as walks end, 1 one ray per thread, speculative while-while
   int sort_rays = 0;         // bnx_render: reorder secondary generations by direction and origin
-  int shade_block = 1024;    // threads per shade block (256 or 1024)
+  int shade_block = 256;     // threads per shade block (256 or 1024)
   int trace_refill = 16;    // secondary rays of large scenes: idle lanes that make a trace wave take new rays
   long long trace_refill_prims = 1 << 20;   // "large": at least this many primitives
   int trace_blocks_per_cu = 8;   // at most this many times four trace waves per CU

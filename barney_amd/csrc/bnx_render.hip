@@ -523,12 +523,18 @@ BNX_D void pack_ps(uint4 &ps, v3 tp, int ndiff, int gen, int pixel, float mis)
 // different requests at different depths of their paths.  Each block lies
 // inside one request's segment: the request's parameters are block-uniform
 // (scalar registers) and the block appends to that request's output region.
-// SHADE_BLOCK is 1024 or 256 threads (a tuning field): a block of 1024 takes
-// one atomic per 1024 rays on its request's counter but fits one block per
-// CU at this kernel's register count; 256 fits more waves per SIMD.
+// SHADE_BLOCK is 256 or 1024 threads (a tuning field): a block of 1024 takes
+// one atomic per 1024 rays on its request's counter, but only one fits a CU,
+// which idles while its last waves reach the append.  Bound by its gathers
+// (instance, geometry, indices, vertices, attributes, one after the other)
+// and the queue's 76 bytes in and up to 112 out a ray; six waves per SIMD (40
+// bytes of scratch a ray; at eight, 132, the traffic to scratch takes the
+// gain back: 8.4 ms).  1920x1080, 8 spp, 37.5M primitives: 5.2 ms in blocks
+// of 256, 7.5 in blocks of 1024; 1024x1024, 16 spp, 256^3 volume: 593 us and
+// 708; 512x512, 1 spp, 1.05M triangles: 57 us and 50.
 template <int SHADE_BLOCK>
-__global__ __launch_bounds__(SHADE_BLOCK) void k_shade(const SlotDev *__restrict__ slots, SegView sv, RayQueue in,
-                                                       RayQueue out, SlotOut so, unsigned long long *stats)
+__global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(SHADE_BLOCK == 256 ? 6 : 4))) void k_shade(
+    const SlotDev *__restrict__ slots, SegView sv, RayQueue in, RayQueue out, SlotOut so, unsigned long long *stats)
 {
   __shared__ int wave_base[SHADE_BLOCK / 64];
   __shared__ int wave_paths[SHADE_BLOCK / 64];

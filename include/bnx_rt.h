@@ -444,7 +444,7 @@ typedef struct bnx_tuning {
                                        of one per generation (0: never; <= 2^26)    */
 } bnx_tuning;
 /* a new device starts with 8 x 8 tiles, 16 LDS entries, walk 0, no reordering,
- * 1024-thread shade blocks, 8 blocks per CU,
+ * 256-thread shade blocks, 8 blocks per CU,
  * refill 16 for worlds of 2^20 primitives or more, 2^23 paths per batch and
  * captured bounce loops for batches of up to 2^22 paths */
 

@@ -4,7 +4,8 @@ the frame, so one render of N samples per pixel is compared, channel by
 channel and bit for bit, with N renders of one sample (whose waves hold runs
 of other lengths, and whose sums are the same integers), for runs shorter
 than, equal to and longer than a wave, pixel 0 included, and for whole frames
-below a wave."""
+below a wave.  The renders of one sample run with shade blocks of 1024
+threads, the others with the 256 of a new device."""
 import numpy as np
 import pytest
 
@@ -33,8 +34,14 @@ def test_samples_together_equal_samples_apart(dev, kind, w, h, spp):
     rend = abi.renderer(bg=sc.bg_color, ambient=sc.ambient)
     together, apart = bx.Frame(dev, w, h), bx.Frame(dev, w, h)
     bx.render(world.world, cam, rend, together, spp)
-    for _ in range(spp):
-        bx.render(world.world, cam, rend, apart, 1)
+    tuning = dev.tuning()
+    assert tuning["shade_block"] == 256
+    try:
+        dev.set_tuning(shade_block=1024)
+        for _ in range(spp):
+            bx.render(world.world, cam, rend, apart, 1)
+    finally:
+        dev.set_tuning(**tuning)
     for ch in CHANNELS:
         a, b = together.read(ch), apart.read(ch)
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), ch
