@@ -245,6 +245,19 @@ int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool sur
   return launch_shade(dev, slots, sv, sl.blocks256, sl.blocks1024, in, out, so, st);
 }
 
+// Where a generation's launches write the wall clock: t[0], t[1] bracket the
+// trace and t[2], t[3] the march.  The set-up launch before them writes the
+// first, each launch after them the ones that the launch before it ends.
+struct GenStamps {
+  Stamp first, march, shade;
+  GenStamps(unsigned long long *t, bool trace, bool volumes)
+  {
+    first = Stamp{trace ? t : t + 2, 1};
+    march = trace ? Stamp{t + 1, 2} : Stamp{};
+    shade = Stamp{volumes ? t + 3 : t + 1, 1};
+  }
+};
+
 // Enqueue G device-driven generations of one request's batch (slot 0, the
 // primary rays in queue cur0, count0 of them): each generation's segment
 // and counter reset come from k_gen_setup, and every launch is sized for
@@ -267,24 +280,17 @@ int enqueue_dd(Device *dev, Wavefront &F, int cur0, int G, const BatchShape &b)
     const int refill = g == 0 ? 64 : b.refill;
     const long long c = g == 0 ? b.count0 : b.cap;
     const int blocks256 = (int)((c + 255) / 256), blocks1024 = (int)((c + 1023) / 1024);
-    if ((rc = launch_gen_setup(dev, F.segs.as<Segment>(), F.out_cnt.as<int>(), F.gen_counts.as<long long>(), g,
-                               (int)b.count0, refill)) != BNX_OK)
+    const GenStamps at(F.stamps.as<unsigned long long>() + 4 * g, trace, b.volumes);
+    if ((rc = launch_gen_setup(dev, sv, blocks256, blocks1024, F.out_cnt.as<int>(), F.gen_counts.as<long long>(), g,
+                               (int)b.count0, refill, at.first)) != BNX_OK)
       return rc;
-    if ((rc = launch_segment_blocks(dev, sv, 1, blocks256, blocks1024)) != BNX_OK) return rc;
     RayQueue in = Q.q(cur), out = Q.q(1 - cur);
     TraceQueue tq{in.org, in.dir, in.hit, in.hit_v, in.rng, in.ps};
-    unsigned long long *ts = F.stamps.as<unsigned long long>() + 4 * g;
-    if (trace) {
-      if ((rc = launch_stamp(dev, ts)) != BNX_OK) return rc;
-      if ((rc = launch_trace_queue(dev, slots, sv, 1, blocks256, b.ext, tq, st)) != BNX_OK) return rc;
-      if ((rc = launch_stamp(dev, ts + 1)) != BNX_OK) return rc;
-    }
-    if (b.volumes) {
-      if ((rc = launch_stamp(dev, ts + 2)) != BNX_OK) return rc;
-      if ((rc = launch_volume_march(dev, slots, sv, 1, blocks256, in, trace, b.march, st)) != BNX_OK) return rc;
-      if ((rc = launch_stamp(dev, ts + 3)) != BNX_OK) return rc;
-    }
-    if ((rc = launch_shade(dev, slots, sv, blocks256, blocks1024, in, out, so, st)) != BNX_OK) return rc;
+    if (trace && (rc = launch_trace_queue(dev, slots, sv, 1, blocks256, b.ext, tq, st)) != BNX_OK) return rc;
+    if (b.volumes &&
+        (rc = launch_volume_march(dev, slots, sv, 1, blocks256, in, trace, b.march, st, at.march)) != BNX_OK)
+      return rc;
+    if ((rc = launch_shade(dev, slots, sv, blocks256, blocks1024, in, out, so, st, at.shade)) != BNX_OK) return rc;
   }
   return BNX_OK;
 }
@@ -1242,21 +1248,15 @@ struct Server {
       if (added_max > 0 && O > 0 &&
           (rc = launch_raygen_dev(dev, p.chunks, O, slots, p.scal + 1, added_max, in)) != BNX_OK)
         return rc;
-      if ((rc = launch_segment_blocks(dev, sv, nsegs, blocks256, blocks1024)) != BNX_OK) return rc;
+      const GenStamps at(F.stamps.as<unsigned long long>() + 4 * g, trace, volumes);
+      if ((rc = launch_segment_blocks(dev, sv, nsegs, blocks256, blocks1024, at.first)) != BNX_OK) return rc;
       TraceQueue tq{in.org, in.dir, in.hit, in.hit_v, in.rng, in.ps};
-      unsigned long long *tsp = F.stamps.as<unsigned long long>() + 4 * g;
-      if (trace) {
-        if ((rc = launch_stamp(dev, tsp)) != BNX_OK) return rc;
-        if ((rc = launch_trace_queue(dev, slots, sv, nsegs, blocks256, cut, tq, stat)) != BNX_OK)
-          return rc;
-        if ((rc = launch_stamp(dev, tsp + 1)) != BNX_OK) return rc;
-      }
-      if (volumes) {
-        if ((rc = launch_stamp(dev, tsp + 2)) != BNX_OK) return rc;
-        if ((rc = launch_volume_march(dev, slots, sv, nsegs, blocks256, in, trace, march, stat)) != BNX_OK) return rc;
-        if ((rc = launch_stamp(dev, tsp + 3)) != BNX_OK) return rc;
-      }
-      if ((rc = launch_shade(dev, slots, sv, blocks256, blocks1024, in, out, so, stat)) != BNX_OK) return rc;
+      if (trace && (rc = launch_trace_queue(dev, slots, sv, nsegs, blocks256, cut, tq, stat)) != BNX_OK) return rc;
+      if (volumes &&
+          (rc = launch_volume_march(dev, slots, sv, nsegs, blocks256, in, trace, march, stat, at.march)) != BNX_OK)
+        return rc;
+      if ((rc = launch_shade(dev, slots, sv, blocks256, blocks1024, in, out, so, stat, at.shade)) != BNX_OK)
+        return rc;
       cur = 1 - cur;
     }
     k_srv_setup<<<1, SRV_TB, 0, st>>>(p, G, 1);

@@ -925,8 +925,9 @@ constexpr int iso_waves(int field) { return field == FIELD_KIND_CELLS ? 3 : 5; }
 template <int FIELD>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves(FIELD)))) void k_volume_march(
     const SlotDev *__restrict__ slots, SegView sv, RayQueue q, int k, int nsegs, int program, int fresh,
-    unsigned long long *stats)
+    unsigned long long *stats, Stamp stamp)
 {
+  if (blockIdx.x == 0 && threadIdx.x == 0) stamp_write(stamp);
   __shared__ uint32_t ready[READY * 64];
   __shared__ uint32_t ring[FIELD == FIELD_KIND_CELLS ? PQ_SHORT * 64 : 1];
   Claims cl;
@@ -939,8 +940,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves(
 template <int FIELD>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(iso_waves(FIELD)))) void k_iso_march(
     const SlotDev *__restrict__ slots, SegView sv, RayQueue q, int k, int nsegs, int program, int fresh,
-    unsigned long long *stats)
+    unsigned long long *stats, Stamp stamp)
 {
+  if (blockIdx.x == 0 && threadIdx.x == 0) stamp_write(stamp);
   __shared__ IsoShared L;
   __shared__ uint32_t ring[FIELD == FIELD_KIND_CELLS ? PQ_SHORT * 64 : 1];
   Claims cl;
@@ -950,7 +952,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(iso_waves(FI
   });
 }
 
-using MarchKernel = void (*)(const SlotDev *, SegView, RayQueue, int, int, int, int, unsigned long long *);
+using MarchKernel = void (*)(const SlotDev *, SegView, RayQueue, int, int, int, int, unsigned long long *, Stamp);
 const MarchKernel KERNELS[2][FIELD_KINDS] = {
     {k_volume_march<FIELD_KIND_STRUCTURED>, k_volume_march<FIELD_KIND_TETS>, k_volume_march<FIELD_KIND_CELLS>},
     {k_iso_march<FIELD_KIND_STRUCTURED>, k_iso_march<FIELD_KIND_TETS>, k_iso_march<FIELD_KIND_CELLS>}};
@@ -958,7 +960,8 @@ const MarchKernel KERNELS[2][FIELD_KINDS] = {
 } // namespace
 
 int launch_volume_march(Device *dev, const SlotDev *slots, const SegView &sv, int nsegs, int blocks256,
-                        const RayQueue &q, bool surfaces, const MarchKind &kind, unsigned long long *stats)
+                        const RayQueue &q, bool surfaces, const MarchKind &kind, unsigned long long *stats,
+                        const Stamp &stamp)
 {
   if (blocks256 <= 0 || nsegs <= 0) return BNX_OK;
   int launch = 0;
@@ -983,7 +986,7 @@ int launch_volume_march(Device *dev, const SlotDev *slots, const SegView &sv, in
         if (rc != BNX_OK) return rc;
       }
       kernel<<<std::max(CLAIM_GROUPS, waves), 64, 0, dev->stream>>>(slots, sv, q, k, nsegs, slot, surfaces ? 0 : 1,
-                                                                    stats);
+                                                                    stats, launch == 0 ? stamp : Stamp{});
       launch++;
     }
   }

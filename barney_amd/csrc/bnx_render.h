@@ -183,13 +183,19 @@ int launch_raygen(Device *dev, const RaygenChunk *d_chunks, int num_chunks, cons
 // launch
 int launch_raygen_dev(Device *dev, const RaygenChunk *d_chunks, int num_chunks, const SlotDev *d_slots,
                       const long long *d_range, long long max_total, const RayQueue &q);
+// Launch timing where events are not available (captured loops, steps without
+// read-back): a launch writes the device wall clock (ticks of wall_clock_khz)
+// to the n words at t as it begins, that is when the launches before it have
+// ended
+struct Stamp {
+  unsigned long long *t = nullptr;
+  int n = 0;
+};
 // a device-driven generation's single segment from the previous shade's
-// output counter (count0 when g == 0); clears the counter, keeps the count
-// in gen_counts[g]
-int launch_gen_setup(Device *dev, Segment *segs, int *out_cnt, long long *gen_counts, int g, int count0, int refill);
-// write the device wall clock (ticks of wall_clock_khz) to *t once the
-// stream reaches this point
-int launch_stamp(Device *dev, unsigned long long *t);
+// output counter (count0 when g == 0), with its block maps and claim
+// counters; clears the counter, keeps the count in gen_counts[g]
+int launch_gen_setup(Device *dev, const SegView &sv, int blocks256, int blocks1024, int *out_cnt,
+                     long long *gen_counts, int g, int count0, int refill, const Stamp &stamp);
 
 // scratch of the ray reordering (keys, indices, radix-sort temporaries)
 struct SortScratch {
@@ -201,14 +207,15 @@ int sort_rays(Device *dev, SortScratch &S, const RayQueue &src, const RayQueue &
               const float hi[3]);
 // fill the block -> segment maps of nsegs segments (blocks256 / blocks1024
 // blocks in all) and clear the claim counters
-int launch_segment_blocks(Device *dev, const SegView &sv, int nsegs, int blocks256, int blocks1024);
+int launch_segment_blocks(Device *dev, const SegView &sv, int nsegs, int blocks256, int blocks1024,
+                          const Stamp &stamp = {});
 // the claim counters of one more launch
 int launch_claims_clear(Device *dev, int *counters);
 // shade every ray of the segments (blocks256 blocks of 256 threads or
 // blocks1024 of 1024, by the device's shade_block),
 // appending each request's shadow and continuation rays to its region of out
 int launch_shade(Device *dev, const SlotDev *d_slots, const SegView &sv, int blocks256, int blocks1024, const RayQueue &in,
-                 const RayQueue &out, const SlotOut &so, unsigned long long *stats);
+                 const RayQueue &out, const SlotOut &so, unsigned long long *stats, const Stamp &stamp = {});
 int trace_stack_capacity();
 
 // the per-request frame loop behind bnx_render
@@ -219,6 +226,13 @@ void wavefront_destroy(Device *dev);
 
 // The segment of this block of a B-thread launch, and the ray this thread
 // takes (i, valid).  Every thread of a block gets the same segment.
+BNX_D void stamp_write(const Stamp &s)
+{
+  if (s.n == 0) return;
+  const unsigned long long now = wall_clock64();
+  for (int k = 0; k < s.n; k++) s.t[k] = now;
+}
+
 template <int B> BNX_D Segment segment_of(const SegView &sv, int &i, bool &valid)
 {
   const int k = (B == 256 ? sv.blk256 : sv.blk1024)[blockIdx.x];

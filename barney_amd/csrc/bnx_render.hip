@@ -534,8 +534,10 @@ BNX_D void pack_ps(uint4 &ps, v3 tp, int ndiff, int gen, int pixel, float mis)
 // 708; 512x512, 1 spp, 1.05M triangles: 57 us and 50.
 template <int SHADE_BLOCK>
 __global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(SHADE_BLOCK == 256 ? 6 : 4))) void k_shade(
-    const SlotDev *__restrict__ slots, SegView sv, RayQueue in, RayQueue out, SlotOut so, unsigned long long *stats)
+    const SlotDev *__restrict__ slots, SegView sv, RayQueue in, RayQueue out, SlotOut so, unsigned long long *stats,
+    Stamp stamp)
 {
+  if (blockIdx.x == 0 && threadIdx.x == 0) stamp_write(stamp);
   __shared__ int wave_base[SHADE_BLOCK / 64];
   __shared__ int wave_paths[SHADE_BLOCK / 64];
   __shared__ int block_base;
@@ -804,9 +806,10 @@ __global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(SHA
 }
 
 // block -> segment maps: one thread per block of either launch width
-__global__ void k_segment_blocks(SegView sv, int nsegs, int blocks256, int blocks1024)
+__global__ void k_segment_blocks(SegView sv, int nsegs, int blocks256, int blocks1024, Stamp stamp)
 {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b == 0) stamp_write(stamp);
   if (blockIdx.x == 0)
     for (int i = threadIdx.x; i < CLAIMS_LAUNCHES * CLAIM_GROUPS; i += blockDim.x) sv.claims[i * CLAIM_STRIDE] = 0;
   const Segment *segs = sv.segs;
@@ -833,23 +836,26 @@ __global__ void k_segment_blocks(SegView sv, int nsegs, int blocks256, int block
 // One generation's set-up for a device-driven bounce loop (one request,
 // one segment, no read-back between generations): the segment takes its
 // count from the previous shade's output counter (count0 for the primary
-// generation), the counter is cleared for this generation's shade, and the
-// count is kept in gen_counts[g] for the host.
-__global__ void k_gen_setup(Segment *segs, int *out_cnt, long long *gen_counts, int g, int count0, int refill)
+// generation), the counter is cleared for this generation's shade, the
+// count is kept in gen_counts[g] for the host, and every block belongs to
+// the one segment.  With the block maps and the stamps in launches of their
+// own a generation of a small frame spent 23 us in four launches of one
+// thread's work (96x96, 1 spp: three generations, 57 of 303 us).
+__global__ void k_gen_setup(SegView sv, int blocks256, int blocks1024, int *out_cnt, long long *gen_counts, int g,
+                            int count0, int refill, Stamp stamp)
 {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b < blocks256) ((int *)sv.blk256)[b] = 0;
+  if (b < blocks1024) ((int *)sv.blk1024)[b] = 0;
+  if (blockIdx.x != 0) return;
+  for (int i = threadIdx.x; i < CLAIMS_LAUNCHES * CLAIM_GROUPS; i += blockDim.x) sv.claims[i * CLAIM_STRIDE] = 0;
   if (threadIdx.x != 0) return;
   const int count = g == 0 ? count0 : out_cnt[0];
-  segs[0] = Segment{0, 0, count, 0, 0, refill, {}};
+  ((Segment *)sv.segs)[0] = Segment{0, 0, count, 0, 0, refill, {}};
   out_cnt[0] = 0;
   out_cnt[1] = 0;
   gen_counts[g] = count;
-}
-
-// the device's constant-rate wall clock, for timing launches inside a
-// captured graph (where event timestamps are not available)
-__global__ void k_stamp(unsigned long long *t)
-{
-  if (threadIdx.x == 0) *t = wall_clock64();
+  stamp_write(stamp);
 }
 
 // ----------------------------------------------------------- frame ops
@@ -1064,35 +1070,32 @@ int launch_raygen_dev(Device *dev, const RaygenChunk *chunks, int num_chunks, co
 }
 
 int launch_shade(Device *dev, const SlotDev *slots, const SegView &sv, int blocks256, int blocks1024,
-                 const RayQueue &in, const RayQueue &out, const SlotOut &so, unsigned long long *stats)
+                 const RayQueue &in, const RayQueue &out, const SlotOut &so, unsigned long long *stats,
+                 const Stamp &stamp)
 {
   if (dev->shade_block == 256) {
-    if (blocks256 > 0) k_shade<256><<<blocks256, 256, 0, dev->stream>>>(slots, sv, in, out, so, stats);
+    if (blocks256 > 0) k_shade<256><<<blocks256, 256, 0, dev->stream>>>(slots, sv, in, out, so, stats, stamp);
   } else if (blocks1024 > 0) {
-    k_shade<1024><<<blocks1024, 1024, 0, dev->stream>>>(slots, sv, in, out, so, stats);
+    k_shade<1024><<<blocks1024, 1024, 0, dev->stream>>>(slots, sv, in, out, so, stats, stamp);
   }
   BNX_HIP(hipGetLastError());
   return BNX_OK;
 }
 
-int launch_gen_setup(Device *dev, Segment *segs, int *out_cnt, long long *gen_counts, int g, int count0, int refill)
+int launch_gen_setup(Device *dev, const SegView &sv, int blocks256, int blocks1024, int *out_cnt,
+                     long long *gen_counts, int g, int count0, int refill, const Stamp &stamp)
 {
-  k_gen_setup<<<1, 64, 0, dev->stream>>>(segs, out_cnt, gen_counts, g, count0, refill);
+  k_gen_setup<<<nblk(std::max(1, blocks256), 256), 256, 0, dev->stream>>>(sv, blocks256, blocks1024, out_cnt,
+                                                                          gen_counts, g, count0, refill, stamp);
   BNX_HIP(hipGetLastError());
   return BNX_OK;
 }
 
-int launch_stamp(Device *dev, unsigned long long *t)
-{
-  k_stamp<<<1, 64, 0, dev->stream>>>(t);
-  BNX_HIP(hipGetLastError());
-  return BNX_OK;
-}
-
-int launch_segment_blocks(Device *dev, const SegView &sv, int nsegs, int blocks256, int blocks1024)
+int launch_segment_blocks(Device *dev, const SegView &sv, int nsegs, int blocks256, int blocks1024,
+                          const Stamp &stamp)
 {
   if (nsegs > 0 && blocks256 > 0)
-    k_segment_blocks<<<nblk(blocks256, 256), 256, 0, dev->stream>>>(sv, nsegs, blocks256, blocks1024);
+    k_segment_blocks<<<nblk(blocks256, 256), 256, 0, dev->stream>>>(sv, nsegs, blocks256, blocks1024, stamp);
   BNX_HIP(hipGetLastError());
   return BNX_OK;
 }

@@ -157,7 +157,8 @@ struct MarchKind {
 // blocks of 256 rays) through its request's isosurfaces and volumes; surfaces: false when the
 // trace kernel did not run, so the hit records are not written yet
 int launch_volume_march(Device *dev, const SlotDev *d_slots, const SegView &sv, int nsegs, int blocks256,
-                        const RayQueue &q, bool surfaces, const MarchKind &kind, unsigned long long *stats);
+                        const RayQueue &q, bool surfaces, const MarchKind &kind, unsigned long long *stats,
+                        const Stamp &stamp = {});
 
 // ---------------------------------------------------------------- device
 
