@@ -531,7 +531,7 @@ BNX_D void pack_ps(uint4 &ps, v3 tp, int ndiff, int gen, int pixel, float mis)
 // bytes of scratch a ray; at eight, 132, the traffic to scratch takes the
 // gain back: 8.4 ms).  1920x1080, 8 spp, 37.5M primitives: 5.2 ms in blocks
 // of 256, 7.5 in blocks of 1024; 1024x1024, 16 spp, 256^3 volume: 593 us and
-// 708; 512x512, 1 spp, 1.05M triangles: 57 us and 50.
+// 708; 512x512, 1 spp, 20k triangles: 57 us and 50.
 template <int SHADE_BLOCK>
 __global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(SHADE_BLOCK == 256 ? 6 : 4))) void k_shade(
     const SlotDev *__restrict__ slots, SegView sv, RayQueue in, RayQueue out, SlotOut so, unsigned long long *stats,

@@ -654,12 +654,12 @@ BNX_D HitRec traverse_spec(const SceneDev &S, const float4 *rorg, const float4 *
 }
 
 // Into how many chunks a launch is cut at least.  Half as many as waves: full
-// waves before all waves (1.05M triangles, 512x512, 1 spp: 406 us in three
+// waves before all waves (20k triangles, 512x512, 1 spp: 406 us in three
 // launches, and 552 with a chunk for each; 60001 rays: 111 and 135).  The
 // extended kernels run a leaf step once for each kind of primitive in the
 // wave, and a wave with 64 long rays is one that the launch waits for: twice
-// as many as waves (instances of four kinds, 640x360: 3.3 ms, and 4.7 with
-// half as many).
+// as many as waves (27 instances each of cylinders, capsules and cones,
+// 641x363, 4 spp: 3.3 ms, and 4.7 with half as many).
 BNX_D int least_chunks(bool ext) { return ext ? 2 * (int)gridDim.x : (int)gridDim.x / 2; }
 
 // rays and hits of the ray-array entry point

@@ -126,8 +126,9 @@ def roofline(tot, workload=None, trace_kernel="k_trace_static<16, false, false>"
     from the oracle's counts (model: how they were counted); without it the
     GPU's own counters are priced at the same per-item sizes"""
     if tot.get("march_ms", 0.0) >= tot.get("trace_ms", 0.0) and tot.get("march_launches", 0) > 0:
-        # the full variant (MARCH_FULL = 1) runs for tet fields and
-        # isosurfaces, the lean one (0) otherwise
+        # the kernel of the field's kind: 1 for tets (with the isosurface's,
+        # k_iso_march<1>, in the same march time and profile line), 0 for
+        # structured fields
         full = tot.get("umesh_nodes", 0) > 0 or workload == "c4"
         kernel = "k_volume_march<1>" if full else "k_volume_march<0>"
         kms, launches = tot["march_ms"], tot["march_launches"]
