@@ -482,8 +482,8 @@ int build_tet_neighbors(Device *dev, const int4 *tets, int ntet, DevMem &nbr)
 // The value ranges: every cell adds the range of its vertices' scalars to the
 // grid cells that its box touches, grown by a twentieth of its extent and
 // 1e-5 of its coordinates (a test accepts points outside the cell by far
-// less, see k_cell_pack).  A cell with more than FINE_MOST grid cells adds to
-// the range that all grid cells share.  Values are means of the scalars with
+// less, see k_cell_pack).  A cell with more than FINE_MOST grid cells, and a
+// tet too flat for that, adds to the range that all grid cells share.  Values are means of the scalars with
 // weights above -1e-3 (a Newton inversion's last step), so the ranges take in
 // a thousandth of their width and 1e-5 of the scalars at either end.
 constexpr int FINE_MOST = 4096;
@@ -503,7 +503,19 @@ __global__ void k_fine_ranges(const int4 *tets, const int4 *ext, const uint8_t *
   const int ax = a % nx, ay = (a / nx) % ny, az = a / (nx * ny), bx = b % nx, by = (b / nx) % ny, bz = b / (nx * ny);
   const int vl = f2o(l.w - slack), vh = f2o(h.w + slack);
   const bool finite = slack < INFINITY;       // an infinite scalar: any value may come of it
-  if (!finite || (long long)(bx - ax + 1) * (by - ay + 1) * (bz - az + 1) > FINE_MOST) {
+  // A tet's planes, computed with an error e, accept the tet scaled by
+  // (r + e) / r about its incentre, r the radius of its inscribed sphere: with
+  // e below 1e-6 of the distance to it and r a thousandth of its size that is
+  // well inside the margin.  A flatter one may accept any point of its leaf.
+  bool flat = false;
+  if (!types || types[c] == CELL_TET) {
+    const v3 p0 = xyz(cell_vertex(tets, ext, verts, c, 0)), p1 = xyz(cell_vertex(tets, ext, verts, c, 1)),
+             p2 = xyz(cell_vertex(tets, ext, verts, c, 2)), p3 = xyz(cell_vertex(tets, ext, verts, c, 3));
+    const v3 e1 = p1 - p0, e2 = p2 - p0, e3 = p3 - p0;
+    const v3 n0 = cross(e2 - e1, e3 - e1), n1 = cross(e2, e3), n2 = cross(e3, e1), n3 = cross(e1, e2);
+    flat = !(fabsf(dot(e1, n1)) >= 1e-3f * size * (length(n0) + length(n1) + length(n2) + length(n3)));
+  }
+  if (!finite || flat || (long long)(bx - ax + 1) * (by - ay + 1) * (bz - az + 1) > FINE_MOST) {
     atomicMin(all, finite ? vl : f2o(-INFINITY));
     atomicMax(all + 1, finite ? vh : f2o(INFINITY));
     return;
