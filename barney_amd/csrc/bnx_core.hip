@@ -1170,9 +1170,11 @@ static int set_tf(Volume *v, const bnx_transfer_function *tf)
   v->dd.dom1 = tf->domain[1];
   v->dd.base_density = tf->base_density;
   v->dd.rcp_span = 1.f / (tf->domain[1] - tf->domain[0]);
-  // majorants are alphas of the map, or weighted means of two, times the
-  // density: with these bounds they and the quotients by them stay far from
-  // the ends of the float range
+  // Majorants are alphas of the map, or weighted means of two, times the
+  // density: these bounds keep them from the upper end of the float range.
+  // They do not keep them from the lower one, since the mean of an alpha of 0
+  // and the next may be as small as the scalars: the march looks at each
+  // cell's majorant itself (short_majorant)
   auto in = [](float x, float lo, float hi) { return x >= lo && x <= hi; };
   bool rn = in(tf->base_density, 0x1p-30f, 0x1p30f) && in(tf->domain[1] - tf->domain[0], 0x1p-60f, 0x1p60f);
   for (int i = 0; i < tf->num_values && rn; i++) {

@@ -69,14 +69,12 @@ BNX_D v3 ld3(const float *p) { return v3{p[0], p[1], p[2]}; }
 // b = 0 gives NaN where 1/b gives an infinity.
 BNX_D float rcp_rn(float b)
 {
-  const float y = __builtin_amdgcn_rcpf(b);
-  return __builtin_fmaf(__builtin_fmaf(-b, y, 1.f), y, y);
+  return bnx_num::rcp_step(b, __builtin_amdgcn_rcpf(b));
 }
 // a / b with y = rcp_rn(b)
 BNX_D float div_rn(float a, float b, float y)
 {
-  const float q = a * y;
-  return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+  return bnx_num::div_step(a, b, y);
 }
 BNX_D float sqrt_rn(float x)
 {

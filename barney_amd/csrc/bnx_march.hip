@@ -301,7 +301,7 @@ template <int FIELD> struct March {
     uint64_t rs = 0;
     float maj = 0.f, t = 0.f, upper = 0.f, T = 1.f;
     bool ratio = false;
-    float rmaj = 0.f;                   // rcp_rn(maj)
+    float rmaj = 0.f;                   // rcp_rn(maj), 0 where the draws divide by maj
     // point query: the tet being tested, the one that held the last point,
     // the walk's steps and whether it started from the seed; the value found
     int cur = 0, last = -1, walk = 0;
@@ -353,10 +353,10 @@ template <int FIELD> struct March {
     auto consume = [&]() {
       const float f = value;
       n_samples++;
-      const float4 s = isnan(f) ? make_float4(0.f, 0.f, 0.f, 0.f) : tf_map(v, f);
+      const float4 s = isnan(f) ? make_float4(0.f, 0.f, 0.f, 0.f) : tf_map(v, f, rmaj > 0.f);
       mode = M_DRAW;
       if (ratio) {
-        T *= fmx(0.f, 1.f - (v.rn ? div_rn(s.w, maj, rmaj) : s.w / maj));
+        T *= fmx(0.f, 1.f - bnx_num::over_majorant(s.w, maj, rmaj));
         if (T == 0.f) hit(tmax, v3{0.f, 0.f, 0.f});
       } else if (s.w >= rnd() * maj) {
         hit(t, v3{s.x, s.y, s.z});
@@ -509,7 +509,7 @@ template <int FIELD> struct March {
             if (maj != 0.f) {
               upper = fmn(c1, tmax);
               t = c0;
-              rmaj = rcp_rn(maj);
+              rmaj = v.rn && bnx_num::short_majorant(maj) ? rcp_rn(maj) : 0.f;
               mode = M_DRAW;
             }
           }
@@ -517,8 +517,8 @@ template <int FIELD> struct March {
         if (mode == M_DRAW) {
           const float r = rnd();
           const float s = -fast_log(1.f - r);
-          t += v.rn ? div_rn(s, maj, rmaj) : s / maj;
-          if (t >= upper) {
+          t += bnx_num::over_majorant(s, maj, rmaj);
+          if (!(t < upper)) {           // also where a NaN in the transfer function made t one
             mode = M_CELL;
           } else {
             P = o + t * d;

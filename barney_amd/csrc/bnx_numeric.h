@@ -48,6 +48,27 @@ static constexpr float INV_F10 = 0x1.27e4fcp-22f;
 static constexpr float INV_F11 = 0x1.ae6456p-26f;
 static constexpr float INV_F12 = 0x1.1eed8ep-29f;
 
+// One fused correction each of an estimate y of 1 / b and of a * y, the
+// quotient a / b (Markstein, "Computation of elementary functions on the IBM
+// RISC System/6000 processor", 1990).
+BNX_HD inline float rcp_step(float b, float y) { return __builtin_fmaf(__builtin_fmaf(-b, y, 1.f), y, y); }
+BNX_HD inline float div_step(float a, float b, float y)
+{
+  const float q = a * y;
+  return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+// x over a macrocell's majorant, of which rmaj is the reciprocal, or 0 where
+// the short form does not hold.  A majorant is an alpha of the transfer
+// function or a mean of two, and next to an alpha of 0 the mean is as small
+// as the cell's scalars: below about 2^-126 the reciprocal is infinite and
+// div_step gives NaN.  Down to 2^-60 every quotient in use is far from both
+// ends of the float range.
+BNX_HD inline bool short_majorant(float maj) { return maj >= 0x1p-60f; }
+BNX_HD inline float over_majorant(float x, float maj, float rmaj)
+{
+  return rmaj > 0.f ? div_step(x, maj, rmaj) : x / maj;
+}
+
 // sin on |r| <= pi/4 (Taylor to r^11, Horner in r^2)
 BNX_HD inline float sin_kernel(float r)
 {

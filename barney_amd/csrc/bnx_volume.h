@@ -84,7 +84,8 @@ struct VolumeDev {
   int ntf;
   float dom0, dom1, base_density;
   float rcp_span;             // 1 / (dom1 - dom0) (host float division)
-  int rn;                     // spacings, domain and densities lie where rcp_rn and div_rn are exact
+  int rn;                     // spacings, domain and densities lie where rcp_rn and div_rn are exact; a
+                              // cell's majorant has to as well (short_majorant)
   int rtc_inst;               // rtc instance index (seeds the march RNG)
   int user_inst;
   int user_id;
@@ -533,14 +534,17 @@ BNX_D int seed_cell(const VolumeDev &v, v3 P)
   return (c[2] * v.seed_dims[1] + c[1]) * v.seed_dims[0] + c[0];
 }
 
-// TransferFunction::DD::map (volume/TransferFunction.h:67-87)
-BNX_D float4 tf_map(const VolumeDev &v, float s)
+// TransferFunction::DD::map (volume/TransferFunction.h:67-87).  rn: v.rn,
+// and the macrocell's majorant is none of the tiny ones.  There a scalar so
+// close to the domain's begin that its short quotient may be off in the last
+// bit has a density below any product of the majorant with a draw but 0.
+BNX_D float4 tf_map(const VolumeDev &v, float s, bool rn)
 {
   const int N = v.ntf;
   const float span = v.dom1 - v.dom0, x = s - v.dom0;
   float f = x * v.rcp_span;
   // far above the domain (infinite scalars too) the quotient need not be exact
-  if (!v.rn) f = x / span;
+  if (!rn) f = x / span;
   else if (f < 2.f) f = div_rn(x, span, v.rcp_span);
   f = fmn(fmx(f, 0.f), 1.f);
   f *= (float)(N - 1);

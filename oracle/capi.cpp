@@ -6,6 +6,7 @@
 #include "dda.h"
 
 #include <chrono>
+#include <cmath>
 #include <cstdio>
 
 namespace orc {
@@ -739,6 +740,24 @@ int orc_cone_intersect_n(const float *rays, int n, const float *cone, float tmin
 }
 
 void orc_sincos(float x, float *s, float *c) { bnx_num::sincos(x, *s, *c); }
+// An estimate of 1 / b, `ulps` off the rounded one; where that overflows, or b
+// is subnormal, it is infinite, as the hardware's is
+static float rcp_estimate(float b, int ulps)
+{
+  float y = std::fabs(b) < 0x1p-126f ? std::copysign(INFINITY, b) : 1.f / b;
+  for (int k = 0; k < std::abs(ulps) && std::isfinite(y); k++) y = std::nextafter(y, ulps > 0 ? INFINITY : -INFINITY);
+  return y;
+}
+// x[i] over the majorant maj[i] as the march computes it; guard 0: without
+// its look at the majorant
+void orc_over_majorant_n(const float *x, const float *maj, int ulps, int guard, int n, float *out)
+{
+  for (int i = 0; i < n; i++) {
+    const bool rn = !guard || bnx_num::short_majorant(maj[i]);
+    const float r = rn ? bnx_num::rcp_step(maj[i], rcp_estimate(maj[i], ulps)) : 0.f;
+    out[i] = guard ? bnx_num::over_majorant(x[i], maj[i], r) : bnx_num::div_step(x[i], maj[i], r);
+  }
+}
 void orc_atan2_n(const float *y, const float *x, int n, float *out)
 {
   for (int i = 0; i < n; i++) out[i] = bnx_num::atan2(y[i], x[i]);

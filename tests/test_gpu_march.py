@@ -1,7 +1,8 @@
 """The march kernels where they can go wrong, on the GPU against the CPU
 oracle: frames whose rays do not fill a wave, a 256-ray block or its chunks;
 more volumes in a world than a launch has claim counters; scalars that are
-not finite (no corner copy, open value ranges); isosurfaces whose samples'
+not finite (no corner copy, open value ranges); macrocells whose majorants are
+as small as floats get; isosurfaces whose samples'
 sides come from a fine grid of a single cell up to one a few cells wide, at
 values inside, at the ends and outside of the field's range, and over cells
 collapsed to triangles and lines.  IDs, ray and
@@ -69,6 +70,28 @@ def test_scalars_not_finite(dev, orc, bad):
     f[9:11, 7, 12] = bad
     vs = dataclasses.replace(vs, scalars=f)
     _compare(dev, orc, vs, bx.VolumeWorld(dev, vs).world, orc.volume_scene(vs), 1)
+
+
+@pytest.mark.parametrize("flags", [0, abi.BNX_RENDER_RATIO_TRACKING])
+@pytest.mark.parametrize("kind", ["structured", "tets"])
+def test_tiny_majorants(dev, orc, kind, flags):
+    """one narrow Gaussian whose tails run through every exponent down to 0, and a map that begins at 0"""
+    print(f"march tiny majorants {kind} flags={flags}", flush=True)
+    if kind == "structured":
+        vs = scenes.config2(n=64, mc_grid=16, width=64, height=64)
+        x = (np.arange(64) / 63.0 - 0.5) ** 2
+        r2 = x[:, None, None] + x[None, :, None] + x[None, None, :]
+        vs = dataclasses.replace(vs, scalars=np.exp(-r2 / (2 * .05 ** 2)).astype(np.float32))
+        world, scene = bx.VolumeWorld(dev, vs).world, orc.volume_scene(vs)
+    else:
+        vs = scenes.config4(n=16, width=48, height=48)
+        r2 = ((vs.vertices.astype(np.float64) - vs.vertices.mean(0)) ** 2).sum(1)
+        f = np.exp(-r2 / (2 * (.05 * np.ptp(vs.vertices)) ** 2)).astype(np.float32)
+        vs = dataclasses.replace(vs, scalars=f, tf_domain=(0.0, 1.0))
+        world, scene = bx.UMeshWorld(dev, vs).world, orc.umesh_scene(vs)
+    tails = vs.scalars[(vs.scalars > 0) & (vs.scalars < 1e-38)]
+    assert tails.size > 50 and vs.tf[0, 3] == 0
+    _compare(dev, orc, vs, world, scene, 2, flags)
 
 
 @pytest.mark.parametrize("n,iso", [(1, .2), (2, .3), (3, .05), (5, 1.), (5, 0.), (5, -3.), (9, .3)])
