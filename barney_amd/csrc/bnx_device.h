@@ -57,6 +57,10 @@ BNX_D v3 normalize(v3 a) { return a * (1.f / sqrtf(dot(a, a))); }
 BNX_D float reduce_max(v3 a) { return fmx(fmx(a.x, a.y), a.z); }
 BNX_D v3 vabs(v3 a) { return v3{fabsf(a.x), fabsf(a.y), fabsf(a.z)}; }
 BNX_D v3 xyz(float4 f) { return v3{f.x, f.y, f.z}; }
+BNX_D bool finite(v3 a)
+{
+  return __builtin_isfinite(a.x) & __builtin_isfinite(a.y) & __builtin_isfinite(a.z);
+}
 BNX_D v3 ld3(const float *p) { return v3{p[0], p[1], p[2]}; }
 
 // Correctly rounded reciprocal, quotient and square root for operands whose

@@ -335,26 +335,27 @@ BNX_D void instance_ray(const float4 w2o[3], const float4 *rorg, const float4 *r
   inv = v3{1.f / d.x, 1.f / d.y, 1.f / d.z};
 }
 
-// into the instance of TLAS leaf entry i: its BLAS, and, if it moves the ray
-// (XF), the ray in its frame; true: moved
+// into the instance of TLAS leaf entry e: its BLAS, and, if it moves the ray
+// (XF), the ray in its frame.  false: the ray is not finite there (the
+// instance's transform flattens it, and has no inverse) and hits nothing.
 template <bool XF>
 BNX_D bool enter_instance(const EnterDev BNX_G *e, const float4 *rorg, const float4 *rdir, Blas &b, v3 &o, v3 &d,
                           v3 &inv)
 {
   const EnterDev E = *e;
   b = Blas{E.nodes, E.prims, E.refs, E.type, E.inst, E.geom_base, E.translucent != 0};
-  if (!XF || E.identity) return false;
+  if (!XF || E.identity) return true;
   instance_ray(E.w2o, rorg, rdir, o, d, inv);
-  return true;
+  return finite(o) && finite(d);
 }
 
 // entry distance of child k of a 4-wide node, +inf when the ray misses it.
 // Branch-free, so the six box vectors of a node are loaded together up front
 // (a short-circuit on the child code let the compiler sink each child's box
 // loads behind the code load, doubling the dependent fetches per node).
-// |inv| <= 1e6 (|d| >= 1e-6 after fix_dir) and empty slots hold inverted
-// infinite boxes, so no slab distance is NaN and fminf/fmaxf give the same
-// values as compares.
+// Rays are finite, |inv| <= 1e6 (|d| >= 1e-6 after fix_dir) and empty slots
+// hold inverted infinite boxes, so no slab distance is NaN and fminf/fmaxf
+// give the same values as compares.
 BNX_D float child_entry(v3 o, v3 inv, float lx, float hx, float ly, float hy, float lz, float hz, uint32_t code,
                         float tmin, float tmax)
 {
@@ -394,9 +395,8 @@ BNX_D Octant octant_of(v3 d)
 // the ray misses it.  |inv| <= 1e6 (|d| >= 1e-6 after fix_dir), so the
 // distances are those of the slab test with its minima and maxima taken:
 // (plane - o) * inv is monotone in the plane.  An empty slot's planes are
-// inverted infinities: its entry lies behind its exit for every finite
-// origin, and an origin that is not finite hits nothing whichever way it
-// goes through the tree.
+// inverted infinities: its entry lies behind its exit for every finite ray,
+// and a ray that is not finite never comes here.
 BNX_D float slab_entry(v3 o, v3 inv, float nx, float fx, float ny, float fy, float nz, float fz, float tmin, float tmax)
 {
   const float tn = fmaxf(fmaxf(fmaxf(tmin, (nx - o.x) * inv.x), (ny - o.y) * inv.y), (nz - o.z) * inv.z);
@@ -471,7 +471,9 @@ BNX_D void walk_rays(Claims &pr, const SceneDev &S, const SRC &src, int take, ui
           nodes = S.tlas_nodes;
           in_blas = false;
           sp = low = 0;
-          cur = S.num_insts > 0 ? 0 : EMPTY4;
+          // a ray that is not finite would pass every slab test, those of
+          // unused child slots too, and no hit could come of it
+          cur = S.num_insts > 0 && finite(o) && finite(d) ? 0 : EMPTY4;
         }
       }
       continue;
@@ -530,13 +532,16 @@ BNX_D void walk_rays(Claims &pr, const SceneDev &S, const SRC &src, int take, ui
       pop();
     } else if (!in_blas && (cur & LEAF_BIT) != 0) {
       // ------------------------------------ ... or a TLAS leaf: into its own
-      if (enter_instance<XF>(S.enter + ((cur & ~LEAF_BIT) >> 3), src.org(ray), src.dir(ray), blas, o, d, inv))
-        oct = octant_of(d);
-      room();
-      slot(sp++) = LEAVE_BLAS;
+      const uint32_t entry = (cur & ~LEAF_BIT) >> 3;
+      cur = LEAVE_BLAS;
+      if (enter_instance<XF>(S.enter + entry, src.org(ray), src.dir(ray), blas, o, d, inv)) {
+        if (XF) oct = octant_of(d);
+        room();
+        slot(sp++) = LEAVE_BLAS;
+        nodes = blas.nodes;
+        cur = 0;
+      }
       in_blas = true;
-      nodes = blas.nodes;
-      cur = 0;
     }
   }
   if (ray >= 0) src.store(S, ray, best, rej);
@@ -582,7 +587,7 @@ BNX_D HitRec traverse_spec(const SceneDev &S, const float4 *rorg, const float4 *
   const Node4 BNX_G *nodes = S.tlas_nodes;
   Blas blas{};
   bool in_blas = false;
-  uint32_t cur = 0;
+  uint32_t cur = finite(o) && finite(d) ? 0 : EMPTY4;
   uint32_t leaf = 0;             // primitive leaf set aside (leaf codes carry LEAF_BIT)
   uint32_t nvis = 0;
   // every node is entered at most once per ray; the cap only bounds the
@@ -631,15 +636,15 @@ BNX_D HitRec traverse_spec(const SceneDev &S, const float4 *rorg, const float4 *
     } else if ((cur & LEAF_BIT) && !in_blas) {
       // a TLAS leaf (the node phase sets every BLAS leaf aside): enter its
       // instance
-      (void)enter_instance<XF>(S.enter + ((cur & ~LEAF_BIT) >> 3), rorg, rdir, blas, o, d, inv);
+      const bool in = enter_instance<XF>(S.enter + ((cur & ~LEAF_BIT) >> 3), rorg, rdir, blas, o, d, inv);
       if (EXT) {
         cut.geom_base = blas.geom_base;
         cut.translucent = blas.translucent;
       }
-      push(LEAVE_BLAS);
+      if (in) push(LEAVE_BLAS);
       in_blas = true;
       nodes = blas.nodes;
-      cur = 0;
+      cur = in ? 0 : LEAVE_BLAS;
     } else if (cur == LEAVE_BLAS) {
       in_blas = false;
       if (XF) world_ray(rorg, rdir, o, d, inv);

@@ -927,6 +927,11 @@ void pair_hit(const Instance &in, const Geom &g, int prim, vec3 o, vec3 d, float
   }
 }
 
+// A ray that is not finite hits nothing; a transform that flattens its
+// instance has no inverse, and gives such a ray.  (Its slab and primitive
+// tests would be decided by NaN, and by the order of the walk.)
+static bool finite(vec3 a) { return std::isfinite(a.x) && std::isfinite(a.y) && std::isfinite(a.z); }
+
 Hit trace_bvh(const Scene &s, vec3 org, vec3 dir0, float tmin, float tmax, bool any_hit, TraceCounters *ctr,
               const float *cut_plane, const uint64_t *seed, Hit *rej)
 {
@@ -937,6 +942,7 @@ Hit trace_bvh(const Scene &s, vec3 org, vec3 dir0, float tmin, float tmax, bool 
   best.t = tmax;
   best.u = best.v = 0.f;
   if (ctr) ctr->rays++;
+  if (!finite(org) || !finite(dir)) return best;
   vec3 winv(1.f / dir.x, 1.f / dir.y, 1.f / dir.z);
   // stack entries: cnt == 0 inner node, cnt > 0 leaf [ref, ref+cnt),
   // ENTER: instance 'ref' (TLAS leaf), LEAVE: back to the TLAS
@@ -968,7 +974,7 @@ Hit trace_bvh(const Scene &s, vec3 org, vec3 dir0, float tmin, float tmax, bool 
         inv = vec3(1.f / d.x, 1.f / d.y, 1.f / d.z);
       }
       stack[sp++] = {0, LEAVE};
-      stack[sp++] = {0, 0};
+      if (finite(o) && finite(d)) stack[sp++] = {0, 0};
       continue;
     }
     const Bvh &bvh = in_blas ? s.groups[s.insts[inst].group].bvh : s.tlas;
@@ -1019,6 +1025,7 @@ Hit trace_brute(const Scene &s, vec3 org, vec3 dir0, float tmin, float tmax, con
       o = xfm_point(in.w2o, org);
       d = fix_dir(xfm_vector(in.w2o, dir));
     }
+    if (!finite(o) || !finite(d)) continue;
     const Group &g = s.groups[in.group];
     for (int k = 0; k < (int)g.bvh.order.size(); k++)
       prim_test(s, g, k, o, d, tmin, best, inst, nullptr, cut, seed, rej);

@@ -2,7 +2,8 @@
 ray counts at the edges of a wave, of a chunk and of a 256-ray block, for
 every variant of the ray-array kernel (triangles and spheres, or all
 primitives; with and without instance transforms); rays along and against
-every axis and rays that are not finite; and rays traced by several threads
+every axis and rays that are not finite; instances whose transform flattens
+them and has no inverse, among others; and rays traced by several threads
 of one device at once.  Hits are compared bit for bit."""
 import threading
 
@@ -61,6 +62,35 @@ def test_rays_not_finite(dev):
         rays[k::3, 0:3] = bad
     assert (g.trace(rays)["prim_id"] == -1).all()
     assert (g.trace(rays, any_hit=True)["prim_id"] == -1).all()
+
+
+@pytest.mark.parametrize("ext", [False, True])
+@pytest.mark.parametrize("flat", [(1, 0, 0, 0, 1, 0, 0, 0, 0), (0, 0, 0, 0, 0, 0, 0, 0, 1), (0,) * 9])
+def test_flat_instances(dev, orc, ext, flat):
+    """a flattened instance is not hit, and a ray that meets its box goes on
+    to the instances behind it: the IDs below and above the flat ones"""
+    print(f"trace waves flat instances ext={ext} {flat}", flush=True)
+    spec = helpers.sticks_spec(True) if ext else helpers.instanced_spec()
+    plain = list(spec.insts)
+    m = np.array(list(flat) + [0.1, -0.2, 0.3], np.float32)
+    inv = np.full(12, np.nan, np.float32)
+    at = (0, 2, len(plain) + 1)
+    for k in at:
+        spec.insts.insert(k, (plain[-1][0], 90 + k, m, inv))
+    rays = scenes.random_rays(24, 20000, radius=6.0, spread=3.0)
+    o = spec.oracle(orc)
+    want = o.trace(rays)[0]
+    hit = want["prim_id"] >= 0
+    assert hit.sum() > 1000 and not np.isin(want["inst"], at).any()
+    # as without them, but for the places of the others
+    spec.insts = plain
+    without = spec.oracle(orc).trace(rays)[0]
+    assert np.array_equal(want["t"], without["t"]) and np.array_equal(want["prim_id"], without["prim_id"])
+    for k in at:
+        spec.insts = spec.insts[:k] + [(plain[-1][0], 90 + k, m, inv)] + spec.insts[k:]
+    g = spec.gpu(dev)
+    _same(g.trace(rays), want)
+    assert np.array_equal(g.trace(rays, any_hit=True)["prim_id"] >= 0, hit)
 
 
 def test_threads(dev, orc):
