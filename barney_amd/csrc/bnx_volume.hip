@@ -482,51 +482,102 @@ int build_tet_neighbors(Device *dev, const int4 *tets, int ntet, DevMem &nbr)
 // The value ranges: every cell adds the range of its vertices' scalars to the
 // grid cells that its box touches, grown by a twentieth of its extent and
 // 1e-5 of its coordinates (a test accepts points outside the cell by far
-// less, see k_cell_pack).  A cell with more than FINE_MOST grid cells, and a
-// tet too flat for that, adds to the range that all grid cells share.  Values are means of the scalars with
-// weights above -1e-3 (a Newton inversion's last step), so the ranges take in
-// a thousandth of their width and 1e-5 of the scalars at either end.
-constexpr int FINE_MOST = 4096;
+// less, see k_cell_pack).  Values are means of the scalars with weights above
+// -1e-3 (a Newton inversion's last step), so the ranges take in a thousandth
+// of their width and 1e-5 of the scalars at either end.
+//
+// A tet adds less: only to the grid cells that reach past none of its planes
+// by more than a hundredth of its size, and there only the values that its
+// linear function takes between the cell's corners.  With its whole range in
+// every grid cell of its box a mesh of few tets, whose boxes take in most of
+// it, settled hardly a sample (jittered cubes of five tets, 1920x1080, 2 spp,
+// isosurface and volume: 8^3 15.5 ms then, 11.4 now; 14^3 13.2 and 9.7; 40^3
+// 12.5 and 10.0; 160^3 13.5 and 12.9).
+//
+// A cell with more than `most` grid cells in its box, and a tet too flat for
+// its planes to bound where it is accepted, adds its whole range to the one
+// that all grid cells share.  LANES threads work on a cell.
 constexpr float FINE_SLACK = 1e-5f;
+template <int LANES>
 __global__ void k_fine_ranges(const int4 *tets, const int4 *ext, const uint8_t *types, const float4 *verts, int n,
-                              VolumeDev d, int *lo, int *hi, int *all)
+                              VolumeDev d, long long most, int *lo, int *hi, int *all)
 {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int c = (int)(tid / LANES), sub = (int)(tid % LANES);
   if (c >= n) return;
   float4 l, h;
   cell_box(tets, ext, types, verts, c, l, h);
   const float size = fmx(fmx(h.x - l.x, h.y - l.y), h.z - l.z);
   const float far = fmx(fmx(fmx(fabsf(l.x), fabsf(h.x)), fmx(fabsf(l.y), fabsf(h.y))), fmx(fabsf(l.z), fabsf(h.z)));
-  const float m = .05f * size + 1e-5f * far, slack = 1e-3f * (h.w - l.w) + FINE_SLACK * fmx(fabsf(l.w), fabsf(h.w));
+  const float m = .05f * size + 1e-5f * far, slack = 2e-3f * (h.w - l.w) + FINE_SLACK * fmx(fabsf(l.w), fabsf(h.w));
   const int a = seed_cell(d, v3{l.x - m, l.y - m, l.z - m}), b = seed_cell(d, v3{h.x + m, h.y + m, h.z + m});
   const int nx = d.seed_dims[0], ny = d.seed_dims[1];
   const int ax = a % nx, ay = (a / nx) % ny, az = a / (nx * ny), bx = b % nx, by = (b / nx) % ny, bz = b / (nx * ny);
-  const int vl = f2o(l.w - slack), vh = f2o(h.w + slack);
   const bool finite = slack < INFINITY;       // an infinite scalar: any value may come of it
   // A tet's planes, computed with an error e, accept the tet scaled by
   // (r + e) / r about its incentre, r the radius of its inscribed sphere: with
   // e below 1e-6 of the distance to it and r a thousandth of its size that is
   // well inside the margin.  A flatter one may accept any point of its leaf.
+  const bool tet = !types || types[c] == CELL_TET;
   bool flat = false;
-  if (!types || types[c] == CELL_TET) {
-    const v3 p0 = xyz(cell_vertex(tets, ext, verts, c, 0)), p1 = xyz(cell_vertex(tets, ext, verts, c, 1)),
-             p2 = xyz(cell_vertex(tets, ext, verts, c, 2)), p3 = xyz(cell_vertex(tets, ext, verts, c, 3));
-    const v3 e1 = p1 - p0, e2 = p2 - p0, e3 = p3 - p0;
-    const v3 n0 = cross(e2 - e1, e3 - e1), n1 = cross(e2, e3), n2 = cross(e3, e1), n3 = cross(e1, e2);
-    flat = !(fabsf(dot(e1, n1)) >= 1e-3f * size * (length(n0) + length(n1) + length(n2) + length(n3)));
+  v3 N[4], at[4], grad{0.f, 0.f, 0.f};
+  float past[4], s[4], sum = 0.f;
+  const float mid = .5f * l.w + .5f * h.w;
+  if (tet) {
+    float4 q[4];
+    for (int k = 0; k < 4; k++) q[k] = cell_vertex(tets, ext, verts, c, k);
+    // the planes of tet_planes: t[k] = dot(P - at[k], N[k])
+    N[0] = cross(xyz(q[3]) - xyz(q[1]), xyz(q[2]) - xyz(q[1]));
+    N[1] = cross(xyz(q[2]) - xyz(q[0]), xyz(q[3]) - xyz(q[0]));
+    N[2] = cross(xyz(q[3]) - xyz(q[0]), xyz(q[1]) - xyz(q[0]));
+    N[3] = cross(xyz(q[1]) - xyz(q[0]), xyz(q[2]) - xyz(q[0]));
+    for (int k = 0; k < 4; k++) at[k] = xyz(q[k == 0 ? 1 : 0]);
+    sum = dot(xyz(q[1]) - xyz(q[0]), N[1]);
+    float area = 0.f;
+    for (int k = 0; k < 4; k++) area += length(N[k]);
+    flat = !(fabsf(sum) > 1e-3f * size * area);
+    for (int k = 0; k < 4; k++) {
+      s[k] = (q[k].w - mid) / sum;
+      grad = grad + s[k] * N[k];
+    }
   }
-  if (!finite || flat || (long long)(bx - ax + 1) * (by - ay + 1) * (bz - az + 1) > FINE_MOST) {
-    atomicMin(all, finite ? vl : f2o(-INFINITY));
-    atomicMax(all + 1, finite ? vh : f2o(INFINITY));
+  const long long cells = (long long)(bx - ax + 1) * (by - ay + 1) * (bz - az + 1);
+  if (!finite || flat || cells > most) {
+    if (sub == 0) {
+      atomicMin(all, f2o(finite ? l.w - slack : -INFINITY));
+      atomicMax(all + 1, f2o(finite ? h.w + slack : INFINITY));
+    }
     return;
   }
-  for (int z = az; z <= bz; z++)
-    for (int y = ay; y <= by; y++)
-      for (int x = ax; x <= bx; x++) {
-        const int i = (z * ny + y) * nx + x;
-        atomicMin(lo + i, vl);
-        atomicMax(hi + i, vh);
+  // half the sides of a grid cell, with what the cell that a point is given
+  // to may be off by
+  const v3 side{1.f / d.seed_rcp[0], 1.f / d.seed_rcp[1], 1.f / d.seed_rcp[2]};
+  const v3 half{.52f * side.x + 1e-5f * far, .52f * side.y + 1e-5f * far, .52f * side.z + 1e-5f * far};
+  if (tet)
+    for (int k = 0; k < 4; k++) past[k] = dot(vabs(N[k]), half) + 1e-2f * size * length(N[k]);
+  const float reach = dot(vabs(grad), half);
+  const int wx = bx - ax + 1, wy = by - ay + 1;
+  for (long long j = sub; j < cells; j += LANES) {
+    const int x = ax + (int)(j % wx), y = ay + (int)((j / wx) % wy), z = az + (int)(j / ((long long)wx * wy));
+    float vl = l.w, vh = h.w;
+    if (tet) {
+      const v3 C{d.seed_origin[0] + ((float)x + .5f) * side.x, d.seed_origin[1] + ((float)y + .5f) * side.y,
+                 d.seed_origin[2] + ((float)z + .5f) * side.z};
+      float f = mid;
+      bool out = false;
+      for (int k = 0; k < 4; k++) {
+        const float t = dot(C - at[k], N[k]);
+        out |= t < -past[k];
+        f += t * s[k];
       }
+      vl = fmx(vl, f - reach);
+      vh = fmn(vh, f + reach);
+      if (out || vl - slack > vh + slack) continue;
+    }
+    const int i = (z * ny + y) * nx + x;
+    atomicMin(lo + i, f2o(vl - slack));
+    atomicMax(hi + i, f2o(vh + slack));
+  }
 }
 
 // per grid cell the tet (depth-first query) holding its centre, and its range
@@ -551,8 +602,12 @@ __global__ __launch_bounds__(SEED_TB) void k_fine_pack(VolumeDev d, int ncells, 
   fine[c] = make_float4(__int_as_float(seed), o2f(min(lo[c], all[0])), o2f(max(hi[c], all[1])), 0.f);
 }
 
-// fine grid of about one cell per two tets, or eight per other cell, over the
-// bounds (at most 256 a side); ext, types null: tets
+// Fine grid over the bounds: of a mesh of tets about one cell per two tets, and
+// no fewer than FINE_MC a side of a macrocell (a march's sub-steps are a tenth
+// of one; 2: 14^3 10.2 ms and 40^3 11.7, 6: 10.7 and 9.6, in three times the
+// memory), of another mesh eight per cell; at most 256 a side.  ext, types
+// null: tets
+constexpr int FINE_MC = 4;
 int build_fine_grid(Volume *v, const int4 *tets, const int4 *ext, const uint8_t *types, const float4 *verts, int n)
 {
   VolumeDev &d = v->dd;
@@ -569,7 +624,8 @@ int build_fine_grid(Volume *v, const int4 *tets, const int4 *ext, const uint8_t 
   const double h = std::cbrt(vol / std::max(1.0, d.field == FIELD_KIND_TETS ? n / 2.0 : 8.0 * n));
   long long ncells = 1;
   for (int k = 0; k < 3; k++) {
-    d.seed_dims[k] = (int)std::min(256.0, std::max(1.0, std::ceil(size[k] / h)));
+    const double least = d.field == FIELD_KIND_TETS ? (double)FINE_MC * d.mc[k] : 1.0;
+    d.seed_dims[k] = (int)std::min(256.0, std::max(least, std::ceil(size[k] / h)));
     d.seed_origin[k] = d.lo[k];
     d.seed_rcp[k] = (float)d.seed_dims[k] / (float)size[k];
     ncells *= d.seed_dims[k];
@@ -582,8 +638,14 @@ int build_fine_grid(Volume *v, const int4 *tets, const int4 *ext, const uint8_t 
   DevMem all;
   BNX_HIP(all.ensure(2 * sizeof(int)));
   k_fill_ranges<<<1, 64, 0, st>>>(all.as<int>(), all.as<int>() + 1, 1);
-  k_fine_ranges<<<nblk(n, 256), 256, 0, st>>>(tets, ext, types, verts, n, d, lo.as<int>(), hi.as<int>(),
-                                              all.as<int>());
+  // few cells meet many grid cells each: more of these, and more threads, for each
+  const long long most = std::max(4096LL, (1LL << 26) / std::max(1, n));
+  if (n < (1 << 18))
+    k_fine_ranges<64><<<nblk(64L * n, 256), 256, 0, st>>>(tets, ext, types, verts, n, d, most, lo.as<int>(),
+                                                          hi.as<int>(), all.as<int>());
+  else
+    k_fine_ranges<1><<<nblk(n, 256), 256, 0, st>>>(tets, ext, types, verts, n, d, most, lo.as<int>(), hi.as<int>(),
+                                                   all.as<int>());
   k_fine_pack<<<nblk(ncells, SEED_TB), SEED_TB, 0, st>>>(d, (int)ncells, lo.as<int>(), hi.as<int>(), all.as<int>(),
                                                          v->ufine.as<float4>());
   BNX_HIP(hipGetLastError());

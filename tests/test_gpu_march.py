@@ -105,6 +105,32 @@ def test_isosurface_sides(dev, orc, kind, n, iso):
     _compare(dev, orc, us, bx.UMeshWorld(dev, us).world, orc.umesh_scene(us), 1)
 
 
+@pytest.mark.parametrize("n,mc", [(1, (9, 9, 9)), (6, (5, 40, 17)), (12, (64, 64, 64)), (5, (300, 4, 4)),
+                                  (38, (32, 32, 32))])
+def test_isosurface_fine_grids(dev, orc, n, mc):
+    """few tets with many grid cells each, grids of other shapes than cubes and
+    at their largest, tets with more grid cells than they may have ranges in
+    (12: some 20,000), and enough tets for a thread each (38)"""
+    print(f"iso march fine grid n={n} mc={mc}", flush=True)
+    us = dataclasses.replace(scenes.config4(n=n, width=60, height=52, volume=False), mc_dims=mc)
+    _compare(dev, orc, us, bx.UMeshWorld(dev, us).world, orc.umesh_scene(us), 1)
+
+
+@pytest.mark.parametrize("n", [4, 8, 14, 40])
+def test_isosurface_queries_of_coarse_meshes(dev, n):
+    """Tet tests a ray: 46, 34, 27 and 25 when every sub-step up to the crossing
+    was queried in turn, each from the last one's tet; the samples that the fine
+    grid does not settle have to be far fewer than that, on meshes of few cells
+    too (6 to 14)."""
+    print(f"iso march queries n={n}", flush=True)
+    us = scenes.config4(n=n, width=160, height=120, volume=False)
+    world, c, fr = bx.UMeshWorld(dev, us), us.camera, bx.Frame(dev, 160, 120)
+    st = bx.render(world.world, bx.camera_perspective(c["position"], c["direction"], c["up"], c["fovy"]),
+                   abi.renderer(bg=us.bg_color, ambient=us.ambient), fr, 1)
+    fr.close()
+    assert st["umesh_tets"] <= 20 * st["rays"], st["umesh_tets"] / st["rays"]
+
+
 @pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
 def test_isosurface_of_scalars_not_finite(dev, orc, bad):
     print(f"iso march scalar {bad}", flush=True)
