@@ -44,6 +44,7 @@ constexpr int TAKE = 8;          // a new ray, already set up
 constexpr int SEED_AT = 4;       // a tet mesh's seed
 constexpr int CELL_AT = 12;      // a macrocell, where point queries are most of the work
 constexpr int NODE_AT = 10;      // a depth-first query
+constexpr int SIDES_AT = 24;     // the sides of a macrocell's sub-steps (isosurfaces; 16 to 32 within 1%)
 
 // what a lane's ray waits for
 enum Mode {
@@ -599,25 +600,31 @@ template <int FIELD> struct March {
 // grid's value range at its point holds the iso value: otherwise its side is
 // known, and an interval between two samples of one side has no crossing; a
 // sample of known side is queried after all when the one next to it turns
-// out to lie on the other.  Bound by the records that the queries read (about
+// out to lie on the other.  The owner looks all sides of a cell up itself,
+// eleven loads in flight at once, and posts what is left: most cells end
+// there, and dealing their samples out for a look at the grid each cost more
+// than the queries that remain (8^3 cubes of five tets, 1920x1080, 2 spp: 11.0
+// ms with that, 7.8 so; 160^3: 12.7 and 11.3).  Bound by the records that the queries read (about
 // 1.8 requests beyond the L1 for each tet tested), so what helps is to ask for
 // fewer samples: 20.5M tets, 1024^2, 4 spp, isosurface and volume: 24.2 ms a
-// pass as nested loops, 16.7 with the samples dealt out, 13.2 with sides from
-// the fine grid; 14^3 mixed cells, 320x240, 2 spp: 41.6, 8.2, 6.6.
-enum Owner { O_IDLE = 0, O_CELL, O_WAIT };
+// pass as nested loops, 16.7 with the samples dealt out, 13.5 with sides from
+// the fine grid, 12.3 with the owners' look; 14^3 mixed cells, 320x240, 2 spp:
+// 41.6, 8.2, 6.6, 6.0.
+enum Owner { O_IDLE = 0, O_CELL, O_SIDES, O_WAIT };
 enum Worker { W_FREE = 0, W_WALK, W_NODE, W_TEST };
 
 constexpr int ISO_SUBS = 10, ISO_GRADS = 7, ISO_SLOTS = ISO_SUBS + 1;
 constexpr int ISO_ITEMS = 1024;  // ring of posted samples: at most ISO_SLOTS per lane
 static_assert(64 * ISO_SLOTS <= ISO_ITEMS, "sample ring");
-constexpr int ITEM_GRADIENT = 1 << 10, ITEM_VALUE = 1 << 11;   // a gradient's sample; a value, not a side, is wanted
+constexpr uint32_t ALL_SLOTS = (1u << ISO_SLOTS) - 1u;
+constexpr int ITEM_GRADIENT = 1 << 10;
 struct IsoShared {
   float ray[6][64];              // origin, direction
   float t0[64], t1[64];          // the cell's range, or twice the crossing
   float value[ISO_SLOTS][64];
   int open[64];                  // samples not yet taken
   uint32_t side[64];             // slots that hold a side (an infinity) for a value
-  uint16_t item[ISO_ITEMS];      // owner | slot << 6 | ITEM_*
+  uint16_t item[ISO_ITEMS];      // owner | slot << 6 | ITEM_GRADIENT
 };
 
 template <int FIELD> struct IsoMarch {
@@ -693,10 +700,11 @@ template <int FIELD> struct IsoMarch {
       wave_sync();
       const bool done = own == O_WAIT && L.open[lane] == 0;
       const int n_done = __popcll(__ballot(done)), n_cell = __popcll(__ballot(own == O_CELL));
+      const int n_sides = __popcll(__ballot(own == O_SIDES));
       const uint64_t free = __ballot(work == W_FREE);
       const int n_free = __popcll(free), items = tail - head;
       const bool starved = n_free == 64 && items == 0;
-      if (!pr.dry && (n_idle >= 16 || (starved && n_idle > 0 && n_done + n_cell < 16))) {
+      if (!pr.dry && (n_idle >= 16 || (starved && n_idle > 0 && n_done + n_cell + n_sides < 16))) {
         // ---------------------------------------------------- new rays
         bool on;
         const int i = pr.claim(n_idle, __popcll(idle & lanemask_lt()), on);
@@ -730,7 +738,7 @@ template <int FIELD> struct IsoMarch {
         continue;
       }
       if (n_idle == 64) break;
-      if (n_done >= 16 || (starved && n_done >= n_cell && n_done > 0)) {
+      if (n_done >= 16 || (starved && n_done >= max(n_cell, n_sides) && n_done > 0)) {
         // ------------------------------------------- use the values taken
         uint32_t which = 0;
         int kind = 0;
@@ -755,7 +763,6 @@ template <int FIELD> struct IsoMarch {
             a0 = a1;
           }
           if (which) {
-            kind = ITEM_VALUE;
             L.side[lane] = side & ~which;
           } else if (gradient) {
             which = (1u << ISO_GRADS) - 1u;
@@ -787,9 +794,58 @@ template <int FIELD> struct IsoMarch {
         post(which, kind);
         continue;
       }
-      if (n_cell >= 16 || (starved && n_cell > 0)) {
-        // ------------------------------------------------ next macrocells
+      if (n_sides >= SIDES_AT || (starved && n_sides > 0 && n_sides >= n_cell)) {
+        // --------------------------- sides of a macrocell's sub-steps, ...
         uint32_t which = 0;
+        if (own == O_SIDES) {
+          const float t0 = L.t0[lane], t1 = L.t1[lane];
+          // a cell that begins where the last one's sub-steps ended knows its
+          // first value
+          uint32_t side = 0, over = 0, under = 0, open = ALL_SLOTS;
+          if (last_t == t0) {
+            L.value[0][lane] = last_f;
+            side = last_side;
+            over = last_f > iso || isnan(last_f) ? 1u : 0u;
+            under = last_f < iso || isnan(last_f) ? 1u : 0u;
+            open &= ~1u;
+          }
+          if (v.ufine) {
+            float2 g[ISO_SLOTS];
+#pragma unroll
+            for (int i = 0; i < ISO_SLOTS; i++) {
+              const v3 Q = place(lane, i == 0 ? t0 : at(i, t0, t1));
+              const float BNX_G *r = (const float BNX_G *)(v.ufine + seed_cell(v, Q));
+              g[i] = make_float2(r[1], r[2]);
+            }
+#pragma unroll
+            for (int i = 0; i < ISO_SLOTS; i++) {
+              const uint32_t bit = open & (1u << i);
+              if (bit != 0 && (g[i].x > iso || g[i].y < iso)) {
+                L.value[i][lane] = g[i].x > iso ? INFINITY : -INFINITY;
+                over |= g[i].x > iso ? bit : 0u;
+                under |= g[i].x > iso ? 0u : bit;
+                side |= bit;
+                open &= ~bit;
+              }
+            }
+          }
+          if (over == ALL_SLOTS || under == ALL_SLOTS) {
+            // no crossing
+            own = O_CELL;
+            last_t = at(ISO_SUBS, t0, t1);
+            last_f = L.value[ISO_SUBS][lane];
+            last_side = 1;
+          } else {
+            L.side[lane] = side;
+            own = O_WAIT;
+            which = open;
+          }
+        }
+        post(which, 0);
+        continue;
+      }
+      if (n_cell >= 16 || (starved && n_cell > 0)) {
+        // --------------------------------------- ... next macrocells, ...
         if (own == O_CELL) {
           if (D.over) {
             own = O_IDLE;
@@ -799,23 +855,14 @@ template <int FIELD> struct IsoMarch {
             n_cells++;
             if (c0 < fmn(c1, tmax)) {
               const float2 vr = v.ranges[ci];
-              if (iso >= vr.x && iso <= vr.y) which = (1u << ISO_SLOTS) - 1u;
-            }
-            if (which) {
-              L.t0[lane] = c0;
-              L.t1[lane] = c1;
-              L.side[lane] = 0;
-              // a cell that begins where the last one's sub-steps ended
-              // knows its first value
-              if (last_t == c0) {
-                L.value[0][lane] = last_f;
-                L.side[lane] = last_side;
-                which &= ~1u;
+              if (iso >= vr.x && iso <= vr.y) {
+                L.t0[lane] = c0;
+                L.t1[lane] = c1;
+                own = O_SIDES;
               }
             }
           }
         }
-        post(which, 0);
         continue;
       }
       if (items > 0 && (n_free >= 16 || n_free == 64)) {
@@ -838,17 +885,12 @@ template <int FIELD> struct IsoMarch {
           if (!TETS && !CELLS) {
             deliver(structured_sample(v, P));
           } else {
-            float4 g = make_float4(__int_as_float(-1), -INFINITY, INFINITY, 0.f);
-            if (v.ufine) g = v.ufine[seed_cell(v, P)];
-            if (!(it & (ITEM_GRADIENT | ITEM_VALUE)) && (g.y > iso || g.z < iso)) {
-              atomicOr(&L.side[owner], 1u << slot);
-              deliver(g.y > iso ? INFINITY : -INFINITY);
-            } else if (CELLS) {
+            if (CELLS) {
               code = 0;
               sp = 0;
               work = W_NODE;
             } else {
-              cur = __float_as_int(g.x);
+              cur = v.ufine ? __float_as_int(v.ufine[seed_cell(v, P)].x) : -1;
               walk = 0;
               work = cur >= 0 ? W_WALK : W_NODE;
             }
