@@ -608,7 +608,8 @@ template <int FIELD> struct March {
 // 1.8 requests beyond the L1 for each tet tested), so what helps is to ask for
 // fewer samples: 20.5M tets, 1024^2, 4 spp, isosurface and volume: 24.2 ms a
 // pass as nested loops, 16.7 with the samples dealt out, 13.5 with sides from
-// the fine grid, 12.3 with the owners' look; 14^3 mixed cells, 320x240, 2 spp:
+// the fine grid, 12.3 with the owners' look,
+// 10.8 without spills; 14^3 mixed cells, 320x240, 2 spp:
 // 41.6, 8.2, 6.6, 6.0.
 enum Owner { O_IDLE = 0, O_CELL, O_SIDES, O_WAIT };
 enum Worker { W_FREE = 0, W_WALK, W_NODE, W_TEST };
@@ -960,9 +961,14 @@ template <int FIELD> struct IsoMarch {
   }
 };
 
-// waves per SIMD each kernel is compiled for
-constexpr int march_waves(int field) { return field == FIELD_KIND_CELLS ? 3 : 5; }
-constexpr int iso_waves(int field) { return field == FIELD_KIND_CELLS ? 3 : 5; }
+// Waves per SIMD each kernel is compiled for: as many as their registers
+// allow without spills.  At five, the tet kernels spilled 15 and 31 and the
+// structured isosurface 5, stored and loaded again in every trip (20.5M tets,
+// 1024x1024, 4 spp: 12.3 ms a pass, 10.8 at four; 8^3 cubes of five tets,
+// 1920x1080, 2 spp: 7.8 and 7.2).  What scratch the tet kernels have left is
+// the stack of their few depth-first queries.
+constexpr int march_waves(int field) { return field == FIELD_KIND_CELLS ? 3 : field == FIELD_KIND_TETS ? 4 : 5; }
+constexpr int iso_waves(int field) { return field == FIELD_KIND_CELLS ? 3 : 4; }
 
 template <int FIELD>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves(FIELD)))) void k_volume_march(
