@@ -63,14 +63,19 @@ BNX_D bool finite(v3 a)
 }
 BNX_D v3 ld3(const float *p) { return v3{p[0], p[1], p[2]}; }
 
-// Correctly rounded reciprocal, quotient and square root for operands whose
-// results stay normal (|exponents| up to 100): the hardware estimate and one
-// or two fused corrections (Markstein, "Computation of elementary functions
-// on the IBM RISC System/6000 processor", 1990), 3, 3 more and 5
-// instructions where the general sequences, which also scale and fix up
-// operands at the ends of the range, take 10 to 15.  Compared with 1/b, a/b
-// and sqrtf on gfx950 over every float of those exponents: no bit differs.
-// b = 0 gives NaN where 1/b gives an infinity.
+// Correctly rounded reciprocal and quotient of normal floats whose results,
+// and the residual of the quotient (2^-24 of a), are normal too: the hardware
+// estimate and one or two fused corrections (rcp_step, div_step), 3 and 3 more
+// instructions where the general division, which also scales and fixes up
+// operands at the ends of the range, takes 10 to 15.  Callers see to the
+// range, |b| in [2^-100, 2^126) and a quotient in [2^-100, 2^100] or 0, or
+// divide.  Outside of it b = 0 gives NaN, and an estimate that over- or
+// underflows a NaN or a 0.
+// The reciprocal was compared with 1 / b on gfx950 for every mantissa at
+// exponents from -100 to 100: no bit differs.  From a reciprocal so rounded
+// div_step gives the rounded quotient (Markstein's theorem); it was compared
+// on 64 random numerators for each of those mantissas, and the host's form on
+// quotients next to a midpoint.
 BNX_D float rcp_rn(float b)
 {
   return bnx_num::rcp_step(b, __builtin_amdgcn_rcpf(b));
@@ -79,12 +84,6 @@ BNX_D float rcp_rn(float b)
 BNX_D float div_rn(float a, float b, float y)
 {
   return bnx_num::div_step(a, b, y);
-}
-BNX_D float sqrt_rn(float x)
-{
-  const float y = __builtin_amdgcn_rsqf(x);
-  const float g = x * y, h = .5f * y;
-  return __builtin_fmaf(h, __builtin_fmaf(-g, g, x), g);
 }
 
 // direction fix of traceRays.dev.cu:41-43 and rtcore/cuda/TraceInterface.h:37-39

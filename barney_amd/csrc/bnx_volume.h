@@ -415,10 +415,11 @@ template <int TYPE> BNX_D bool cell_invert(const float4 *V, v3 P, float tol, flo
     f = f - P;
     const float d = det3(cr, cs, ct);
     if (fabsf(d) < tol) return false;
-    const float y = rcp_rn(d);
-    const float d0 = div_rn(det3(f, cs, ct), d, y);
-    const float d1 = div_rn(det3(cr, f, ct), d, y);
-    const float d2 = div_rn(det3(cr, cs, f), d, y);
+    // both sides of each quotient in sixteenths (DET_SCALE)
+    const float den = d * bnx_num::DET_SCALE, y = rcp_rn(den);
+    const float d0 = div_rn(det3(f, cs, ct) * bnx_num::DET_SCALE, den, y);
+    const float d1 = div_rn(det3(cr, f, ct) * bnx_num::DET_SCALE, den, y);
+    const float d2 = div_rn(det3(cr, cs, f) * bnx_num::DET_SCALE, den, y);
     r = r - d0;
     s = s - d1;
     t = t - d2;

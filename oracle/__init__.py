@@ -84,6 +84,9 @@ def lib():
         L.orc_env_sample.argtypes = [vp, C.c_uint32, C.c_uint32, C.c_int, abi.fp, abi.fp, abi.fp]
         L.orc_env_uv_to_world.argtypes = [vp, abi.fp, C.c_int, abi.fp]
         L.orc_over_majorant_n.argtypes = [abi.fp, abi.fp, C.c_int, C.c_int, C.c_int, abi.fp]
+        L.orc_div_n.argtypes = [abi.fp, abi.fp, C.c_float, C.c_int, C.c_int, abi.fp]
+        L.orc_det_scale.restype = C.c_float
+        L.orc_rcp_n.argtypes = [abi.fp, C.c_int, C.c_int, abi.fp]
         L.orc_atan2_n.argtypes = [abi.fp, abi.fp, C.c_int, abi.fp]
         L.orc_acos_n.argtypes = [abi.fp, C.c_int, abi.fp]
         L.orc_env_frame.argtypes = [abi.fp, abi.fp, abi.fp, abi.fp]

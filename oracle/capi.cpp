@@ -740,23 +740,39 @@ int orc_cone_intersect_n(const float *rays, int n, const float *cone, float tmin
 }
 
 void orc_sincos(float x, float *s, float *c) { bnx_num::sincos(x, *s, *c); }
-// An estimate of 1 / b, `ulps` off the rounded one; where that overflows, or b
-// is subnormal, it is infinite, as the hardware's is
-static float rcp_estimate(float b, int ulps)
+// An estimate of 1 / b that is less than an ulp off: the rounded reciprocal
+// or (far) the float on the other side.  The ends of the range are taken at
+// their worst: infinite for a subnormal b, 0 where the reciprocal is subnormal.
+static float rcp_estimate(float b, int far)
 {
-  float y = std::fabs(b) < 0x1p-126f ? std::copysign(INFINITY, b) : 1.f / b;
-  for (int k = 0; k < std::abs(ulps) && std::isfinite(y); k++) y = std::nextafter(y, ulps > 0 ? INFINITY : -INFINITY);
-  return y;
+  if (std::fabs(b) > 0x1p126f) return std::copysign(0.f, b);
+  if (std::fabs(b) < 0x1p-126f) return std::copysign(INFINITY, b);
+  const float y = 1.f / b;
+  const double left = 1.0 / (double)b - (double)y;
+  return !far || left == 0.0 ? y : std::nextafter(y, left > 0.0 ? INFINITY : -INFINITY);
 }
 // x[i] over the majorant maj[i] as the march computes it; guard 0: without
 // its look at the majorant
-void orc_over_majorant_n(const float *x, const float *maj, int ulps, int guard, int n, float *out)
+void orc_over_majorant_n(const float *x, const float *maj, int far, int guard, int n, float *out)
 {
   for (int i = 0; i < n; i++) {
     const bool rn = !guard || bnx_num::short_majorant(maj[i]);
-    const float r = rn ? bnx_num::rcp_step(maj[i], rcp_estimate(maj[i], ulps)) : 0.f;
+    const float r = rn ? bnx_num::rcp_step(maj[i], rcp_estimate(maj[i], far)) : 0.f;
     out[i] = guard ? bnx_num::over_majorant(x[i], maj[i], r) : bnx_num::div_step(x[i], maj[i], r);
   }
+}
+// a[i] / b[i] from both times scale
+void orc_div_n(const float *a, const float *b, float scale, int far, int n, float *out)
+{
+  for (int i = 0; i < n; i++) {
+    const float d = b[i] * scale;
+    out[i] = bnx_num::div_step(a[i] * scale, d, bnx_num::rcp_step(d, rcp_estimate(d, far)));
+  }
+}
+float orc_det_scale() { return bnx_num::DET_SCALE; }
+void orc_rcp_n(const float *b, int far, int n, float *out)
+{
+  for (int i = 0; i < n; i++) out[i] = bnx_num::rcp_step(b[i], rcp_estimate(b[i], far));
 }
 void orc_atan2_n(const float *y, const float *x, int n, float *out)
 {

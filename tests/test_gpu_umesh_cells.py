@@ -7,6 +7,8 @@ isosurface over it -- primary IDs bit-exact, depth within 1e-5 relative,
 pixels within 1e-3, and the same rays and volume samples -- on a jittered
 mesh (non-planar faces: neighbouring cells overlap or leave gaps, where the
 first cell of the depth-first query decides) and on a planar-faced one."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -70,3 +72,25 @@ def test_cell_one_spp_parity(dev, orc, name, volume):
     assert st["rays"] == ost["rays"]
     assert st["volume_samples"] == ost["volume_samples"]
     fr.close()
+
+
+def test_cells_of_huge_determinants(dev, orc):
+    """cells some 2^42 across, whose Jacobian's determinants have no normal reciprocal"""
+    print("mixed cells 1spp of huge cells", flush=True)
+    us = scenes.mixed_volume(n=4, width=48, height=48, jitter=0.05, kinds=(scenes.CELL_HEX,))
+    scale = np.float32(4 * 5.0e12)
+    cells = (us.vertices * scale).astype(np.float32)
+    c = {k: tuple(float(x) * float(scale) for x in v) if k in ("position", "direction", "target") else v
+         for k, v in us.camera.items()}
+    us = dataclasses.replace(us, vertices=cells, base_density=us.base_density / float(scale), camera=c)
+    rend = abi.renderer(bg=us.bg_color, ambient=us.ambient)
+    frames = []
+    for side, o, scene in ((bx, dev, bx.UMeshWorld(dev, us)), (orc, None, orc.umesh_scene(us))):
+        cam = side.camera_perspective(c["position"], c["direction"], c["up"], c["fovy"])
+        fr = bx.Frame(dev, 48, 48) if o else orc.Frame(48, 48)
+        st = bx.render(scene.world, cam, rend, fr, 1) if o else orc.render(scene, cam, rend, fr, 1)[1]
+        frames.append((st["rays"], st["volume_samples"], fr.read(abi.BNX_FB_OBJID), fr.read(abi.BNX_FB_COLOR)))
+    g, r = frames
+    assert (r[2] == us.iso_user_id).sum() > 30 and (r[2] == us.user_id).sum() > 1000
+    assert g[0] == r[0] and g[1] == r[1] and np.array_equal(g[2], r[2])
+    assert np.abs(g[3] - r[3]).max() <= 1e-3
