@@ -212,9 +212,10 @@ struct GenTiming {
 };
 
 // Enqueue one generation over queue `cur`: upload the segments, build the
-// block maps, trace, volume march, shade into queue 1 - cur.  The caller
+// block maps, trace, volume march, shade into queue 1 - cur.  scattered: no
+// primary rays among them.  The caller
 // has uploaded the output region bases and cleared the output counters.
-int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool surfaces, bool volumes,
+int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool surfaces, bool volumes, bool scattered,
                        const MarchKind &march)
 {
   Queues &Q = F.Q;
@@ -238,7 +239,8 @@ int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool sur
   if (timed) BNX_HIP(hipEventRecord(Q.ev_end, dev->stream));
   if (volumes) {
     if (timed) BNX_HIP(hipEventRecord(Q.ev_vbegin, dev->stream));
-    if ((rc = launch_volume_march(dev, slots, sv, sl.n, sl.blocks256, in, trace, march, st)) != BNX_OK) return rc;
+    if ((rc = launch_volume_march(dev, slots, sv, sl.n, sl.blocks256, in, trace, scattered, march, st)) != BNX_OK)
+      return rc;
     if (timed) BNX_HIP(hipEventRecord(Q.ev_vend, dev->stream));
   }
   const SlotOut so{F.out_base.as<int>(), F.out_cnt.as<int>()};
@@ -287,8 +289,10 @@ int enqueue_dd(Device *dev, Wavefront &F, int cur0, int G, const BatchShape &b)
     RayQueue in = Q.q(cur), out = Q.q(1 - cur);
     TraceQueue tq{in.org, in.dir, in.hit, in.hit_v, in.rng, in.ps};
     if (trace && (rc = launch_trace_queue(dev, slots, sv, 1, blocks256, b.ext, tq, st)) != BNX_OK) return rc;
+    // a scattered generation has about half as many rays as the batch paths
+    const bool scattered = g > 0 && b.count0 > 2 * 256LL * SCATTERED_BLOCKS;
     if (b.volumes &&
-        (rc = launch_volume_march(dev, slots, sv, 1, blocks256, in, trace, b.march, st, at.march)) != BNX_OK)
+        (rc = launch_volume_march(dev, slots, sv, 1, blocks256, in, trace, scattered, b.march, st, at.march)) != BNX_OK)
       return rc;
     if ((rc = launch_shade(dev, slots, sv, blocks256, blocks1024, in, out, so, st, at.shade)) != BNX_OK) return rc;
   }
@@ -552,7 +556,7 @@ int render_frame_impl(World *w, const bnx_camera &cam, const bnx_renderer &rr, F
       SegList sl{F.h_segs.as<Segment>()};
       sl.add(0, 0, count, primary ? 64 : trace_refill_for(dev, w));
       if ((rc = zero_words(dev, F.out_cnt.ptr, 2 * sizeof(int), F.noalloc)) != BNX_OK) return rc;
-      if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, march)) != BNX_OK) return rc;
+      if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, !primary, march)) != BNX_OK) return rc;
       BNX_HIP(hipMemcpyAsync(hcnt, F.out_cnt.ptr, 2 * sizeof(int), hipMemcpyDeviceToHost, dev->stream));
       BNX_HIP(hipStreamSynchronize(dev->stream));
       if ((rc = collect_timing(F, count, traced, volumes, tm)) != BNX_OK) return rc;
@@ -1144,7 +1148,7 @@ struct Server {
                               F.Q.q(cur))) != BNX_OK)
         return rc;
     }
-    if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, march)) != BNX_OK) return rc;
+    if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, false, march)) != BNX_OK) return rc;
     int *hcnt = F.h_out_cnt.as<int>();
     BNX_HIP(hipMemcpyAsync(hcnt, F.out_cnt.ptr, sizeof(int) * 2 * max_slot, hipMemcpyDeviceToHost, dev->stream));
     BNX_HIP(hipStreamSynchronize(dev->stream));
@@ -1253,7 +1257,7 @@ struct Server {
       TraceQueue tq{in.org, in.dir, in.hit, in.hit_v, in.rng, in.ps};
       if (trace && (rc = launch_trace_queue(dev, slots, sv, nsegs, blocks256, cut, tq, stat)) != BNX_OK) return rc;
       if (volumes &&
-          (rc = launch_volume_march(dev, slots, sv, nsegs, blocks256, in, trace, march, stat, at.march)) != BNX_OK)
+          (rc = launch_volume_march(dev, slots, sv, nsegs, blocks256, in, trace, false, march, stat, at.march)) != BNX_OK)
         return rc;
       if ((rc = launch_shade(dev, slots, sv, blocks256, blocks1024, in, out, so, stat, at.shade)) != BNX_OK)
         return rc;

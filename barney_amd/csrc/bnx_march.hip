@@ -10,16 +10,16 @@
 // A ray's march is a nest of loops of data-dependent length (macrocells,
 // tentative collisions or sub-steps, the cells a point query tests).  Run as
 // nested loops, one ray per lane, a wave waits at every level for its slowest
-// lane.  So each lane here is a small state machine whose state says which
-// step its ray takes next (Mode): every trip a wave counts the lanes waiting
-// for each group of steps and takes one that enough of them wait for.  Rays
-// are set up 64 at a time, all lanes at work, and wait in LDS (those that
-// miss the field never leave the set-up); lanes whose rays have ended take
-// them from there.  Steps that follow each
-// other (a macrocell and the first collision in it; a value and the next
-// query's first tet) are one group, so that a lane passes through both in a
+// lane.  Where samples are cheap and rays run side by side that costs least
+// (k_volume_rays, structured fields).  Elsewhere each lane is a small state
+// machine whose state says which step its ray takes next (Mode): every trip a
+// wave counts the lanes waiting for each group of steps and takes one that
+// enough of them wait for.  Rays are set up 64 at a time, all lanes at work,
+// and wait in LDS (those that miss the field never leave the set-up); lanes
+// whose rays have ended take them from there.  A macrocell and the first
+// collision in it are one group, so that a lane passes through both in a
 // trip.  Every ray draws the same random numbers and takes the same steps in
-// the same order as in the nested form, so results do not change.
+// the same order in either form, so results do not change.
 //
 // One launch serves one program: isosurface k, or volume k, of every request
 // (isosurfaces first), clipped to the closest hit so far, which the launches
@@ -38,8 +38,7 @@ namespace {
 // lanes waiting for a step that make a wave take it (a wave with no fuller
 // group takes the fullest): the cheaper the step, the sooner.  A structured
 // field is sampled when three in eight of the lanes that have a ray wait for
-// it; a fixed 24 lanes made waves with few rays walk on to their slowest lane
-// (edit of a 97^3 volume, 333x217, 16 rays a wave: 307 us against 156).
+// it; a fixed 24 lanes made waves with few rays walk on to their slowest lane.
 constexpr int TAKE = 8;          // a new ray, already set up
 constexpr int SEED_AT = 4;       // a tet mesh's seed
 constexpr int CELL_AT = 12;      // a macrocell, where point queries are most of the work
@@ -272,12 +271,13 @@ BNX_D void each_segment(Claims &cl, const SlotDev *__restrict__ slots, const Ray
   }
 }
 
-// The volume march.  FIELD: the kind of field this kernel serves
-// (FIELD_KIND_*).  Bound by the gathers of the samples (structured: the eight
+// The volume march (of structured fields, the scattered generations of large
+// frames: k_volume_rays has the others).  FIELD: the kind of field this kernel
+// serves (FIELD_KIND_*).  Bound by the gathers of the samples (structured: the eight
 // corners of a cell in two loads of its corner copy; tets: a 128-byte record)
 // and by how many lanes a trip keeps at work.  With nested loops, one ray a
 // lane, a quarter to a third of the lanes were: 256^3 volume, 1024^2, 16 spp:
-// 3.65 ms a pass then, 1.92 now; edit of a 97^3 volume, 333x217: 171 us, 156.
+// 3.65 ms a pass then, 1.92 so.
 template <int FIELD> struct March {
   static constexpr bool TETS = FIELD == FIELD_KIND_TETS, CELLS = FIELD == FIELD_KIND_CELLS;
   static constexpr bool QUERY = TETS || CELLS;
@@ -1000,6 +1000,112 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(iso_waves(FI
   });
 }
 
+// The volume march of structured fields with one ray a lane from its begin to
+// its end, as nested loops.  What a lane waits for here are others' macrocells
+// and samples, but a step costs no vote and no state, a wave begins and ends
+// by itself, and the corner copy has made a sample one fetch: this is faster
+// than March in all launches but those of many rays that do not run side by
+// side (launch_volume_march).  A wave takes 64 rays, or 32 or 16 where the
+// launch would not fill half of the chip's waves: their loops end sooner.
+// March against this, us a frame: edits of 24^3, 128x96, 251 and 239; 48^3,
+// 205x492, 440 and 336; 200^3, 900x700, 655 and 520; frames of 64^3, 640x480, 2
+// spp, 505 and 365; 30^3, 1920x1080, 1250 and 1060; 256^3, 1024x1024, 4 spp, 1189
+// and 1148.  Six waves per SIMD (four and five within 1%, eight 6% slower).
+constexpr int RAYS_WAVES = 6;
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RAYS_WAVES))) void k_volume_rays(
+    const SlotDev *__restrict__ slots, SegView sv, RayQueue q, int k, int nsegs, int least, int fresh_launch,
+    unsigned long long *stats, Stamp stamp)
+{
+  if (blockIdx.x == 0 && threadIdx.x == 0) stamp_write(stamp);
+  // the generation's 256-ray blocks, each cut into 4, 8 or 16 waves' shares
+  // until there are `least` waves; the grid is as large as that can get
+  const Segment z = uniform_load((const Segment BNX_G *)(sv.segs + nsegs - 1));
+  const int blocks = z.block256 + (z.count + 255) / 256;
+  int shift = 2;
+  while (shift < 4 && (blocks << shift) < least) shift++;
+  const int blk = (int)blockIdx.x >> shift, per = 256 >> shift;
+  if (blk >= blocks) return;
+  const Segment sg =
+      uniform_load((const Segment BNX_G *)(sv.segs + __builtin_amdgcn_readfirstlane(sv.blk256[blk])));
+  const int local = (blk - sg.block256) * 256 + ((int)blockIdx.x - (blk << shift)) * per + (int)threadIdx.x;
+  const int i = sg.begin + local;
+  const SlotDev &SL = slots[sg.slot];
+  const bool fresh = fresh_launch != 0 && k == 0 && SL.num_isos == 0;
+  const bool valid = (int)threadIdx.x < per && local < sg.count;
+  if (k >= SL.num_vols) {
+    if (fresh && SL.num_vols == 0 && valid) q.hit[i] = make_int4(-1, -1, -1, 0);
+    return;
+  }
+  const VolumeDev v = uniform_load(SL.vols + k);
+  if (v.field != FIELD_KIND_STRUCTURED) return;
+  const bool last_vol = k + 1 == SL.num_vols, ratio_on = (SL.rr.flags & BNX_RENDER_RATIO_TRACKING) != 0;
+  uint32_t n_samples = 0, n_cells = 0;
+  if (valid) {
+    const float4 qo = q.org[i], qd = q.dir[i];
+    const bool shadow = (__float_as_uint(qd.w) & FLAG_SHADOW) != 0;
+    int prim = -1;
+    if (fresh) q.hit[i] = make_int4(-1, -1, -1, 0);
+    else prim = q.hit[i].x;
+    const v3 o = xyz(qo), d = fix_dir(xyz(qd));
+    const float tmax = qo.w;
+    const bool ratio = ratio_on && shadow, done = shadow && prim >= 0;   // an occluded shadow ray is done
+    float T = ratio && !done && k > 0 ? q.hit_v[i] : 1.f, at = 0.f, r0 = 0.f, r1 = tmax;
+    v3 c{0.f, 0.f, 0.f};
+    bool in = false, hit = false;
+    uint64_t rs = 0;
+    Dda D{};
+    if (!done && clip_bounds(v, o, d, r0, r1)) {
+      uint64_t parent = q.rng[i];
+      rs = parent;
+      rng_next(parent);
+      rng_next_h(rs, fnv3((uint32_t)v.rtc_inst, 0u, 0u));
+      q.rng[i] = parent;
+      in = dda_init(v, o, d, r1, D);
+    }
+    auto rnd = [&]() -> float { return (float)(rng_next(rs) & 0x00FFFFFFu) * (1.f / (float)0x01000000); };
+    while (in && !D.over && !hit) {
+      float c0, c1;
+      const int ci = dda_cell(v, D, c0, c1);
+      n_cells++;
+      const float maj = v.majorants[ci];
+      if (maj == 0.f) continue;
+      const float upper = fmn(c1, tmax), rmaj = v.rn && bnx_num::short_majorant(maj) ? rcp_rn(maj) : 0.f;
+      float t = c0;
+      while (!hit) {
+        const float r = rnd();
+        const float s = -fast_log(1.f - r);
+        t += bnx_num::over_majorant(s, maj, rmaj);
+        if (!(t < upper)) break;
+        const float f = structured_sample(v, o + t * d);
+        n_samples++;
+        const float4 m = isnan(f) ? make_float4(0.f, 0.f, 0.f, 0.f) : tf_map(v, f, rmaj > 0.f);
+        if (ratio) {
+          T *= fmx(0.f, 1.f - bnx_num::over_majorant(m.w, maj, rmaj));
+          hit = T == 0.f;
+          at = tmax;
+        } else if (m.w >= rnd() * maj) {
+          hit = true;
+          at = t;
+          c = v3{m.x, m.y, m.z};
+        }
+      }
+    }
+    if (hit) {
+      q.org[i].w = at;
+      q.hit[i] = make_int4(0, VOLUME_GEOM_BASE + k, v.rtc_inst, 0);
+      q.vcol[i] = make_float4(c.x, c.y, c.z, 0.f);
+    } else if (ratio && !done) {
+      if (!last_vol) q.hit_v[i] = T;
+      else if (T < 1.f) q.ps[i].w = __float_as_uint(__uint_as_float(q.ps[i].w) * T);
+    }
+  }
+  const uint32_t a = wave_sum(n_samples), b = wave_sum(n_cells);
+  if (lane_id() == 0) {
+    stat_add(stats, STAT_SAMPLES, a);
+    stat_add(stats, STAT_CELLS, b);
+  }
+}
+
 using MarchKernel = void (*)(const SlotDev *, SegView, RayQueue, int, int, int, int, unsigned long long *, Stamp);
 const MarchKernel KERNELS[2][FIELD_KINDS] = {
     {k_volume_march<FIELD_KIND_STRUCTURED>, k_volume_march<FIELD_KIND_TETS>, k_volume_march<FIELD_KIND_CELLS>},
@@ -1008,8 +1114,8 @@ const MarchKernel KERNELS[2][FIELD_KINDS] = {
 } // namespace
 
 int launch_volume_march(Device *dev, const SlotDev *slots, const SegView &sv, int nsegs, int blocks256,
-                        const RayQueue &q, bool surfaces, const MarchKind &kind, unsigned long long *stats,
-                        const Stamp &stamp)
+                        const RayQueue &q, bool surfaces, bool scattered, const MarchKind &kind,
+                        unsigned long long *stats, const Stamp &stamp)
 {
   if (blocks256 <= 0 || nsegs <= 0) return BNX_OK;
   int launch = 0;
@@ -1018,6 +1124,15 @@ int launch_volume_march(Device *dev, const SlotDev *slots, const SegView &sv, in
     const int k = iso ? p : p - kind.isos;
     for (int f = 0; f < FIELD_KINDS; f++) {
       if (!(kind.fields & (1 << f))) continue;
+      if (!iso && f == FIELD_KIND_STRUCTURED && (!scattered || blocks256 < SCATTERED_BLOCKS)) {
+        // half of the resident waves; a grid of fewer than that many shares
+        // is cut again, into less than twice as many
+        const int least = 2 * RAYS_WAVES * dev->num_cus;
+        k_volume_rays<<<std::max(4 * blocks256, std::min(16 * blocks256, 2 * least)), 64, 0, dev->stream>>>(
+            slots, sv, q, k, nsegs, least, surfaces ? 0 : 1, stats, launch == 0 ? stamp : Stamp{});
+        launch++;
+        continue;
+      }
       const MarchKernel kernel = KERNELS[iso ? 1 : 0][f];
       // as many waves as are resident at once, in whole rounds of the groups,
       // and no more than there are chunks of 16 rays

@@ -45,6 +45,37 @@ def test_ray_counts(dev, orc, w, h, flags):
     _compare(dev, orc, vs, bx.VolumeWorld(dev, vs).world, orc.volume_scene(vs), 1, flags)
 
 
+@pytest.mark.parametrize("flags", [0, abi.BNX_RENDER_RATIO_TRACKING])
+def test_scattered_generations(dev, flags):
+    """the later generations of a frame of some millions of rays, which another kernel marches, against the same
+    frame in batches below that"""
+    print(f"march scattered generations flags={flags}", flush=True)
+    w, h, spp = 1000, 900, 9
+    vs = scenes.config2(n=33, mc_grid=8, width=w, height=h)
+    world, c = bx.VolumeWorld(dev, vs).world, vs.camera
+    cam = bx.camera_perspective(c["position"], c["direction"], c["up"], 22.0)
+    rend = abi.renderer(bg=vs.bg_color, ambient=vs.ambient, flags=flags)
+    tuning, frames, stats = dev.tuning(), [bx.Frame(dev, w, h) for _ in range(3)], []
+    try:
+        for fr, t in zip(frames, ({}, dict(render_paths=1 << 20, graph_paths=0),
+                                  dict(render_paths=1 << 24, graph_paths=1 << 24))):
+            dev.set_tuning(**t)
+            for _ in range(2):          # the second time a captured loop, if there is one
+                fr.reset()
+                stats.append(bx.render(world, cam, rend, fr, spp))
+    finally:
+        dev.set_tuning(**tuning)
+    assert stats[0]["rays"] - w * h * spp > 2 << 21
+    for st in stats[1:]:
+        assert st["rays"] == stats[0]["rays"] and st["volume_samples"] == stats[0]["volume_samples"]
+    for ch in (abi.BNX_FB_COLOR, abi.BNX_FB_DEPTH, abi.BNX_FB_OBJID, abi.BNX_FB_NORMAL):
+        a, *others = [fr.read(ch) for fr in frames]
+        for b in others:
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), ch
+    for fr in frames:
+        fr.close()
+
+
 @pytest.mark.parametrize("n,flags", [(2, 0), (11, 0), (11, abi.BNX_RENDER_RATIO_TRACKING)])
 def test_many_volumes(dev, orc, n, flags):
     print(f"march of {n} volumes flags={flags}", flush=True)
