@@ -27,16 +27,20 @@ template <typename T> BNX_D T uniform_load(const T BNX_G *p)
 }
 
 // How the waves of a launch share its rays.  The generation's blocks of 256
-// rays, each inside one segment, are cut into up to 16 chunks each until there
-// are `least` chunks (so that a small generation still has some for every
-// wave) and dealt to CLAIM_GROUPS
+// rays, each inside one segment, are cut into chunks: down to 64 rays until
+// there are `balance` (a wave's first chunk is its own, and what no chunk is
+// left for is time that waves with short rays wait for those with long ones),
+// and down to 16 until there are `least` (so that a small generation still has
+// some for every wave).  They are dealt to CLAIM_GROUPS
 // groups of waves; a wave starts on a chunk of its own and then takes its
 // group's next one from the group's counter, or another group's once its own
 // is out.  One counter for all waves would be in the way: its atomics are
 // served one after the other beyond the XCDs' caches (14 ns each, 3.4
 // against 2.4 ms on the 256^3 volume).  Shares fixed beforehand would leave
 // the waves with the long rays behind (isosurface of 20.5M tets: 19.6
-// against 12.9 ms).
+// against 12.9 ms), and so do chunks as large as the waves are many: 82k
+// triangles, 900x600, 2 spp, traces in 4219 chunks on 5120 waves, 1.92 ms a
+// frame, and 1.57 in 16876; tets of 80^3 cubes, 1024x768, 2 spp, 5.77 and 3.99.
 struct Claims {
   const Segment *segs;
   const int *blk;              // segment of each 256-ray block
@@ -48,19 +52,19 @@ struct Claims {
   int base, next, stop;        // [next, stop) is in hand, segment-local, from queue index base
   bool dry;                    // none left in this segment
 
-  BNX_D void begin(const SegView &sv, int nsegs, int program, int least)
+  BNX_D void begin(const SegView &sv, int nsegs, int program, int least, int balance)
   {
     segs = sv.segs;
     blk = sv.blk256;
     const Segment z = uniform_load((const Segment BNX_G *)(segs + nsegs - 1));
-    deal(z.block256 + (z.count + 255) / 256, sv.claims + program * CLAIM_GROUPS * CLAIM_STRIDE, least);
+    deal(z.block256 + (z.count + 255) / 256, sv.claims + program * CLAIM_GROUPS * CLAIM_STRIDE, least, balance);
   }
   // n rays without segments
   BNX_D void begin(int n, int *counters, int least)
   {
     segs = nullptr;
     blk = nullptr;
-    deal((n + 255) / 256, counters, least);
+    deal((n + 255) / 256, counters, least, 0);
     seg = first = base = 0;
     total = n;
     dry = chunk < 0;
@@ -68,11 +72,12 @@ struct Claims {
     if (!dry) range();
     refill();
   }
-  BNX_D void deal(int blocks, int *counters, int least)
+  BNX_D void deal(int blocks, int *counters, int least, int balance)
   {
     ctr = counters;
     waves = (int)gridDim.x;
     shift = 0;
+    while (shift < 2 && (blocks << shift) < balance) shift++;
     while (shift < 4 && (blocks << shift) < least) shift++;
     per = 256 >> shift;
     chunks = blocks << shift;

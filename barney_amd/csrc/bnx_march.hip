@@ -39,6 +39,7 @@ namespace {
 // group takes the fullest): the cheaper the step, the sooner.  A structured
 // field is sampled when three in eight of the lanes that have a ray wait for
 // it; a fixed 24 lanes made waves with few rays walk on to their slowest lane.
+constexpr int BALANCE = 4;       // chunks a wave, where there are as many rays
 constexpr int TAKE = 8;          // a new ray, already set up
 constexpr int SEED_AT = 4;       // a tet mesh's seed
 constexpr int CELL_AT = 12;      // a macrocell, where point queries are most of the work
@@ -979,7 +980,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(march_waves(
   __shared__ uint32_t ready[READY * 64];
   __shared__ uint32_t ring[FIELD == FIELD_KIND_CELLS ? PQ_SHORT * 64 : 1];
   Claims cl;
-  cl.begin(sv, nsegs, program, (int)gridDim.x);
+  cl.begin(sv, nsegs, program, (int)gridDim.x, BALANCE * (int)gridDim.x);
   each_segment(cl, slots, q, k, fresh != 0, false, [&](const SlotDev &SL, bool f) -> bool {
     return March<FIELD>::run(cl, SL, q, k, f, stats, ready, ring);
   });
@@ -994,7 +995,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(iso_waves(FI
   __shared__ IsoShared L;
   __shared__ uint32_t ring[FIELD == FIELD_KIND_CELLS ? PQ_SHORT * 64 : 1];
   Claims cl;
-  cl.begin(sv, nsegs, program, (int)gridDim.x);
+  cl.begin(sv, nsegs, program, (int)gridDim.x, BALANCE * (int)gridDim.x);
   each_segment(cl, slots, q, k, fresh != 0, true, [&](const SlotDev &SL, bool f) -> bool {
     return IsoMarch<FIELD>::run(cl, SL, q, k, f, stats, L, ring);
   });

@@ -56,6 +56,10 @@ constexpr int TB = 256;        // threads per block
 // to a private array, STACK_CAP entries in all whatever SH is
 constexpr int STACK_CAP = 192;
 constexpr int API_SHORT = 16;  // the ray-array entry point's ring
+// Chunks a wave of a frame's trace, where there are as many rays: pixels next
+// to each other differ by what they see.  (An array's rays are dealt without:
+// a million random any-hit rays, 314 us so and 345 in chunks of 128.)
+constexpr int BALANCE = 2;
 constexpr int TAKE = 16;       // idle lanes that make a wave take new rays
 
 struct HitRec {
@@ -806,7 +810,7 @@ BNX_D void trace_waves(const SlotDev *__restrict__ slots, const SegView &sv, int
                        unsigned long long *counters, uint32_t *ring)
 {
   Claims cl;
-  cl.begin(sv, nsegs, CLAIMS_TRACE, least_chunks(EXT));
+  cl.begin(sv, nsegs, CLAIMS_TRACE, least_chunks(EXT), BALANCE * (int)gridDim.x);
   Counts cnt{0, 0, 0};
   while (cl.chunk >= 0) {
     const Segment sg = cl.open();
