@@ -77,11 +77,12 @@ struct BatchShape {
   int refill = 64, stack = 16, walk = 0, blocks_per_cu = 8, shade_block = 256;
   bool ext = false;   // the trace kernels with the cylinder test and the cut plane
   bool xf = false;    // the trace kernels that change the ray's frame at instances
+  bool few = false;   // few_prims
   bool operator<(const BatchShape &o) const
   {
-    return std::tie(count0, cap, surfaces, volumes, march.fields, march.isos, march.vols, refill, stack, walk, blocks_per_cu, shade_block, ext, xf) <
+    return std::tie(count0, cap, surfaces, volumes, march.fields, march.isos, march.vols, refill, stack, walk, blocks_per_cu, shade_block, ext, xf, few) <
            std::tie(o.count0, o.cap, o.surfaces, o.volumes, o.march.fields, o.march.isos, o.march.vols, o.refill, o.stack, o.walk, o.blocks_per_cu,
-                    o.shade_block, o.ext, o.xf);
+                    o.shade_block, o.ext, o.xf, o.few);
   }
 };
 
@@ -212,11 +213,11 @@ struct GenTiming {
 };
 
 // Enqueue one generation over queue `cur`: upload the segments, build the
-// block maps, trace, volume march, shade into queue 1 - cur.  scattered: no
-// primary rays among them.  The caller
+// block maps, trace, volume march, shade into queue 1 - cur.  few: the worlds
+// have few primitives (few_prims); scattered: no primary rays among the rays.  The caller
 // has uploaded the output region bases and cleared the output counters.
-int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool surfaces, bool volumes, bool scattered,
-                       const MarchKind &march)
+int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool surfaces, bool volumes, bool few,
+                       bool scattered, const MarchKind &march)
 {
   Queues &Q = F.Q;
   RayQueue in = Q.q(cur), out = Q.q(1 - cur);
@@ -234,7 +235,7 @@ int enqueue_generation(Device *dev, Wavefront &F, int cur, SegList &sl, bool sur
   bool cut = false;
   const SlotDev *hs = F.h_slots.as<SlotDev>();
   for (int k = 0; k < sl.n; k++) cut = cut || has_cut_plane(hs[sl.v[k].slot].rr);
-  if (trace && (rc = launch_trace_queue(dev, slots, sv, sl.n, sl.blocks256, cut, tq, st)) != BNX_OK)
+  if (trace && (rc = launch_trace_queue(dev, slots, sv, sl.n, sl.blocks256, cut, few, tq, st)) != BNX_OK)
     return rc;
   if (timed) BNX_HIP(hipEventRecord(Q.ev_end, dev->stream));
   if (volumes) {
@@ -288,7 +289,7 @@ int enqueue_dd(Device *dev, Wavefront &F, int cur0, int G, const BatchShape &b)
       return rc;
     RayQueue in = Q.q(cur), out = Q.q(1 - cur);
     TraceQueue tq{in.org, in.dir, in.hit, in.hit_v, in.rng, in.ps};
-    if (trace && (rc = launch_trace_queue(dev, slots, sv, 1, blocks256, b.ext, tq, st)) != BNX_OK) return rc;
+    if (trace && (rc = launch_trace_queue(dev, slots, sv, 1, blocks256, b.ext, b.few, tq, st)) != BNX_OK) return rc;
     // a scattered generation has about half as many rays as the batch paths
     const bool scattered = g > 0 && b.count0 > 2 * 256LL * SCATTERED_BLOCKS;
     if (b.volumes &&
@@ -386,6 +387,19 @@ int trace_refill_for(const Device *dev, const World *w)
 }
 
 namespace {
+
+// Many rays in a world of few primitives: a walk is short, a launch's waves
+// are many more than are resident at once, and sharing rays out among those
+// that are costs more than it gives.  Such batches keep one ray per thread
+// (trace_walk 1).  us a frame, waves and a ray a thread: 484 spheres and 80
+// triangles, 1280x720, 860 and 733; 21k primitives, 1920x1080, 2 spp, 2592 and
+// 2297; 30k, 1024x768, 8 spp, 6124 and 6776; 1.3k, 400x300, 330 and 333 and, with
+// 1,000 spheres, 200x150, 360 and 401.
+constexpr long long FEW_PRIMS = 3 << 13, FEW_PATHS = 1 << 19;
+bool few_prims(const World *w, long long paths)
+{
+  return paths >= FEW_PATHS && w->instances->blas_prims + (long long)w->instances->groups.size() < FEW_PRIMS;
+}
 
 // march: what the world's rays have to be marched through
 int fill_slot(World *w, const bnx_camera &cam, const bnx_renderer &rr, Frame *f, SlotDev &s, MarchKind &march)
@@ -495,7 +509,7 @@ int render_frame_impl(World *w, const bnx_camera &cam, const bnx_renderer &rr, F
     const BatchShape shape{np * nS,          2 * np * nS,           surfaces,
                            volumes,          march,                 trace_refill_for(dev, w),
                            dev->trace_stack_lds, dev->trace_walk, dev->trace_blocks_per_cu, dev->shade_block,
-                           ext_kernels(dev, has_cut_plane(rr)), dev->xf_worlds > 0};
+                           ext_kernels(dev, has_cut_plane(rr)), dev->xf_worlds > 0, few_prims(w, np * nS)};
     int dd_gens = 0;
     if (dd) {
       auto it = F.gens_seen.find(shape);
@@ -556,7 +570,7 @@ int render_frame_impl(World *w, const bnx_camera &cam, const bnx_renderer &rr, F
       SegList sl{F.h_segs.as<Segment>()};
       sl.add(0, 0, count, primary ? 64 : trace_refill_for(dev, w));
       if ((rc = zero_words(dev, F.out_cnt.ptr, 2 * sizeof(int), F.noalloc)) != BNX_OK) return rc;
-      if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, !primary, march)) != BNX_OK) return rc;
+      if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, shape.few, !primary, march)) != BNX_OK) return rc;
       BNX_HIP(hipMemcpyAsync(hcnt, F.out_cnt.ptr, 2 * sizeof(int), hipMemcpyDeviceToHost, dev->stream));
       BNX_HIP(hipStreamSynchronize(dev->stream));
       if ((rc = collect_timing(F, count, traced, volumes, tm)) != BNX_OK) return rc;
@@ -1148,7 +1162,7 @@ struct Server {
                               F.Q.q(cur))) != BNX_OK)
         return rc;
     }
-    if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, false, march)) != BNX_OK) return rc;
+    if ((rc = enqueue_generation(dev, F, cur, sl, surfaces, volumes, false, false, march)) != BNX_OK) return rc;
     int *hcnt = F.h_out_cnt.as<int>();
     BNX_HIP(hipMemcpyAsync(hcnt, F.out_cnt.ptr, sizeof(int) * 2 * max_slot, hipMemcpyDeviceToHost, dev->stream));
     BNX_HIP(hipStreamSynchronize(dev->stream));
@@ -1255,7 +1269,7 @@ struct Server {
       const GenStamps at(F.stamps.as<unsigned long long>() + 4 * g, trace, volumes);
       if ((rc = launch_segment_blocks(dev, sv, nsegs, blocks256, blocks1024, at.first)) != BNX_OK) return rc;
       TraceQueue tq{in.org, in.dir, in.hit, in.hit_v, in.rng, in.ps};
-      if (trace && (rc = launch_trace_queue(dev, slots, sv, nsegs, blocks256, cut, tq, stat)) != BNX_OK) return rc;
+      if (trace && (rc = launch_trace_queue(dev, slots, sv, nsegs, blocks256, cut, false, tq, stat)) != BNX_OK) return rc;
       if (volumes &&
           (rc = launch_volume_march(dev, slots, sv, nsegs, blocks256, in, trace, false, march, stat, at.march)) != BNX_OK)
         return rc;

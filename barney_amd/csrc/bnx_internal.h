@@ -257,9 +257,9 @@ struct SlotDev;
 struct SegView;
 // trace every ray of the generation's nsegs segments (blocks256 blocks of 256
 // rays); cut: a request in the launch has a cut plane (the launch then takes
-// the kernels that apply it)
+// the kernels that apply it); few: many rays in a world of few primitives
 int launch_trace_queue(Device *dev, const SlotDev *d_slots, const SegView &sv, int nsegs, int blocks256, bool cut,
-                       const TraceQueue &q, unsigned long long *counters);
+                       bool few, const TraceQueue &q, unsigned long long *counters);
 // whether a trace launch takes the extended kernels (cylinder test, cut
 // plane, stochastic opacity): a built world holds cylinders or translucent
 // triangles, or a request of the launch has a cut plane

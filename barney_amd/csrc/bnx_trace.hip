@@ -910,11 +910,12 @@ int launch_trace_api(Group *g, const bnx_ray *d_rays, int n, bnx_hit *d_hits, ui
 }
 
 int launch_trace_queue(Device *dev, const SlotDev *slots, const SegView &sv, int nsegs, int blocks256, bool cut,
-                       const TraceQueue &q, unsigned long long *counters)
+                       bool few, const TraceQueue &q, unsigned long long *counters)
 {
   if (blocks256 <= 0) return BNX_OK;
   const int sh = dev->trace_stack_lds;
-  const bool ext = ext_kernels(dev, cut), xf = dev->xf_worlds > 0, spec = dev->trace_walk == 1;
+  const bool ext = ext_kernels(dev, cut), xf = dev->xf_worlds > 0;
+  const bool spec = dev->trace_walk == 1 || (few && !ext);
   const TraceKernel kernel = sh == 8    ? trace_kernel<8>(spec, ext, xf)
                              : sh == 32 ? trace_kernel<32>(spec, ext, xf)
                                         : trace_kernel<16>(spec, ext, xf);

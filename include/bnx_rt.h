@@ -426,9 +426,13 @@ typedef struct bnx_tuning {
   int32_t trace_refill;             /* idle lanes that make a trace wave take new
                                        rays, 1..64 (64: as for other worlds)         */
   int32_t trace_walk;               /* 0 = waves that take new rays as walks end, a
-                                       node step or a leaf per trip; 1 = one ray per
-                                       thread, speculative while-while (leaves set
-                                       aside until every lane has one)               */
+                                       node step or a leaf per trip (but 1 for a
+                                       batch of bnx_render with 2^19 paths or more
+                                       in a world of fewer than 3 * 2^13 primitives
+                                       and instances, where none needs the extended
+                                       kernels); 1 = one ray per thread,
+                                       speculative while-while (leaves set aside
+                                       until every lane has one)                     */
   int32_t sort_rays;                /* bnx_render: 1 = reorder each secondary
                                        generation of 2^16 rays or more by shadow
                                        flag, direction octant and origin Morton

@@ -10,7 +10,8 @@ import threading
 import numpy as np
 import pytest
 
-from barney_amd import scenes
+import barney_amd as bx
+from barney_amd import abi, scenes
 from tests import helpers
 
 pytestmark = pytest.mark.gpu
@@ -91,6 +92,38 @@ def test_flat_instances(dev, orc, ext, flat):
     g = spec.gpu(dev)
     _same(g.trace(rays), want)
     assert np.array_equal(g.trace(rays, any_hit=True)["prim_id"] >= 0, hit)
+
+
+@pytest.mark.parametrize("kind", ["plain", "cylinders", "volume"])
+def test_many_rays_few_primitives(dev, kind):
+    """a batch that keeps one ray per thread against the same frame in batches too small for that"""
+    print(f"trace waves few primitives {kind}", flush=True)
+    w, h = 653, 461
+    sc = scenes.config1(width=w, height=h)
+    if kind == "cylinders":
+        sc.cylinders.append(scenes.sticks(300))
+    world, c = bx.SurfaceWorld(dev, sc), sc.camera
+    if kind == "volume":
+        vs = scenes.config2(n=17, mc_grid=4, width=w, height=h)
+        vol = bx.Volume(dev, vs)
+        world.world.add_volume(vol, 3)
+    cam = bx.camera_perspective(c["position"], c["direction"], c["up"], c["fovy"])
+    rend = abi.renderer(bg=sc.bg_color, ambient=sc.ambient)
+    tuning, frames, stats = dev.tuning(), [bx.Frame(dev, w, h) for _ in range(3)], []
+    assert w * h < 1 << 19 <= 2 * w * h
+    try:
+        for fr, t in zip(frames, ({}, dict(graph_paths=0), dict(render_paths=1 << 18))):
+            dev.set_tuning(**t)
+            stats.append(bx.render(world.world, cam, rend, fr, 2))
+    finally:
+        dev.set_tuning(**tuning)
+    assert len({st["rays"] for st in stats}) == 1
+    for ch in (abi.BNX_FB_COLOR, abi.BNX_FB_DEPTH, abi.BNX_FB_PRIMID, abi.BNX_FB_INSTID, abi.BNX_FB_NORMAL):
+        a, *others = [fr.read(ch) for fr in frames]
+        for b in others:
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), ch
+    for fr in frames:
+        fr.close()
 
 
 def test_threads(dev, orc):
