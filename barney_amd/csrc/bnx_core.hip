@@ -122,6 +122,7 @@ template <typename T> int upload(Device *dev, DevMem &m, const T *host, size_t c
 int build_blas(Group *g)
 {
   Device *dev = g->dev;
+  const BuildScope scope(dev->build);
   std::vector<GeomBuild> gb;
   int n = 0;
   for (Geom *geom : g->geoms) {
@@ -248,6 +249,7 @@ __global__ void k_enter(const int *order, const InstDev *insts, const BlasDev *b
 int build_tlas(Group *g)
 {
   Device *dev = g->dev;
+  const BuildScope scope(dev->build);
   // the group is rebuilt in place: it counts as unbuilt (traces, renders and
   // new worlds refuse it) until every step below, the stack-depth check
   // included, has succeeded
@@ -1123,6 +1125,7 @@ int bnx_bvh_build_boxes(bnx_device d, const float *d_boxes, int n, int max_leaf,
   GUARD_BEGIN
   BNX_CHECK(d && (n == 0 || d_boxes) && n >= 0 && max_leaf >= 1 && max_leaf <= 7, BNX_ERR_INVALID,
             "bnx_bvh_build_boxes: bad argument");
+  const BuildScope scope(d->build);
   DevMem &lo = d->build.box_lo, &hi = d->build.box_hi;
   BNX_HIP(lo.ensure(sizeof(float4) * (size_t)(n ? n : 1)));
   BNX_HIP(hi.ensure(sizeof(float4) * (size_t)(n ? n : 1)));

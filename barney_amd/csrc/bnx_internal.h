@@ -84,11 +84,29 @@ struct Device;
 
 // scratch arrays of the BVH builder, kept per device and grown on demand:
 // the boxes being built over (box_lo, box_hi) with their second copy, the
-// primitives' geometries, and the builder's tables
+// primitives' geometries, and the builder's tables.  Kept from build to build
+// up to KEEP bytes (builds of about ten million primitives); a build that
+// needed more gives all of it back when it ends (BuildScope), which takes it
+// some tenths of a millisecond per million primitives.
 struct BuildScratch {
+  static constexpr size_t KEEP = (size_t)1 << 30;
   DevMem box_lo, box_hi, geoms, pgeom;
   DevMem lo, hi, slot_task, windows, tasks, task_node, bounds, bins, split, mid_tasks, counters;
   DevMem collapse, levels;
+  void trim()
+  {
+    DevMem *const all[] = {&box_lo, &box_hi, &geoms, &pgeom, &lo, &hi, &slot_task, &windows, &tasks, &task_node,
+                           &bounds, &bins, &split, &mid_tasks, &counters, &collapse, &levels};
+    size_t total = 0;
+    for (const DevMem *m : all) total += m->bytes;
+    if (total > KEEP)
+      for (DevMem *m : all) m->release();
+  }
+};
+struct BuildScope {
+  BuildScratch &scratch;
+  explicit BuildScope(BuildScratch &s) : scratch(s) {}
+  ~BuildScope() { scratch.trim(); }
 };
 
 struct Device {

@@ -661,6 +661,7 @@ int volume_build_umesh(Volume *v, const int4 *tets4, const int4 *ext4, const uin
   VolumeDev &d = v->dd;
   hipStream_t st = dev->stream;
   const bool mixed = types != nullptr;
+  const BuildScope scope(dev->build);
   DevMem verts, tets, ext, typ, rlo, rhi;
   DevMem &lo = dev->build.box_lo, &hi = dev->build.box_hi;
   BNX_HIP(verts.ensure(sizeof(float4) * (size_t)nvert));

@@ -2,10 +2,11 @@
 sizes around the block-built task size (1024) and its multiples, boxes in an
 order that puts whole waves into one bin, clusters that split off a few
 primitives at a time, equal centroids (median splits through both phases),
-and every leaf size the entry point takes.  Trees are compared node for node,
+every leaf size the entry point takes, and the scratch that stays.  Trees are compared node for node,
 orders slot for slot."""
 import numpy as np
 import pytest
+import torch
 
 import barney_amd as bx
 from tests import helpers
@@ -42,3 +43,19 @@ def test_builder_phases(dev, orc, kind, n, leaf):
     assert np.array_equal(go, oo)
     assert helpers.canonical_bvh(gn, go, leaf) == helpers.canonical_bvh(on, oo, leaf)
     assert ginfo.max_depth == od and ginfo.num_nodes == len(on)
+
+
+def test_large_builds_give_their_scratch_back(dev):
+    """20M boxes need some 1.6 GB of scratch; of that no more than 1 GiB may stay"""
+    print("builder scratch of 20M boxes", flush=True)
+    bx.bvh_build_boxes(dev, _boxes("random", 5000, 1), 4)
+    before = torch.cuda.mem_get_info(0)[0]
+    r = np.random.default_rng(5)
+    c = r.random((20 << 20, 3), np.float32)
+    _, _, info = bx.bvh_build_boxes(dev, np.concatenate([c, c + np.float32(.001)], 1), 4)
+    assert info.num_nodes > 5 << 20
+    assert before - torch.cuda.mem_get_info(0)[0] < (1024 + 64) << 20
+    # and the next build has its scratch again
+    boxes = _boxes("random", 3000, 2)
+    a, b = bx.bvh_build_boxes(dev, boxes, 4), bx.bvh_build_boxes(dev, boxes, 4)
+    assert np.array_equal(a[1], b[1]) and helpers.canonical_bvh(a[0], a[1], 4) == helpers.canonical_bvh(b[0], b[1], 4)
