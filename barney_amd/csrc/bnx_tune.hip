@@ -1,8 +1,8 @@
 // bnx_tune.hip -- launch tuning of the render path (include/bnx_rt.h,
 // bnx_tuning) and its autotuner: coordinate descent over the raygen tile,
 // the LDS share of the traversal stack, the walk order, the reordering of
-// secondary rays, the shade block size, the pooled trace's refill threshold
-// and launch size, bnx_render's paths per batch and the largest batch run as
+// secondary rays, the shade block size, the trace's refill threshold and
+// launch size, bnx_render's paths per batch and the largest batch run as
 // a captured bounce loop, each candidate timed on
 // probe renders of the caller's request shape.  Host code only.
 #include "bnx_internal.h"
@@ -192,8 +192,10 @@ int bnx_autotune(bnx_world world, const bnx_camera *camera, const bnx_renderer *
   const std::vector<int> onoff = {0, 1};
   const std::vector<int> shade_blocks = {1024, 256};
   const std::vector<std::pair<int, int>> stack_walks = {{8, 0}, {16, 0}, {32, 0}, {8, 1}, {16, 1}, {32, 1}};
-  const std::vector<int> refills = {64, 32, 16, 8, 4};
-  const std::vector<int> blocks = {2, 4, 8, 16};
+  // values that differ from the trace's own: it refills at 16 idle lanes, and
+  // its 20 resident waves per CU (five per SIMD) are five blocks
+  const std::vector<int> refills = {64, 32, 8, 4};
+  const std::vector<int> blocks = {2, 3, 4};
   const std::vector<long long> paths = {2LL << 20, 4LL << 20, 8LL << 20, 16LL << 20};
   const std::vector<long long> graphs = {0LL, 1LL << 20, 4LL << 20, 16LL << 20};
   const long long prims = w->instances->blas_prims;
@@ -214,8 +216,9 @@ int bnx_autotune(bnx_world world, const bnx_camera *camera, const bnx_renderer *
     if (rc == BNX_OK) rc = sweep([](bnx_tuning &t, int v) { t.sort_rays = v; }, onoff);
     if (rc == BNX_OK) rc = sweep([](bnx_tuning &t, int v) { t.shade_block = v; }, shade_blocks);
     // the refill threshold of secondary rays for worlds of this size: 64
-    // keeps the trace's own
-    if (rc == BNX_OK)
+    // keeps the trace's own.  Both fields are the sharing waves'.
+    const bool waves = best.trace_walk == 0;
+    if (rc == BNX_OK && waves)
       rc = sweep(
           [prims, &start](bnx_tuning &t, int v) {
             if (v >= 64) {
@@ -227,8 +230,7 @@ int bnx_autotune(bnx_world world, const bnx_camera *camera, const bnx_renderer *
             }
           },
           refills);
-    const bool pooled = best.trace_refill < 64 && prims >= best.trace_refill_prims;
-    if (rc == BNX_OK && pooled) rc = sweep([](bnx_tuning &t, int v) { t.trace_blocks_per_cu = v; }, blocks);
+    if (rc == BNX_OK && waves) rc = sweep([](bnx_tuning &t, int v) { t.trace_blocks_per_cu = v; }, blocks);
     if (rc == BNX_OK && (long long)np * probe_spp > (1LL << 20))
       rc = sweep([](bnx_tuning &t, long long v) { t.render_paths = v; }, paths);
     if (rc == BNX_OK) rc = sweep([](bnx_tuning &t, long long v) { t.graph_paths = v; }, graphs);

@@ -422,9 +422,11 @@ typedef struct bnx_tuning {
                                        8, 16 or 32 (of 192; the rest in private
                                        memory)                                       */
   int32_t trace_blocks_per_cu;      /* trace launch: at most this many times four
-                                       waves per CU, 1..64                           */
+                                       waves per CU, 1..64 (from 5 on as many as
+                                       are resident; walk 0)                         */
   int32_t trace_refill;             /* idle lanes that make a trace wave take new
-                                       rays, 1..64 (64: as for other worlds)         */
+                                       rays, 1..64 (64: 16, as for other worlds;
+                                       walk 0)                                       */
   int32_t trace_walk;               /* 0 = waves that take new rays as walks end, a
                                        node step or a leaf per trip (but 1 for a
                                        batch of bnx_render with 2^19 paths or more

@@ -137,6 +137,17 @@ def test_autotune_sets_valid_tuning_and_keeps_results(dev, worlds, keep_tuning):
     assert dev.tuning() == chosen
 
 
+def test_autotune_leaves_fields_that_change_nothing(dev, worlds, keep_tuning):
+    """no choice between launches that are the same: 16 idle lanes are the trace's own refill, and five blocks per
+    CU all its resident waves"""
+    gw, sc = worlds["c1"]
+    cam = bx.camera_perspective(sc.camera["position"], sc.camera["direction"], sc.camera["up"], sc.camera["fovy"])
+    start = dev.tuning()
+    chosen, _ = bx.autotune(gw.world, cam, abi.renderer(bg=sc.bg_color, ambient=sc.ambient), 96, 64, probe_spp=1)
+    assert chosen["trace_refill"] in (start["trace_refill"], 32, 8, 4)
+    assert chosen["trace_blocks_per_cu"] in (start["trace_blocks_per_cu"], 2, 3, 4)
+
+
 def _render_mg(dev, gw, sc, w, h, spp, mg):
     cam = bx.camera_perspective(sc.camera["position"], sc.camera["direction"], sc.camera["up"], sc.camera["fovy"])
     rend = abi.renderer(bg=sc.bg_color, ambient=sc.ambient, max_generations=mg)
