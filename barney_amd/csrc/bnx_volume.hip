@@ -555,7 +555,10 @@ __global__ void k_fine_ranges(const int4 *tets, const int4 *ext, const uint8_t *
   const v3 half{.52f * side.x + 1e-5f * far, .52f * side.y + 1e-5f * far, .52f * side.z + 1e-5f * far};
   if (tet)
     for (int k = 0; k < 4; k++) past[k] = dot(vabs(N[k]), half) + 1e-2f * size * length(N[k]);
-  const float reach = dot(vabs(grad), half);
+  // the linear function's rounding: each term's, however much they cancel
+  float reach = dot(vabs(grad), half);
+  if (tet)
+    for (int k = 0; k < 4; k++) reach += 1e-6f * fabsf(s[k]) * dot(vabs(N[k]), half);
   const int wx = bx - ax + 1, wy = by - ay + 1;
   for (long long j = sub; j < cells; j += LANES) {
     const int x = ax + (int)(j % wx), y = ay + (int)((j / wx) % wy), z = az + (int)(j / ((long long)wx * wy));
@@ -563,15 +566,16 @@ __global__ void k_fine_ranges(const int4 *tets, const int4 *ext, const uint8_t *
     if (tet) {
       const v3 C{d.seed_origin[0] + ((float)x + .5f) * side.x, d.seed_origin[1] + ((float)y + .5f) * side.y,
                  d.seed_origin[2] + ((float)z + .5f) * side.z};
-      float f = mid;
+      float f = mid, err = 0.f;
       bool out = false;
       for (int k = 0; k < 4; k++) {
         const float t = dot(C - at[k], N[k]);
         out |= t < -past[k];
         f += t * s[k];
+        err += 1e-6f * fabsf(s[k]) * dot(vabs(C - at[k]), vabs(N[k]));
       }
-      vl = fmx(vl, f - reach);
-      vh = fmn(vh, f + reach);
+      vl = fmx(vl, f - (reach + err));
+      vh = fmn(vh, f + (reach + err));
       if (out || vl - slack > vh + slack) continue;
     }
     const int i = (z * ny + y) * nx + x;

@@ -147,6 +147,16 @@ def test_isosurface_fine_grids(dev, orc, n, mc):
     _compare(dev, orc, us, bx.UMeshWorld(dev, us).world, orc.umesh_scene(us), 1)
 
 
+@pytest.mark.parametrize("n,power", [(12, 3), (20, 5)])
+def test_isosurface_graded_mesh(dev, orc, n, power):
+    """cells from far below a fine-grid cell to many of them"""
+    print(f"iso march graded mesh n={n} power={power}", flush=True)
+    us = scenes.config4(n=n, width=60, height=52, volume=False)
+    v = np.round(us.vertices.astype(np.float64) * n) / n                # the lattice without its jitter
+    us = dataclasses.replace(us, vertices=(v ** power).astype(np.float32))
+    _compare(dev, orc, us, bx.UMeshWorld(dev, us).world, orc.umesh_scene(us), 1)
+
+
 @pytest.mark.parametrize("n", [4, 8, 14, 40])
 def test_isosurface_queries_of_coarse_meshes(dev, n):
     """Tet tests a ray: 46, 34, 27 and 25 when every sub-step up to the crossing
