@@ -5,9 +5,10 @@ not finite (no corner copy, open value ranges); macrocells whose majorants are
 as small as floats get; isosurfaces whose samples'
 sides come from a fine grid of a single cell up to one a few cells wide, at
 values inside, at the ends and outside of the field's range, and over cells
-collapsed to triangles and lines.  IDs, ray and
-sample counts exact; depth within 1e-5 relative and pixels within 1e-3, the
-bounds of the volume tests next to this one."""
+collapsed to triangles and lines, or graded.  IDs, ray and sample counts, depths
+and pixels bit for bit; only where ratio tracking passes several volumes, whose
+estimates the oracle multiplies volume by volume and the march factor by
+factor, pixels within a rounding per factor."""
 import dataclasses
 
 import numpy as np
@@ -19,7 +20,7 @@ from barney_amd import abi, scenes
 pytestmark = pytest.mark.gpu
 
 
-def _compare(dev, orc, sc, world, scene, spp, flags=0):
+def _compare(dev, orc, sc, world, scene, spp, flags=0, rtol=0.0):
     rend = abi.renderer(bg=sc.bg_color, ambient=sc.ambient, flags=flags)
     c = sc.camera
     fr = bx.Frame(dev, sc.width, sc.height)
@@ -30,8 +31,10 @@ def _compare(dev, orc, sc, world, scene, spp, flags=0):
     for ch in (abi.BNX_FB_PRIMID, abi.BNX_FB_INSTID, abi.BNX_FB_OBJID):
         g, r = fr.read(ch), of.read(ch)
         assert np.array_equal(g, r), (ch, int((g != r).sum()))
-    assert np.allclose(fr.read(abi.BNX_FB_DEPTH), of.read(abi.BNX_FB_DEPTH), rtol=1e-5, atol=0)
-    assert np.abs(fr.read(abi.BNX_FB_COLOR) - of.read(abi.BNX_FB_COLOR)).max() <= 1e-3
+    assert np.array_equal(fr.read(abi.BNX_FB_DEPTH).view(np.uint32), of.read(abi.BNX_FB_DEPTH).view(np.uint32))
+    # accumulated in steps of 2^-32 a sample
+    g, r = fr.read(abi.BNX_FB_COLOR), of.read(abi.BNX_FB_COLOR)
+    assert np.allclose(g, r, rtol=rtol, atol=2.0 ** -31 if rtol else 0.0), float(np.abs(g - r).max())
     assert st["rays"] == ost["rays"]
     assert st["volume_samples"] == ost["volume_samples"]
     fr.close()
@@ -90,7 +93,8 @@ def test_many_volumes(dev, orc, n, flags):
         scene.add_volume(t, user_id=k, user_inst=k)
     scene.set_dir_lights(vs.dir_lights)
     scene.build()
-    _compare(dev, orc, vs, world, scene, 2, flags)
+    # up to some hundred factors between 0 and 1, each rounded to 2^-24
+    _compare(dev, orc, vs, world, scene, 2, flags, rtol=200 * 2.0 ** -24 if flags else 0.0)
 
 
 @pytest.mark.parametrize("bad", [np.nan, np.inf])
