@@ -5,11 +5,13 @@
 // kernels/traceRays.dev.cu:26-54.
 //
 // Design (wave64):
-//   * as many waves as fit (five per SIMD: the walk's 96 registers without
-//     spills; seven with 19 to 39 spilled took 34.2 ms where five take 26.4,
+//   * as many waves as fit (five per SIMD: the walk's 96 registers, of which
+//     the plain and the ray-array kernels spill none and the extended ones 19
+//     to 23; seven with 19 to 39 spilled took 34.2 ms where five take 26.4,
 //     secondary rays of 37.5M primitives, 1920x1080, 8 spp) share a
 //     generation's rays out in chunks (Claims) and take new rays as walks
-//     end, so short walks do not idle behind the wave's longest;
+//     end, so short walks do not idle behind the wave's longest; many rays in
+//     a world of few primitives go one to a thread instead (few_prims);
 //   * a wave runs one kind of step a trip, the one most of its lanes are at
 //     (a node, a leaf, into or out of an instance), so that it does not pay
 //     for every kind on every trip.  Bound by VALU issue where it has rays

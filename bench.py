@@ -31,7 +31,8 @@ algorithmic bytes follow the per-ray model 32 (ray in) + 16 (hit out) +
 and the counts taken by the CPU oracle's instrumented traversal of its own
 binary binned-SAH BVH on a stated ray subset of the same workload (shadow
 rays as occlusion queries, as the GPU traces them); per volume sample
-32 B (eight texels) + 4 B per macrocell step.  Beside it: the measured HBM
+32 B (eight texels) + 4 B per macrocell step.  Caches serve most of a walk's
+bytes, so the model's rate may pass the HBM peak.  Beside it: the measured HBM
 traffic of the kernel (rocprofv3 FETCH_SIZE / WRITE_SIZE, in profiles/) and
 its fraction of the HBM peak.
 """
@@ -126,11 +127,12 @@ def roofline(tot, workload=None, trace_kernel="k_trace_static<16, false, false>"
     from the oracle's counts (model: how they were counted); without it the
     GPU's own counters are priced at the same per-item sizes"""
     if tot.get("march_ms", 0.0) >= tot.get("trace_ms", 0.0) and tot.get("march_launches", 0) > 0:
-        # the kernel of the field's kind: 1 for tets (with the isosurface's,
-        # k_iso_march<1>, in the same march time and profile line), 0 for
-        # structured fields
+        # the kernel of the field's kind: k_volume_march<1> for tets (with the
+        # isosurface's, k_iso_march<1>, in the same march time and profile
+        # line), k_volume_rays for structured fields (with k_volume_march<0>,
+        # which has their large scattered generations)
         full = tot.get("umesh_nodes", 0) > 0 or workload == "c4"
-        kernel = "k_volume_march<1>" if full else "k_volume_march<0>"
+        kernel = "k_volume_march<1>" if full else "k_volume_rays"
         kms, launches = tot["march_ms"], tot["march_launches"]
         if tot.get("umesh_nodes", 0) > 0:
             byts = umesh_bytes(tot["umesh_nodes"], tot["umesh_tets"], tot["mc_cells"], tot["march_rays"])
@@ -141,9 +143,8 @@ def roofline(tot, workload=None, trace_kernel="k_trace_static<16, false, false>"
             model = ("32 B per volume sample + 4 B per macrocell step; sample and macrocell counts equal the "
                      "oracle's (the march is bit-exact with it)")
     else:
-        # queue traversal: one ray per thread, or pooled for the secondary rays
-        # of large scenes when the tuning says so; the HIP events bracket
-        # whichever ran
+        # queue traversal: waves that share rays out, or one ray per thread;
+        # the HIP events bracket whichever ran
         kernel = trace_kernel
         kms, launches = tot["trace_ms"], tot["trace_launches"]
         if trace_bytes is not None:
@@ -159,6 +160,9 @@ def roofline(tot, workload=None, trace_kernel="k_trace_static<16, false, false>"
            "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic, "kernel": kernel,
            "bytes_per_launch": round(byts / max(1, launches)), "avg_launch_ms": round(avg_ms, 5),
            "launches": launches, "kernel_ms": round(kms, 3), "byte_model": model}
+    if kernel.startswith("k_trace"):
+        out["note"] = ("the byte model counts every visit, most of which a cache serves: its rate is no share of the "
+                       "HBM peak and may pass it; dram_frac is")
     if traffic:
         dram = traffic / (avg_ms * 1e-3) / 1e9
         out["dram_gbs"] = round(dram, 2)
