@@ -605,13 +605,16 @@ template <int FIELD> struct March {
 // eleven loads in flight at once, and posts what is left: most cells end
 // there, and dealing their samples out for a look at the grid each cost more
 // than the queries that remain (8^3 cubes of five tets, 1920x1080, 2 spp: 11.0
-// ms with that, 7.8 so; 160^3: 12.7 and 11.3).  Bound by the records that the queries read (about
-// 1.8 requests beyond the L1 for each tet tested), so what helps is to ask for
-// fewer samples: 20.5M tets, 1024^2, 4 spp, isosurface and volume: 24.2 ms a
-// pass as nested loops, 16.7 with the samples dealt out, 13.5 with sides from
-// the fine grid, 12.3 with the owners' look,
-// 10.8 without spills; 14^3 mixed cells, 320x240, 2 spp:
-// 41.6, 8.2, 6.6, 6.0.
+// ms with that, 7.8 so; 160^3: 12.7 and 11.3).
+//
+// Bound by the records that the queries read (about 1.8 requests beyond the
+// L1 for each tet tested), so what helps is to ask for fewer samples: 20.5M
+// tets, 1024^2, 4 spp, isosurface and volume: 24.2 ms a pass as nested loops,
+// 16.7 with the samples dealt out, 13.5 with sides from the fine grid, 12.3
+// with the owners' look, 10.8 without spills; 14^3 mixed cells, 320x240, 2 spp:
+// 41.6, 8.2, 6.6, 6.0.  It still writes 4.5 GB a generation of 16M rays, some
+// ten times its results: parts of the queue's lines, and the stack of the
+// depth-first queries (its last 8 entries in LDS: 10.5 ms, and 10.5).
 enum Owner { O_IDLE = 0, O_CELL, O_SIDES, O_WAIT };
 enum Worker { W_FREE = 0, W_WALK, W_NODE, W_TEST };
 
