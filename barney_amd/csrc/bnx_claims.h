@@ -60,11 +60,11 @@ struct Claims {
     deal(z.block256 + (z.count + 255) / 256, sv.claims + program * CLAIM_GROUPS * CLAIM_STRIDE, least, balance);
   }
   // n rays without segments
-  BNX_D void begin(int n, int *counters, int least)
+  BNX_D void begin(int n, int *counters, int least, int balance)
   {
     segs = nullptr;
     blk = nullptr;
-    deal((n + 255) / 256, counters, least, 0);
+    deal((n + 255) / 256, counters, least, balance);
     seg = first = base = 0;
     total = n;
     dry = chunk < 0;

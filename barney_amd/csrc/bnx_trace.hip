@@ -712,11 +712,11 @@ struct ArraySource {
 
 template <bool EXT, bool XF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BNX_TRACE_WAVES))) void k_trace_api(
-    SceneDev S, const bnx_ray *rays, int n, bnx_hit *hits, uint32_t flags, int *claims)
+    SceneDev S, const bnx_ray *rays, int n, bnx_hit *hits, uint32_t flags, int *claims, int least)
 {
   __shared__ uint32_t ring[API_SHORT * 64];
   Claims cl;
-  cl.begin(n, claims, least_chunks(EXT));
+  cl.begin(n, claims, least, EXT ? BALANCE * (int)gridDim.x : 0);
   Counts cnt{0, 0, 0};
   const ArraySource src{rays, hits, (flags & BNX_TRACE_ANY) != 0};
   walk_rays<API_SHORT, EXT, XF>(cl, S, src, TAKE, ring, cnt);
@@ -905,8 +905,16 @@ int launch_trace_api(Group *g, const bnx_ray *d_rays, int n, bnx_hit *d_hits, ui
   if (rc != BNX_OK) return rc;
   const std::lock_guard<std::mutex> one(dev->api_mutex);
   if ((rc = launch_claims_clear(dev, dev->api_claims.as<int>())) != BNX_OK) return rc;
-  kernel<<<trace_waves_for(dev, fit, ((long long)n + 255) / 256), 64, 0, dev->stream>>>(
-      g->scene, d_rays, n, d_hits, flags, dev->api_claims.as<int>());
+  // Half as many chunks as waves, see least_chunks; the extended kernel's rays
+  // go 16 to a wave only where there are not enough for half of the resident
+  // waves at 32, and large arrays in two chunks a wave: capsules, cones and
+  // cylinders, 207 of them, 113354 rays, 123 us in 64s, 133 in 32s and 198 in
+  // 16s; 960 and 27 instances, 16397 rays, 464 in 16s and 524 in 32s; 2500,
+  // 700000 rays, 710 in 64s and 852 in 256s.
+  const int waves = trace_waves_for(dev, fit, ((long long)n + 255) / 256);
+  const int least = ext ? std::min(waves, fit * dev->num_cus / 2) : waves / 2;
+  kernel<<<waves, 64, 0, dev->stream>>>(
+      g->scene, d_rays, n, d_hits, flags, dev->api_claims.as<int>(), least);
   BNX_HIP(hipGetLastError());
   return BNX_OK;
 }

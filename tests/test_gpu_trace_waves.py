@@ -38,6 +38,15 @@ def test_ray_counts(dev, orc, name):
         assert np.array_equal(hit["prim_id"] >= 0, want[:n]["prim_id"] >= 0)
 
 
+@pytest.mark.parametrize("name,n", [("ext", 100001), ("ext_xf", 180007), ("ext", 700001), ("plain", 100001)])
+def test_chunks_of_arrays(dev, orc, name, n):
+    """chunks of 32, of 64 and of more rays"""
+    print(f"trace waves chunks {name} n={n}", flush=True)
+    spec = SPECS[name]()
+    rays = scenes.random_rays(25, n, radius=6.0, spread=3.0)
+    _same(spec.gpu(dev).trace(rays), spec.oracle(orc).trace(rays)[0])
+
+
 @pytest.mark.parametrize("name", ["plain", "xf"])
 def test_directions(dev, orc, name):
     """all signs of a direction, and components that are 0 or -0"""
