@@ -392,10 +392,11 @@ namespace {
 // are many more than are resident at once, and sharing rays out among those
 // that are costs more than it gives.  Such batches keep one ray per thread
 // (trace_walk 1).  us a frame, waves and a ray a thread: 484 spheres and 80
-// triangles, 1280x720, 860 and 733; 21k primitives, 1920x1080, 2 spp, 2592 and
-// 2297; 30k, 1024x768, 8 spp, 6124 and 6776; 1.3k, 400x300, 330 and 333 and, with
-// 1,000 spheres, 200x150, 360 and 401.
-constexpr long long FEW_PRIMS = 3 << 13, FEW_PATHS = 1 << 19;
+// triangles, 1280x720, 860 and 733; 8.1k primitives, 1920x1080, 2 spp, 3219 and
+// 2940, and 1024x768, 8 spp, 4167 and 4197; 10.4k, nearly all spheres, 748x700, 10
+// spp, 6044 and 6562; 1.3k, 400x300, 330 and 333 and, with 1,000 spheres, 200x150,
+// 360 and 401.
+constexpr long long FEW_PRIMS = 1 << 13, FEW_PATHS = 1 << 19;
 bool few_prims(const World *w, long long paths)
 {
   return paths >= FEW_PATHS && w->instances->blas_prims + (long long)w->instances->groups.size() < FEW_PRIMS;

@@ -430,7 +430,7 @@ typedef struct bnx_tuning {
   int32_t trace_walk;               /* 0 = waves that take new rays as walks end, a
                                        node step or a leaf per trip (but 1 for a
                                        batch of bnx_render with 2^19 paths or more
-                                       in a world of fewer than 3 * 2^13 primitives
+                                       in a world of fewer than 2^13 primitives
                                        and instances, where none needs the extended
                                        kernels); 1 = one ray per thread,
                                        speculative while-while (leaves set aside

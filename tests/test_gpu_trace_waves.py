@@ -108,7 +108,7 @@ def test_many_rays_few_primitives(dev, kind):
     """a batch that keeps one ray per thread against the same frame in batches too small for that"""
     print(f"trace waves few primitives {kind}", flush=True)
     w, h = 653, 461
-    sc = scenes.config1(width=w, height=h)
+    sc = scenes.config1(width=w, height=h, subdiv=3)   # 2,280 primitives
     if kind == "cylinders":
         sc.cylinders.append(scenes.sticks(300))
     world, c = bx.SurfaceWorld(dev, sc), sc.camera
